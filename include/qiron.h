@@ -240,8 +240,8 @@ qi_status qi_sumop_expectation(qi_state_t s, const qi_pauli_term *terms, size_t 
 /* qi_sumop_expectation with no allocation of any kind: no counterpart in the
  * reference. For callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid it). The term
- * table, block partials and group results live in a fixed static device
- * array (one per device, 76 KiB, held until the process ends) instead
+ * tables and block partials live in a fixed static device
+ * array (one per device, under 1 MiB, held until the process ends) instead
  * of the context's growable buffers. At most 512 terms (more: InvalidArgument).
  * Same kernels, same summation order and the same result bits as
  * qi_sumop_expectation. Calls on one context are serialised by its lock;

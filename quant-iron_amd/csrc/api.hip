@@ -35,6 +35,21 @@ Status ensure(DevBuf &b, size_t bytes) {
     return Status{};
 }
 
+Status ensure_stage(Ctx &C, size_t bytes) {
+    try {
+        if (C.plan_arena.size() < bytes) C.plan_arena.resize(bytes);
+    } catch (const std::bad_alloc &) {
+        return make_err(QI_ERR_OUT_OF_MEMORY, 0, 0, 0, 0, "host memory");
+    }
+    if (C.stage_bytes >= bytes) return Status{};
+    if (C.stage) (void)hipHostFree(C.stage);
+    C.stage = nullptr;
+    C.stage_bytes = 0;
+    QI_HIP_TRY(hipHostMalloc((void **)&C.stage, bytes));
+    C.stage_bytes = bytes;
+    return Status{};
+}
+
 // ------------------------------------------------------------- validation --
 // validate_qubits, operator.rs:214-273.
 static Status validate_qubits(uint32_t n, const uint64_t *t, uint32_t nt, const uint64_t *c, uint32_t nc, uint32_t expected) {
@@ -584,6 +599,7 @@ qi_status qi_ctx_create(int device, qi_ctx_t *out, qi_error *err) {
     // the no-allocation scratch array's address on this device (the device is current)
     {
         Status ns = noalloc_scratch(device, &C.noalloc);
+        if (ns.ok()) ns = ensure_stage(C, expect_stage_bytes(kNoAllocMaxTerms));
         if (!ns.ok()) QI_RET(ns);
     }
     // an unseeded context draws from an OS-seeded stream, as rand::rng() does
@@ -601,6 +617,7 @@ qi_status qi_ctx_destroy(qi_ctx_t ctx) {
     for (DevBuf *b : {&C.red, &C.red_out, &C.ops, &C.probs, &C.aux, &C.plan, &C.trot, &C.alt})
         if (b->p) (void)hipFree(b->p);
     if (C.host_pinned) (void)hipHostFree(C.host_pinned);
+    if (C.stage) (void)hipHostFree(C.stage);
     if (C.ev0) (void)hipEventDestroy(C.ev0);
     if (C.ev1) (void)hipEventDestroy(C.ev1);
     if (C.stream) (void)hipStreamDestroy(C.stream);

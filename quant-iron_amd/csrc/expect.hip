@@ -1,0 +1,443 @@
+// expect.hip — SumOp::expectation_value (pauli_string.rs:485-507).
+//
+// k_expect_tiles reads the state in tiles (expect_plan.h) and evaluates every
+// term whose X and Y factors lie inside the tile's qubits from that one read:
+// the tile is staged in LDS, a thread takes the 16 amplitudes of a register
+// set into FP64 registers and forms w = conj(a) b once per pair and x mask.
+// Terms that no tile holds (X support too wide) stream the state, one pass per
+// x mask (k_expect_group).
+#include <algorithm>
+
+#include "expect_plan.h"
+#include "qi_internal.h"
+#include "reduce_util.h"
+
+namespace qi {
+
+namespace {
+
+#pragma clang fp contract(off)
+
+// XOR-linear LDS slot of tile-local index e. complex64: bits 1-3 take the
+// bits above them in (pairs stay 16-byte units), complex128: bits 0-2.
+template <typename T> __device__ __forceinline__ uint32_t exp_slot(uint32_t e) {
+    if constexpr (sizeof(T) == 8) return e ^ ((((e >> 4) ^ (e >> 7) ^ (e >> 10)) & 7u) << 1);
+    else return e ^ (((e >> 3) ^ (e >> 6) ^ (e >> 9) ^ (e >> 12)) & 7u);
+}
+__device__ __forceinline__ uint32_t exp_ins0(uint32_t k, uint32_t p) { return ((k >> p) << (p + 1)) | (k & ((1u << p) - 1)); }
+
+// x with its sign flipped when the low bit of `odd` is set
+__device__ __forceinline__ double flip_sign(double x, uint32_t odd) {
+    const uint64_t b = (uint64_t)__double_as_longlong(x) ^ ((uint64_t)(odd & 1u) << 63);
+    return __longlong_as_double((long long)b);
+}
+
+// u = Re w (IM 0) or Im w (IM 1), w = conj(a) b, of the 8 pairs (s, s ^ M) of
+// the register bits, s with the highest bit of M clear, in ascending order of s.
+template <int M, int IM>
+__device__ __forceinline__ void pair_products(const double (&ar)[kExpSlots], const double (&ai)[kExpSlots], double (&u)[8]) {
+    constexpr int P = 31 - __builtin_clz(M);
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        const int s = ((k >> P) << (P + 1)) | (k & ((1 << P) - 1)), t = s ^ M;
+        if (IM) u[k] = __builtin_fma(ar[s], ai[t], -(ai[s] * ar[t]));
+        else u[k] = __builtin_fma(ar[s], ar[t], ai[s] * ai[t]);
+    }
+}
+
+// What bounds it: FP64 issue and one read of the state per pass, about evenly
+// (two 64 KiB tiles per CU, so one loads while the other computes). The
+// four-bit register sets share the LDS reads (16 per thread and set) and the
+// FP64 conversions among the masks of the set; a Heisenberg bond costs a
+// multiply-add pair and one multiply-add per amplitude pair, whatever its
+// number of terms. 29 qubits, complex64, a chain with fields (113 terms, 29 x
+// masks): 67.1 ms with one read of the state per mask, 4.9 ms in three passes.
+// The imaginary sums (complex coefficients) take registers that cost half the
+// waves, so they have an instance of their own.
+template <typename T, bool CPLX>
+__global__ __launch_bounds__(512, CPLX ? 2 : 4) void k_expect_tiles(const T *__restrict__ psi, const ExpPass *__restrict__ passes,
+                                                      const ExpSet *__restrict__ sets, const ExpUnit *__restrict__ units,
+                                                      const ExpDiag *__restrict__ diags, int K, uint32_t per_pass,
+                                                      uint64_t tiles, double *__restrict__ part) {
+    constexpr bool F32 = sizeof(T) == 8;
+    extern __shared__ __attribute__((aligned(16))) unsigned char exp_lds[];
+    T *const tile = reinterpret_cast<T *>(exp_lds);
+    const uint32_t tid = threadIdx.x, nt = 1u << (K - 4);  // threads that hold amplitudes
+    const bool act = tid < nt;
+    const ExpPass &ps = passes[blockIdx.x / per_pass];
+    // Loads: 16-byte units, thread t takes units t, t + nt, ...: the low K - 4
+    // unit bits are the thread's, the rest the unit counter's (uniform).
+    constexpr int UB = F32 ? 1 : 0, NU = kExpSlots >> UB, JB = 4 - UB;  // local bits in a unit, units per thread, counter bits
+    uint64_t at = 0;
+    for (int i = 0; i < K - 4; i++) at |= uint64_t((tid >> i) & 1u) << exp_pos(ps.pos, i + UB);
+    DD acc[2] = {dd_zero(), dd_zero()};
+    for (uint64_t t = blockIdx.x % per_pass; t < tiles; t += per_pass) {
+        uint64_t base = t;
+        for (int k = 0; k < K; k++) {
+            const uint32_t b = exp_pos(ps.pos, k);
+            base = ((base >> b) << (b + 1)) | (base & ((uint64_t(1) << b) - 1));
+        }
+        if (act) {
+            typedef float F4 __attribute__((ext_vector_type(4)));
+            F4 u[NU];
+#pragma unroll
+            for (int j = 0; j < NU; j++) {
+                uint64_t o = 0;
+#pragma unroll
+                for (int b = 0; b < JB; b++)
+                    if ((j >> b) & 1) o |= uint64_t(1) << exp_pos(ps.pos, K - JB + b);
+                u[j] = __builtin_nontemporal_load(reinterpret_cast<const F4 *>(psi + (base | at | o)));
+            }
+            const uint32_t l0 = exp_slot<T>(tid << UB);
+#pragma unroll
+            for (int j = 0; j < NU; j++)
+                *reinterpret_cast<F4 *>(tile + (l0 ^ exp_slot<T>(uint32_t(j) << (K - JB)))) = u[j];
+        }
+        __syncthreads();
+        for (uint32_t si = ps.s0; si < ps.s0 + ps.ns; si++) {
+            const ExpSet &st = sets[si];
+            if (!act) continue;
+            const uint32_t pos = st.pos;
+            const uint32_t tl = exp_ins0(exp_ins0(exp_ins0(exp_ins0(tid, pos & 255u), (pos >> 8) & 255u), (pos >> 16) & 255u), pos >> 24);
+            const uint32_t ls = exp_slot<T>(tl);
+            uint32_t so[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) so[j] = exp_slot<T>(1u << ((pos >> (8 * j)) & 255u));
+            double ar[kExpSlots], ai[kExpSlots];
+#pragma unroll
+            for (int s = 0; s < kExpSlots; s++) {
+                uint32_t o = ls;
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    if ((s >> j) & 1) o ^= so[j];
+                const T a = tile[o];
+                ar[s] = a.x;
+                ai[s] = a.y;
+            }
+            double sr = 0.0, sm = 0.0;  // this set's sums
+            double u[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+            ExpUnit nxt = units[st.u0];
+            for (uint32_t ui = st.u0; ui < st.u0 + st.nu; ui++) {
+                const ExpUnit un = nxt;
+                nxt = units[ui + 1];  // read a unit ahead (the table ends with a spare)
+                // (the amplitudes are opaque per trip: the products of all masks
+                // would otherwise be hoisted out of the loop and spilled)
+#pragma unroll
+                for (int s = 0; s < kExpSlots; s++) asm volatile("" : "+v"(ar[s]), "+v"(ai[s]));
+                if (!(un.flags() & kExpReuse)) {
+                    switch (un.code()) {
+#define QI_M(M) case M: pair_products<M, 0>(ar, ai, u); break; case M + 16: pair_products<M, 1>(ar, ai, u); break;
+                        QI_M(1) QI_M(2) QI_M(3) QI_M(4) QI_M(5) QI_M(6) QI_M(7) QI_M(8)
+                        QI_M(9) QI_M(10) QI_M(11) QI_M(12) QI_M(13) QI_M(14) QI_M(15)
+#undef QI_M
+                    default: {  // wide: the partner from LDS
+                        const uint32_t lx = exp_slot<T>(un.xl()), hi = un.flags() & kExpHigh ? so[3] : 0u;
+#pragma unroll
+                        for (int k = 0; k < 8; k++) {
+                            uint32_t o = ls ^ hi;
+#pragma unroll
+                            for (int j = 0; j < 3; j++)
+                                if ((k >> j) & 1) o ^= so[j];
+                            const T a = tile[o], b = tile[o ^ lx];
+                            const double xr = a.x, xi = a.y, br = b.x, bi = b.y;
+                            u[k] = un.code() ? __builtin_fma(xr, bi, -(xi * br)) : __builtin_fma(xr, br, xi * bi);
+                        }
+                    } break;
+                    }
+                }
+                double v0 = u[0] * un.h[0], v1 = u[1] * un.h[1];
+#pragma unroll
+                for (int k = 2; k < 8; k += 2) {
+                    v0 = __builtin_fma(u[k], un.h[k], v0);
+                    v1 = __builtin_fma(u[k + 1], un.h[k + 1], v1);
+                }
+                const double v = flip_sign(v0 + v1, __popcll(base & un.zo) + __popc(tl & un.zl));
+                if (CPLX && (un.flags() & kExpImag)) sm += v;
+                else sr += v;
+            }
+            if (st.diag) {
+                // Walsh sums W[p] = sum_s (-1)^{popcount(s & p)} |a_s|^2: a term adds
+                // its signed coefficient times the sum of its register-bit pattern
+                double w[kExpSlots];
+#pragma unroll
+                for (int s = 0; s < kExpSlots; s++) w[s] = __builtin_fma(ar[s], ar[s], ai[s] * ai[s]);
+#pragma unroll
+                for (int b = 1; b < kExpSlots; b <<= 1)
+#pragma unroll
+                    for (int s = 0; s < kExpSlots; s++)
+                        if (!(s & b)) {
+                            const double x = w[s], y = w[s | b];
+                            w[s] = x + y;
+                            w[s | b] = x - y;
+                        }
+#pragma unroll
+                for (int p = 0; p < kExpSlots; p++) {
+                    double cr = 0.0, ci = 0.0;
+                    for (uint32_t d = st.doff[p]; d < st.doff[p + 1]; d++) {
+                        const ExpDiag &t1 = diags[d];
+                        const uint32_t odd = __popcll(base & t1.zo) + __popc(tl & t1.zl);
+                        cr += flip_sign(t1.re, odd);
+                        if (CPLX) ci += flip_sign(t1.im, odd);
+                    }
+                    sr = __builtin_fma(w[p], cr, sr);
+                    if (CPLX) sm = __builtin_fma(w[p], ci, sm);
+                }
+            }
+            dd_acc(acc[0], sr);
+            if (CPLX) dd_acc(acc[1], sm);
+        }
+        __syncthreads();  // the next tile overwrites the LDS copy
+    }
+    double *sh = reinterpret_cast<double *>(exp_lds);  // 2 values x 2 doubles per wave
+    block_reduce_dd<2>(acc, sh);
+    if (tid == 0) {
+        part[size_t(blockIdx.x) * 4 + 0] = acc[0].s; part[size_t(blockIdx.x) * 4 + 1] = acc[0].c;
+        part[size_t(blockIdx.x) * 4 + 2] = acc[1].s; part[size_t(blockIdx.x) * 4 + 3] = acc[1].c;
+    }
+}
+
+// A term for the streaming kernel.
+struct TermK {
+    uint64_t x, z;
+    unsigned q0;  // 3 * nY mod 4
+    unsigned pad;
+    double c[2];
+};
+
+// Quarter turns of (-i)^{nY} (-1)^{popcount(i & z)}.
+__device__ __forceinline__ unsigned quarter(uint64_t i, uint64_t z, unsigned q0) {
+    return q0 + 2u * (unsigned)__popcll(i & z);
+}
+__device__ __forceinline__ uint64_t insert_zero(uint64_t k, unsigned p) {
+    return ((k >> p) << (p + 1)) | (k & ((uint64_t(1) << p) - 1));
+}
+
+// Expectation of a group of terms sharing the same x mask, one pass over the
+// state (masks wider than a tile, states of fewer than 4 qubits):
+//   sum_i conj(psi_i) psi_{i^x} h(i),  h(i) = sum_t c_t i^{q_t(i)}.
+// FP64 accumulation with two-sum compensation; one partial per block.
+template <typename T>
+__global__ __launch_bounds__(256) void k_expect_group(const T *__restrict__ psi, uint64_t items, uint64_t x,
+                                                      unsigned pivot, const TermK *__restrict__ terms, int nt,
+                                                      double *__restrict__ part) {
+    __shared__ double sh[4 * 4];
+    DD v[2] = {dd_zero(), dd_zero()};
+    for (uint64_t k = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; k < items; k += uint64_t(gridDim.x) * blockDim.x) {
+        uint64_t i = x == 0 ? k : insert_zero(k, pivot);
+        uint64_t j = i ^ x;
+        double ar = psi[i].x, ai = psi[i].y, br = psi[j].x, bi = psi[j].y;
+        // w = conj(a) * b for index i; for the partner j it is conj(w)
+        double wr = ar * br + ai * bi, wi = ar * bi - ai * br;
+        double hr = 0, hi = 0, gr = 0, gi = 0;
+        for (int t = 0; t < nt; t++) {
+            unsigned qi_ = quarter(i, terms[t].z, terms[t].q0) & 3;
+            double cr = terms[t].c[0], ci = terms[t].c[1];
+            // c * i^q
+            double pr = qi_ == 0 ? cr : qi_ == 1 ? -ci : qi_ == 2 ? -cr : ci;
+            double pi = qi_ == 0 ? ci : qi_ == 1 ? cr : qi_ == 2 ? -ci : -cr;
+            hr += pr; hi += pi;
+            if (x != 0) {
+                unsigned qj = quarter(j, terms[t].z, terms[t].q0) & 3;
+                double qr = qj == 0 ? cr : qj == 1 ? -ci : qj == 2 ? -cr : ci;
+                double qi2 = qj == 0 ? ci : qj == 1 ? cr : qj == 2 ? -ci : -cr;
+                gr += qr; gi += qi2;
+            }
+        }
+        // conj(psi_i) psi_j h(i)
+        dd_acc(v[0], wr * hr - wi * hi);
+        dd_acc(v[1], wr * hi + wi * hr);
+        if (x != 0) {  // conj(psi_j) psi_i h(j) = conj(w) h(j)
+            dd_acc(v[0], wr * gr + wi * gi);
+            dd_acc(v[1], wr * gi - wi * gr);
+        }
+    }
+    block_reduce_dd<2>(v, sh);
+    if (threadIdx.x == 0) {
+        part[size_t(blockIdx.x) * 4 + 0] = v[0].s; part[size_t(blockIdx.x) * 4 + 1] = v[0].c;
+        part[size_t(blockIdx.x) * 4 + 2] = v[1].s; part[size_t(blockIdx.x) * 4 + 3] = v[1].c;
+    }
+}
+
+// ------------------------------------------------------------- host side --
+// Workgroups: a pass takes up to kExpBlocks / passes of them, a streamed mask
+// up to kExpBlocks / 4 / masks, neither fewer than kExpBlocksMin (for at most
+// 512 passes and masks: at most 2 kExpBlocksMin * 512 partials).
+constexpr uint64_t kExpBlocks = 4096, kExpBlocksMin = 16;
+
+size_t up16(size_t b) { return (b + 15) & ~size_t(15); }
+
+struct ExpLaunch {
+    size_t sets, units, diags, far, bytes;  // offsets in the device tables (passes first), their size
+    uint32_t per_pass, per_far;
+    uint64_t tiles;
+    size_t blocks;  // partials of the whole call
+};
+
+TermK far_term(const qi_pauli_term &p) {
+    TermK t{};
+    t.x = p.x_mask; t.z = p.z_mask;
+    t.q0 = (3u * (unsigned)__builtin_popcountll(p.x_mask & p.z_mask)) & 3u;
+    t.c[0] = p.c_re; t.c[1] = p.c_im;
+    return t;
+}
+
+// Plans into `arena` (exp_plan_bytes(nt)); a state of fewer than 4 qubits has
+// no tiles: every mask is streamed.
+ExpLaunch plan_launch(const State &s, const qi_pauli_term *terms, size_t nt, void *arena, ExpPlan &p, size_t *far_terms) {
+    exp_plan_carve(p, arena, nt);
+    const bool c128 = s.prec == QI_C128;
+    if (s.n >= 4) {
+        plan_expect(s.n, c128, terms, nt, p);
+    } else {
+        p.npasses = p.nsets = p.nunits = p.ndiags = p.nfar = 0;
+        p.K = 0;
+        for (size_t k = 0; k < nt; k++) {
+            size_t g = 0;
+            while (g < p.nfar && p.far[g] != terms[k].x_mask) g++;
+            if (g == p.nfar) p.far[p.nfar++] = terms[k].x_mask;
+        }
+    }
+    size_t nf = 0;
+    for (size_t g = 0; g < p.nfar; g++)
+        for (size_t k = 0; k < nt; k++) nf += terms[k].x_mask == p.far[g];
+    *far_terms = nf;
+    ExpLaunch L{};
+    L.sets = up16(p.npasses * sizeof(ExpPass));
+    L.units = L.sets + up16(p.nsets * sizeof(ExpSet));
+    L.diags = L.units + up16((p.nunits + 1) * sizeof(ExpUnit));
+    L.far = L.diags + up16(p.ndiags * sizeof(ExpDiag));
+    L.bytes = L.far + up16(nf * sizeof(TermK));
+    const uint64_t dim = uint64_t(1) << s.n;
+    if (p.npasses) {
+        L.tiles = dim >> p.K;
+        L.per_pass = (uint32_t)std::min<uint64_t>(L.tiles, std::max<uint64_t>(kExpBlocksMin, kExpBlocks / p.npasses));
+    }
+    if (p.nfar) L.per_far = (uint32_t)std::min<uint64_t>((dim + 2047) / 2048, std::max<uint64_t>(kExpBlocksMin, kExpBlocks / 4 / p.nfar));
+    L.blocks = p.npasses * L.per_pass + p.nfar * L.per_far;
+    return L;
+}
+
+// Device tables in the order of ExpLaunch's offsets.
+void pack_tables(const ExpPlan &p, const ExpLaunch &L, const qi_pauli_term *terms, size_t nt, unsigned char *dst) {
+    memcpy(dst, p.passes, p.npasses * sizeof(ExpPass));
+    memcpy(dst + L.sets, p.sets, p.nsets * sizeof(ExpSet));
+    if (p.npasses) memcpy(dst + L.units, p.units, (p.nunits + 1) * sizeof(ExpUnit));
+    memcpy(dst + L.diags, p.diags, p.ndiags * sizeof(ExpDiag));
+    TermK *f = reinterpret_cast<TermK *>(dst + L.far);
+    for (size_t g = 0; g < p.nfar; g++)
+        for (size_t k = 0; k < nt; k++)
+            if (terms[k].x_mask == p.far[g]) *f++ = far_term(terms[k]);
+}
+
+template <typename T>
+Status launch_all(const State &s, const ExpPlan &p, const ExpLaunch &L, const qi_pauli_term *terms, size_t nt,
+                  const unsigned char *tab, double *part, double *out, hipStream_t st) {
+    if (p.npasses) {
+        const unsigned threads = std::max(64u, 1u << (p.K - 4));
+        auto *const kernel = p.complex_out ? k_expect_tiles<T, true> : k_expect_tiles<T, false>;
+        hipLaunchKernelGGL(kernel, dim3(L.per_pass * (unsigned)p.npasses), dim3(threads),
+                           std::max<size_t>(sizeof(T) << p.K, 512), st, (const T *)s.d, (const ExpPass *)tab,
+                           (const ExpSet *)(tab + L.sets), (const ExpUnit *)(tab + L.units),
+                           (const ExpDiag *)(tab + L.diags), p.K, L.per_pass, L.tiles, part);
+    }
+    const TermK *f = reinterpret_cast<const TermK *>(tab + L.far);
+    double *pg = part + size_t(L.per_pass) * p.npasses * 4;
+    for (size_t g = 0; g < p.nfar; g++) {
+        const uint64_t x = p.far[g], dim = uint64_t(1) << s.n;
+        int cnt = 0;
+        for (size_t k = 0; k < nt; k++) cnt += terms[k].x_mask == x;
+        hipLaunchKernelGGL(k_expect_group<T>, dim3(L.per_far), dim3(256), 0, st, (const T *)s.d, x ? dim / 2 : dim, x,
+                           x ? (unsigned)__builtin_ctzll(x) : 0u, f, cnt, pg);
+        f += cnt;
+        pg += size_t(L.per_far) * 4;
+    }
+    hipLaunchKernelGGL(k_reduce_partials<2>, dim3(1), dim3(256), 0, st, (const double *)part, (int)L.blocks, out);
+    QI_HIP_TRY(hipGetLastError());
+    return Status{};
+}
+
+// Uploads the packed tables through the context's pinned staging buffer and
+// runs the launches; the result lands in the context's pinned words.
+Status expect_run(State &s, const qi_pauli_term *terms, size_t nt, const ExpPlan &p, const ExpLaunch &L, void *dtab,
+                  double *part, double *re, double *im, hipStream_t st) {
+    Ctx &C = *s.ctx;
+    pack_tables(p, L, terms, nt, (unsigned char *)C.stage);
+    QI_HIP_TRY(hipMemcpyAsync(dtab, C.stage, L.bytes, hipMemcpyHostToDevice, st));
+    Status e = s.prec == QI_C128
+                   ? launch_all<double2>(s, p, L, terms, nt, (const unsigned char *)dtab, part, C.host_pinned, st)
+                   : launch_all<float2>(s, p, L, terms, nt, (const unsigned char *)dtab, part, C.host_pinned, st);
+    if (!e.ok()) return e;
+    QI_HIP_TRY(hipStreamSynchronize(st));
+    *re = C.host_pinned[0];
+    *im = C.host_pinned[1];
+    return Status{};
+}
+
+}  // namespace
+
+size_t expect_stage_bytes(size_t nt) { return exp_plan_bytes(nt) + nt * sizeof(TermK) + 256; }
+
+Status sumop_expectation(State &s, const qi_pauli_term *terms, size_t nt, double *re, double *im, hipStream_t st) {
+    Ctx &C = *s.ctx;
+    Status e = ensure_stage(C, expect_stage_bytes(nt));
+    if (!e.ok()) return e;
+    ExpPlan p;
+    size_t nf;
+    const ExpLaunch L = plan_launch(s, terms, nt, C.plan_arena.data(), p, &nf);
+    if (!(e = ensure(C.ops, L.bytes)).ok()) return e;
+    if (!(e = ensure(C.red, L.blocks * 4 * sizeof(double))).ok()) return e;
+    return expect_run(s, terms, nt, p, L, C.ops.p, (double *)C.red.p, re, im, st);
+}
+
+// ---------------------------------------------------- no-allocation variant --
+// qi_sumop_expectation_noalloc keeps its tables and block partials in this
+// fixed device array instead of the context's growable buffers (the host
+// arena and staging buffer of the context hold kNoAllocMaxTerms terms from its
+// creation): no allocation on any call. Each device that the library runs on
+// holds its own copy until the process ends. Every location a call reads is
+// written earlier in the same call, so nothing needs clearing; calls that
+// overlap on one device (different contexts, or threads without the context's
+// lock) race on it.
+namespace {
+struct NoAllocScratch {
+    unsigned char tab[kNoAllocMaxTerms * (sizeof(ExpPass) + sizeof(ExpSet) + 4 * sizeof(ExpUnit) + sizeof(ExpDiag) +
+                                          sizeof(TermK)) + 512];
+    double part[(kExpBlocks + 2 * kExpBlocksMin * kNoAllocMaxTerms) * 4];
+};
+}  // namespace
+
+static __device__ __align__(256) unsigned char scratch[sizeof(NoAllocScratch)];
+
+Status noalloc_scratch(int device, void **out) {
+    static std::mutex mu;
+    static void *ptrs[64] = {nullptr};
+    if (device < 0 || device >= 64) return make_err(QI_ERR_INVALID_ARGUMENT, 0, 0, 0, 0, "device index");
+    std::lock_guard<std::mutex> lk(mu);
+    if (!ptrs[device]) {
+        // the host-side name of `scratch` is not a device address: take the
+        // address of this device's copy once, with the device current
+        void *p = nullptr;
+        QI_HIP_TRY(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)));
+        ptrs[device] = p;
+    }
+    *out = ptrs[device];
+    return Status{};
+}
+
+Status sumop_expectation_noalloc(State &s, const qi_pauli_term *terms, size_t nt, double *re, double *im, hipStream_t st) {
+    void *base = s.ctx->noalloc;
+    if (!base) return make_err(QI_ERR_DEVICE, 0, 0, 0, 0, "no scratch address for this device");
+    if (nt > (size_t)kNoAllocMaxTerms)
+        return make_err(QI_ERR_INVALID_ARGUMENT, nt, kNoAllocMaxTerms, 0, 0, "more terms than the no-allocation maximum (512)");
+    *re = 0.0; *im = 0.0;
+    if (nt == 0) return Status{};
+    NoAllocScratch *sc = reinterpret_cast<NoAllocScratch *>(base);
+    ExpPlan p;
+    size_t nf;
+    const ExpLaunch L = plan_launch(s, terms, nt, s.ctx->plan_arena.data(), p, &nf);
+    if (L.bytes > sizeof sc->tab || L.blocks * 4 * sizeof(double) > sizeof sc->part)
+        return make_err(QI_ERR_DEVICE, 0, 0, 0, 0, "expectation scratch");
+    return expect_run(s, terms, nt, p, L, sc->tab, sc->part, re, im, st);
+}
+
+}  // namespace qi

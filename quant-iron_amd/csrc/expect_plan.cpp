@@ -1,0 +1,220 @@
+// expect_plan.cpp — host planner of expect_plan.h. Works in arrays the caller
+// owns: no allocation of its own (the no-allocation entry point plans with it).
+#include "expect_plan.h"
+
+#include <cstring>
+
+namespace qi {
+
+namespace {
+
+size_t up16(size_t b) { return (b + 15) & ~size_t(15); }
+int popc(uint64_t x) { return __builtin_popcountll(x); }
+
+// The tile-local image of a qubit mask inside the tile.
+uint32_t local_bits(uint64_t mask, const ExpPass &p, int K) {
+    uint32_t r = 0;
+    for (int k = 0; k < K; k++) r |= uint32_t((mask >> exp_pos(p.pos, k)) & 1u) << k;
+    return r;
+}
+// The pattern of a tile-local mask on a set's register bits.
+uint32_t reg_bits(uint32_t l, const ExpSet &s) {
+    uint32_t r = 0;
+    for (int j = 0; j < 4; j++) r |= ((l >> exp_pos(&s.pos, j)) & 1u) << j;
+    return r;
+}
+
+// Union growth: adds to `u` every mask of take[] that fits into `cap` bits,
+// the ones that need the fewest new bits first; above kGreedyMax masks simply
+// in list order (the search is quadratic).
+constexpr size_t kGreedyMax = 256;
+
+}  // namespace
+
+size_t exp_plan_bytes(size_t nt) {
+    return up16(nt * sizeof(ExpPass)) + up16(nt * sizeof(ExpSet)) + up16((4 * nt + 1) * sizeof(ExpUnit)) +
+           up16(nt * sizeof(ExpDiag)) + 2 * up16(nt * sizeof(uint64_t)) +
+           up16(2 * nt * sizeof(uint32_t));
+}
+
+void exp_plan_carve(ExpPlan &p, void *arena, size_t nt) {
+    unsigned char *a = (unsigned char *)arena;
+    auto take = [&](size_t bytes) { void *r = a; a += up16(bytes); return r; };
+    p.passes = (ExpPass *)take(nt * sizeof(ExpPass));
+    p.sets = (ExpSet *)take(nt * sizeof(ExpSet));
+    p.units = (ExpUnit *)take((4 * nt + 1) * sizeof(ExpUnit));
+    p.diags = (ExpDiag *)take(nt * sizeof(ExpDiag));
+    p.far = (uint64_t *)take(nt * sizeof(uint64_t));
+    p.xs = (uint64_t *)take(nt * sizeof(uint64_t));
+    p.gid = (uint32_t *)take(2 * nt * sizeof(uint32_t));
+}
+
+int exp_tile_qubits(uint32_t n, bool c128) {
+    const int most = c128 ? kExpMaxK - 1 : kExpMaxK;
+    return (int)n < most ? (int)n : most;
+}
+
+void plan_expect(uint32_t n, bool c128, const qi_pauli_term *terms, size_t nt, ExpPlan &p) {
+    const int K = exp_tile_qubits(n, c128), low = exp_low_qubits(c128);
+    p.K = K;
+    p.npasses = p.nsets = p.nunits = p.ndiags = p.nfar = 0;
+    p.complex_out = false;
+    const bool whole = (int)n == K;
+    const uint64_t lowmask = whole ? (uint64_t(1) << n) - 1 : (uint64_t(1) << low) - 1;
+    // distinct nonzero x masks in order of appearance; next term of the same mask in gid[nt + k]
+    size_t nx = 0;
+    uint32_t *const head = p.gid, *const next = p.gid + nt;  // head: first term of mask g
+    bool diag = false;
+    for (size_t k = 0; k < nt; k++) {
+        p.complex_out = p.complex_out || terms[k].c_im != 0.0;
+        next[k] = UINT32_MAX;
+        if (!terms[k].x_mask) { diag = true; continue; }
+        size_t g = nx;
+        // (terms of one mask are often neighbours: look from the back)
+        while (g > 0 && p.xs[g - 1] != terms[k].x_mask) g--;
+        if (g == 0) {
+            p.xs[nx] = terms[k].x_mask;
+            head[nx++] = (uint32_t)k;
+        } else {
+            uint32_t t = head[g - 1];
+            while (next[t] != UINT32_MAX) t = next[t];
+            next[t] = (uint32_t)k;
+        }
+    }
+    // masks that no tile holds go to the streaming kernel
+    size_t nleft = 0;
+    for (size_t g = 0; g < nx; g++) {
+        if (popc(p.xs[g] | lowmask) > K) { p.far[p.nfar++] = p.xs[g]; continue; }
+        p.xs[nleft] = p.xs[g];
+        head[nleft++] = head[g];
+    }
+    bool diag_todo = diag;
+    size_t at = 0;  // masks [at, nleft) are unplanned; a pass moves its masks to the front
+    while (at < nleft || diag_todo) {
+        ExpPass &ps = p.passes[p.npasses++];
+        memset(&ps, 0, sizeof ps);
+        // the tile: the low qubits, then masks that need the fewest new qubits
+        uint64_t q = lowmask;
+        for (bool grown = true; grown;) {
+            grown = false;
+            size_t best = SIZE_MAX;
+            int least = 64;
+            for (size_t g = at; g < nleft; g++) {
+                const int add = popc(p.xs[g] & ~q);
+                if (!add || popc(q) + add > K || add >= least) continue;
+                best = g; least = add;
+                if (nleft - at > kGreedyMax || add == 1) break;
+            }
+            if (best != SIZE_MAX) { q |= p.xs[best]; grown = true; }
+        }
+        for (uint32_t b = 0; b < n && popc(q) < K; b++) q |= uint64_t(1) << b;
+        ps.qmask = q;
+        for (int k = 0, b = 0; k < K; b++)
+            if ((q >> b) & 1) { ps.pos[k >> 2] |= (uint32_t)b << (8 * (k & 3)); k++; }
+        ps.s0 = (uint32_t)p.nsets;
+        const size_t first = at;
+        for (size_t g = at; g < nleft; g++)
+            if (!(p.xs[g] & ~q)) {
+                const uint64_t x = p.xs[g]; p.xs[g] = p.xs[at]; p.xs[at] = x;
+                const uint32_t h = head[g]; head[g] = head[at]; head[at] = h;
+                at++;
+            }
+        // register sets over this pass's masks [first, at)
+        bool pass_diag = diag_todo;
+        diag_todo = false;
+        size_t s_at = first;
+        while (s_at < at || pass_diag) {
+            ExpSet &st = p.sets[p.nsets++];
+            memset(&st, 0, sizeof st);
+            uint32_t r = 0;
+            for (bool grown = true; grown;) {
+                grown = false;
+                size_t best = SIZE_MAX;
+                int least = 64;
+                for (size_t g = s_at; g < at; g++) {
+                    const int add = popc(local_bits(p.xs[g], ps, K) & ~r);
+                    if (!add || popc(r) + add > 4 || add >= least) continue;
+                    best = g; least = add;
+                    if (at - s_at > kGreedyMax || add == 1) break;
+                }
+                if (best != SIZE_MAX) { r |= local_bits(p.xs[best], ps, K); grown = true; }
+            }
+            for (int b = K - 1; b >= 0 && popc(r) < 4; b--) r |= 1u << b;
+            for (int j = 0, b = 0; j < 4; b++)
+                if ((r >> b) & 1) st.pos |= (uint32_t)b << (8 * j++);
+            st.u0 = (uint32_t)p.nunits;
+            // the masks inside the set, and (with no set of their own) the ones of more than four bits
+            for (size_t g = s_at; g < at; g++) {
+                const uint32_t xl = local_bits(p.xs[g], ps, K);
+                const bool wide = popc(xl) > 4;
+                if (!wide && (xl & ~r)) continue;
+                const uint32_t xm = wide ? 0 : reg_bits(xl, st);
+                const int pivot = xm ? 31 - __builtin_clz(xm) : -1;
+                // one run of units per u: Re w or Im w, and for wide masks the two halves of the slots
+                for (int run = 0; run < (wide ? 4 : 2); run++) {
+                    const int im_w = run & 1, high = run >> 1;
+                    const size_t e0 = p.nunits;
+                    for (uint32_t t = head[g]; t != UINT32_MAX; t = next[t]) {
+                        const qi_pauli_term &tm = terms[t];
+                        const int ny = popc(tm.x_mask & tm.z_mask);
+                        if ((ny & 1) != im_w) continue;
+                        // phi(i) = (-i)^ny (-1)^{popcount(i & z)}: Re(phi w) is s Re w (ny 0: s = 1, ny 2: -1)
+                        // or s Im w (ny 1: phi = -i, s = 1; ny 3: phi = i, s = -1)
+                        const double s0 = (ny & 3) < 2 ? 1.0 : -1.0;
+                        const uint32_t zl = local_bits(tm.z_mask, ps, K), zr = reg_bits(zl, st);
+                        for (int part = 0; part < 2; part++) {
+                            const double c = part ? tm.c_im : tm.c_re;
+                            if (part && c == 0.0) continue;
+                            const uint64_t zo = tm.z_mask & ~q;
+                            const uint32_t fl = part ? kExpImag : 0u;
+                            size_t e = e0;
+                            while (e < p.nunits && !(p.units[e].zo == zo && p.units[e].zl == (zl & ~r) &&
+                                                     (p.units[e].flags() & kExpImag) == fl))
+                                e++;
+                            ExpUnit &un = p.units[e];
+                            if (e == p.nunits) {
+                                memset(&un, 0, sizeof un);
+                                un.zo = zo; un.zl = zl & ~r;
+                                un.info = (xm + 16u * im_w) | xl << 16 |
+                                          (fl | (e > e0 ? kExpReuse : 0u) | (high ? kExpHigh : 0u)) << 8;
+                                p.nunits++;
+                            }
+                            // a pair is visited once (factor 2); a wide mask visits both its members
+                            const double f = (xm ? 2.0 : 1.0) * s0 * c;
+                            for (uint32_t k = 0; k < 8; k++) {
+                                const uint32_t slot =
+                                    xm ? ((k >> pivot) << (pivot + 1)) | (k & ((1u << pivot) - 1)) : k + 8u * high;
+                                un.h[k] += (popc(slot & zr) & 1) ? -f : f;
+                            }
+                        }
+                    }
+                }
+                const uint64_t x = p.xs[g]; p.xs[g] = p.xs[s_at]; p.xs[s_at] = x;
+                const uint32_t h = head[g]; head[g] = head[s_at]; head[s_at] = h;
+                s_at++;
+            }
+            st.nu = (uint32_t)p.nunits - st.u0;
+            if (pass_diag) {  // counting sort by register-bit pattern
+                pass_diag = false;
+                st.diag = 1;
+                uint32_t cnt[kExpSlots + 1] = {0};
+                for (size_t k = 0; k < nt; k++)
+                    if (!terms[k].x_mask) cnt[reg_bits(local_bits(terms[k].z_mask, ps, K), st) + 1]++;
+                for (int b = 0; b < kExpSlots; b++) cnt[b + 1] += cnt[b];
+                memcpy(st.doff, cnt, sizeof cnt);
+                for (size_t k = 0; k < nt; k++) {
+                    if (terms[k].x_mask) continue;
+                    const uint32_t zl = local_bits(terms[k].z_mask, ps, K);
+                    ExpDiag &d = p.diags[cnt[reg_bits(zl, st)]++];
+                    d.zo = terms[k].z_mask & ~q; d.zl = zl & ~r; d.pad = 0;
+                    d.re = terms[k].c_re; d.im = terms[k].c_im;
+                    p.ndiags++;
+                }
+            }
+        }
+        ps.ns = (uint32_t)p.nsets - ps.s0;
+    }
+    memset(&p.units[p.nunits], 0, sizeof(ExpUnit));
+}
+
+}  // namespace qi

@@ -1,0 +1,97 @@
+// expect_plan.h — how the expectation of a SumOp is cut into tile passes
+// (planned on the host in expect_plan.cpp, run by expect.hip).
+//
+// A tile is the 2^K amplitudes spanned by a set of K qubits. A term whose X
+// and Y factors lie inside that set needs only amplitudes of one tile, so one
+// read of the state serves every such term, whatever its Z factors. Inside a
+// tile the terms with one x mask are a group: P is Hermitian, so the pair
+// (i, i ^ x) adds c 2 Re(phi(i) conj(psi_i) psi_{i^x}) with phi(i) a sign or a
+// sign times i, and a group's terms share Re w or Im w of each pair.
+// A register set is four tile qubits whose 16 amplitudes one thread holds:
+// groups inside a set cost no memory traffic.
+#pragma once
+
+#include <cstddef>
+#include <cstdint>
+
+#include "../../include/qiron.h"
+
+#ifdef __HIP__
+#define QI_HD __host__ __device__
+#else
+#define QI_HD
+#endif
+
+namespace qi {
+
+constexpr int kExpSlots = 16;     // amplitudes per thread: four register bits
+constexpr int kExpMaxK = 13;      // tile qubits at most
+
+// One step of a register set: the signed coefficients of one x mask's terms
+// that share a Z support outside the register bits and the parity of their
+// number of Y factors: adds sign * sum_k h[k] u[k] over the 8 pairs of the
+// mask (slots with its highest bit clear), u = Re w or Im w. A mask of more
+// than four tile bits ("wide") visits both members of each pair, partners
+// read from LDS, in two units of 8 slots.
+struct ExpUnit {
+    uint64_t zo;      // Z bits outside the tile
+    uint32_t zl;      // Z bits inside the tile, outside the register bits (tile-local)
+    uint32_t info;    // (dword fields: the kernel reads its tables with scalar loads) byte 0: register-bit pattern
+                      // of the mask (1..15), 0: wide; + 16: u = Im w (odd number of Y factors); byte 1: flags
+                      // below; bits 16-31: the mask in tile-local bits
+    double h[8];
+    QI_HD uint32_t code() const { return info & 31u; }
+    QI_HD uint32_t flags() const { return (info >> 8) & 255u; }
+    QI_HD uint32_t xl() const { return info >> 16; }
+};
+enum : uint32_t {
+    kExpReuse = 1,    // the unit before has the same u
+    kExpImag = 2,     // adds to the imaginary part (imaginary parts of the coefficients)
+    kExpHigh = 4,     // wide: slots 8..15 (else 0..7)
+};
+// One diagonal term (x = 0): c (-1)^{popcount(i & z)} |psi_i|^2.
+struct ExpDiag {
+    uint64_t zo;
+    uint32_t zl;
+    uint32_t pad;
+    double re, im;
+};
+struct ExpSet {
+    uint32_t pos;       // tile-local positions of the four register bits, ascending, a byte each
+    uint32_t u0, nu;    // units
+    uint32_t diag;      // 1: the diagonal terms run here, sorted by their register-bit pattern
+    uint32_t doff[kExpSlots + 1];
+};
+struct ExpPass {
+    uint64_t qmask;     // tile qubits
+    uint32_t s0, ns;    // register sets
+    uint32_t pos[4];    // qubit of each tile-local bit, ascending, a byte each
+};
+// Byte k of a packed position list.
+QI_HD inline uint32_t exp_pos(const uint32_t *p, int k) { return (p[k >> 2] >> (8 * (k & 3))) & 255u; }
+
+// The plan, in arrays the caller owns (capacities for nt terms below).
+struct ExpPlan {
+    ExpPass *passes;    // <= nt
+    ExpSet *sets;       // <= nt
+    ExpUnit *units;     // <= 4 nt + 1 (one spare: the kernel reads a unit ahead)
+    ExpDiag *diags;     // <= nt
+    uint64_t *far;      // x masks that no tile can hold: <= nt
+    uint64_t *xs;       // scratch: the distinct x masks, <= nt
+    uint32_t *gid;      // scratch: 2 per term
+    size_t npasses, nsets, nunits, ndiags, nfar;
+    int K;              // tile qubits
+    bool complex_out;   // an imaginary part can be nonzero
+};
+// Bytes of the planning arena for nt terms.
+size_t exp_plan_bytes(size_t nt);
+// Carves the arrays out of `arena` (exp_plan_bytes(nt) bytes, 16-byte aligned).
+void exp_plan_carve(ExpPlan &p, void *arena, size_t nt);
+// Tile width for n qubits (n >= 4): the whole state up to kExpMaxK - 1 = 12
+// qubits, else 13 (complex64) or 12 (complex128) of them.
+int exp_tile_qubits(uint32_t n, bool c128);
+// Qubits 0 .. low-1 are always in a tile: 128-byte runs in memory.
+inline int exp_low_qubits(bool c128) { return c128 ? 3 : 4; }
+void plan_expect(uint32_t n, bool c128, const qi_pauli_term *terms, size_t nt, ExpPlan &p);
+
+}  // namespace qi

@@ -72,7 +72,13 @@ struct Ctx {
     // SplitMix64 stream for measurements whose uniform draw is not injected
     // (the reference draws from rand::rng(), state.rs:601-602)
     uint64_t rng = 0;
-    void *noalloc = nullptr;  // this device's copy of the no-allocation scratch array (pauli.hip)
+    void *noalloc = nullptr;  // this device's copy of the no-allocation scratch array (expect.hip)
+    // SumOp expectations: host planning arena and the pinned staging buffer of
+    // the device tables, both large enough for kNoAllocMaxTerms terms from the
+    // context's creation and grown by longer term lists
+    std::vector<unsigned char> plan_arena;
+    unsigned char *stage = nullptr;
+    size_t stage_bytes = 0;
     // cached graph of the last captured gate list
     hipGraphExec_t graph_exec = nullptr;
     std::vector<unsigned char> graph_key;
@@ -152,15 +158,17 @@ struct DiagPass {
     DiagTab tab[kDiagTabMax];
 };
 Status launch_diag_tables(State &s, const DiagPass &p, const double2 *dtables, hipStream_t st);
+// Expectation of a list of terms (expect.hip); result (re, im) summed in FP64 compensated.
+Status sumop_expectation(State &s, const qi_pauli_term *terms, size_t nt, double *re, double *im, hipStream_t st);
+size_t expect_stage_bytes(size_t nt);
+// Ctx::plan_arena and Ctx::stage of at least `bytes` bytes (no call of the context in flight).
+Status ensure_stage(Ctx &C, size_t bytes);
 // The no-allocation expectation: at most kNoAllocMaxTerms terms, all scratch in
 // a static device array whose per-device address noalloc_scratch returns.
 constexpr int kNoAllocMaxTerms = 512;
 Status noalloc_scratch(int device, void **out);
 Status sumop_expectation_noalloc(State &s, const qi_pauli_term *terms, size_t nt, double *re, double *im,
                                  hipStream_t st);
-// Expectation of a list of terms; result (re, im) summed in FP64 compensated.
-Status sumop_expectation(State &s, const qi_pauli_term *terms, size_t nt, double *re, double *im,
-                         hipStream_t st);
 
 // Measurement kernels (measure.hip)
 Status measure_probs_device(State &s, const uint64_t *qubits, uint32_t m, double **dprobs,
