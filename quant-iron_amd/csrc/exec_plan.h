@@ -154,7 +154,7 @@ struct ExecPlan {
 // the op's form: the same values plan_tiled writes for that gate at that angle.
 void param_op_coeffs(RegOp &op, double theta);
 
-int default_tile_qubits(const State &s);
+int default_tile_qubits(const State &s, int TB);  // TB: the thread bits asked for, 0 for the default
 int default_tile_threads_log2(int prec, int K);
 int tile_low_qubits(int prec);
 // Register-resident passes for one state (ExecStep::REG, plan.reg_ops).

@@ -28,7 +28,30 @@ namespace qi {
 
 int tile_low_qubits(int prec) { return prec == QI_C128 ? 3 : 4; }  // 128-byte rows
 
-int default_tile_qubits(const State &s) { return s.prec == QI_C128 ? 11 : 12; }
+// Wide tiles take more gates per HBM round trip, narrow ones give more waves
+// with shorter op bodies. A small state leaves most of the chip idle with wide
+// tiles (18 qubits in 2^12 tiles: 64 waves for 1024 SIMDs), and a pass lasts
+// as long as one wave walks its ops. Device time of the one-wave executor in
+// us, tiles of 2^10 / 2^11 / 2^12 (an ansatz of 6 layers; a random circuit of
+// depth 10):
+//   complex64   18 qubits  168 / 216 / 306;   110 / 127 / 189
+//               21         313 / 336 / 422;   173 / 163 / 217
+//               22         413 / 395 / 488;   214 / 209 / 268
+//               24        1333 / 1150 / 1247;  778 / 690 / 736
+//               25        2520 / 2246 / 2167; 1411 / 1169 / 1281
+//   complex128  18         208 / 294;          121 / 171
+//               21         363 / 432;          199 / 233
+//               22         605 / 608;          348 / 323
+//               24        2231 / 2040;        1307 / 1231
+// A thread count asked for keeps the widest tile, which it was chosen for;
+// states smaller than that stream gate by gate.
+int default_tile_qubits(const State &s, int TB) {
+    const bool c128 = s.prec == QI_C128;
+    const int widest = c128 ? 11 : 12;
+    if (TB > 0 || (int)s.n < widest) return widest;
+    if (s.n <= 21) return 10;
+    return c128 || s.n >= 25 ? widest : 11;
+}
 
 // Tiles of up to 4096 complex64 / 2048 complex128 amplitudes run as one wave
 // (no LDS, no barriers, 64 / 32 amplitudes per lane, the per-op scalar work
@@ -775,7 +798,7 @@ struct Phase {
 }  // namespace
 
 static Status plan_tiled_list(const State &s, const std::vector<Lowered> &gates, int K, int TB, ExecPlan &plan) {
-    if (K <= 0) K = default_tile_qubits(s);
+    if (K <= 0) K = default_tile_qubits(s, TB);
     if (TB <= 0) TB = default_tile_threads_log2(s.prec, K);
     if (TB != 6 && TB != 8 && TB != 9) return make_err(QI_ERR_INVALID_ARGUMENT, 0, 0, 0, 0, "tile threads out of range");
     const int kmax = s.prec == QI_C128 ? 12 : 13;
@@ -1138,7 +1161,7 @@ Status plan_tiled(const State &s, const std::vector<Lowered> &gates, int K, int 
     Status st = plan_tiled_list(s, gates, K, TB, best);
     if (!st.ok()) return st;
     const bool any = std::any_of(gates.begin(), gates.end(), is_relabel);
-    const int Kr = K <= 0 ? default_tile_qubits(s) : K;
+    const int Kr = K <= 0 ? default_tile_qubits(s, TB) : K;
     if (any && (int)s.n >= Kr) {
         for (int order = 0; order < 2; order++) {
             ExecPlan alt;
@@ -1191,7 +1214,7 @@ void param_op_coeffs(RegOp &op, double theta) {
 
 // ------------------------------------------------------------- LDS passes --
 Status plan_lds_passes(const State &s, const std::vector<Lowered> &gates, int K, ExecPlan &plan) {
-    if (K <= 0) K = default_tile_qubits(s);
+    if (K <= 0) K = default_tile_qubits(s, 0);
     const int kmax = s.prec == QI_C128 ? 12 : 13;
     if (K < 10 || K > kmax) return make_err(QI_ERR_INVALID_ARGUMENT, 0, 0, 0, 0, "tile width out of range");
     if ((int)s.n < K) {
