@@ -362,8 +362,9 @@ static Status run_maybe_graph(Ctx &C, State &s, bool use_graph, const void *key,
 // the chosen executor, other Gate variants (measurement, Pauli strings) become
 // host-orchestrated steps between them.
 // `slots` (may be NULL): the angle slot of each gate, -1 for none (parametric circuits).
+// `small`: runs of two gates or more on a state of one workgroup's size go in one launch.
 static Status build_plan(State &s, const qi_gate *gates, size_t ng, int mode, const qi_exec_opts &o, ExecPlan &plan,
-                         const int32_t *slots = nullptr, bool allow_oop = false) {
+                         const int32_t *slots = nullptr, bool allow_oop = false, bool small = false) {
     size_t k = 0;
     while (k < ng) {
         if (!is_operator(gates[k].kind)) { plan.steps.push_back(ExecStep::host(k)); k++; continue; }
@@ -380,7 +381,14 @@ static Status build_plan(State &s, const qi_gate *gates, size_t ng, int mode, co
         Status e;
         if (mode == QI_EXEC_TILED) e = plan_tiled(s, seg, o.tile_qubits, o.tile_threads_log2, plan, allow_oop);
         else if (mode == QI_EXEC_FUSED_MFMA) e = plan_fused(s, seg, o.block_qubits, plan);
-        else for (const Lowered &L : seg) plan.steps.push_back(ExecStep::gate(L));
+        else if (small && seg.size() > 1) {
+            ExecStep st;
+            st.type = ExecStep::SMALL;
+            st.op0 = (int32_t)plan.small_ops.size();
+            st.nops = (int32_t)seg.size();
+            for (const Lowered &L : seg) plan.small_ops.push_back(small_op(L, s.n));
+            plan.steps.push_back(st);
+        } else for (const Lowered &L : seg) plan.steps.push_back(ExecStep::gate(L));
         if (!e.ok()) return e;
         k = j;
     }
@@ -403,6 +411,9 @@ static Status launch_plan(State &s, const ExecPlan &plan, const qi_gate *gates, 
         on.d = cur;
         switch (step.type) {
         case ExecStep::GATE: e = launch_gate(on, step.L, st); break;
+        case ExecStep::SMALL:
+            e = launch_small_gates(on, (const SmallOp *)((const unsigned char *)blob + plan.small_offset()) + step.op0, step.nops, st);
+            break;
         case ExecStep::REG: {
             void *dst = cur;
             if (step.reg.oop) {
@@ -442,6 +453,7 @@ static Status apply_gates(State &s, uint32_t n_circuit, const qi_gate *gates, si
     if (opts) o = *opts;
     if (o.mode < QI_EXEC_PER_GATE || o.mode > QI_EXEC_AUTO) return make_err(QI_ERR_INVALID_ARGUMENT, 0, 0, 0, 0, "exec mode");
     int mode = o.mode;
+    const bool small = mode == QI_EXEC_AUTO && s.n <= kSmallQubits;
     if (mode == QI_EXEC_AUTO) mode = s.n >= 12 ? QI_EXEC_TILED : QI_EXEC_PER_GATE;
     bool all_ops = true;
     for (size_t k = 0; k < ng; k++) all_ops = all_ops && is_operator(gates[k].kind);
@@ -477,19 +489,22 @@ static Status apply_gates(State &s, uint32_t n_circuit, const qi_gate *gates, si
         plan = std::static_pointer_cast<ExecPlan>(C.cached_plan);
     } else {
         plan = std::make_shared<ExecPlan>();
-        Status e = build_plan(s, gates, ng, mode, o, *plan, nullptr, allow_oop);
+        Status e = build_plan(s, gates, ng, mode, o, *plan, nullptr, allow_oop, small);
         if (!e.ok()) return e;
         C.cached_plan.reset();
         C.plan_key.clear();
         if (plan->blob_bytes() > 0) {
             if (!(e = ensure(C.plan, plan->blob_bytes())).ok()) return e;
-            QI_HIP_TRY(hipStreamSynchronize(C.stream));  // the previous plan may still be in use
             // a cached graph reads the op table about to be overwritten
             if (C.graph_exec) { (void)hipGraphExecDestroy(C.graph_exec); C.graph_exec = nullptr; C.graph_key.clear(); }
-            std::vector<unsigned char> blob(plan->blob_bytes(), 0);
-            if (!plan->reg_ops.empty()) memcpy(blob.data(), plan->reg_ops.data(), plan->reg_ops.size() * sizeof(RegOp));
-            if (!plan->mats.empty()) memcpy(blob.data() + plan->mats_offset(), plan->mats.data(), plan->mats.size());
-            QI_HIP_TRY(hipMemcpy(C.plan.p, blob.data(), blob.size(), hipMemcpyHostToDevice));
+            // through the pinned staging buffer (idle between calls); the stream
+            // orders the copy after the previous plan's launches
+            if (!(e = ensure_stage(C, plan->blob_bytes())).ok()) return e;
+            if (!plan->reg_ops.empty()) memcpy(C.stage, plan->reg_ops.data(), plan->reg_ops.size() * sizeof(RegOp));
+            if (!plan->mats.empty()) memcpy(C.stage + plan->mats_offset(), plan->mats.data(), plan->mats.size());
+            if (!plan->small_ops.empty())
+                memcpy(C.stage + plan->small_offset(), plan->small_ops.data(), plan->small_ops.size() * sizeof(SmallOp));
+            QI_HIP_TRY(hipMemcpyAsync(C.plan.p, C.stage, plan->blob_bytes(), hipMemcpyHostToDevice, C.stream));
         }
         C.cached_plan = plan;
         C.plan_key = key;

@@ -128,12 +128,13 @@ struct FusedBlock {
 };
 
 struct ExecStep {
-    enum Type { GATE = 0, TILE = 1, FUSED = 2, HOST = 3, REG = 4 } type = GATE;
+    enum Type { GATE = 0, TILE = 1, FUSED = 2, HOST = 3, REG = 4, SMALL = 5 } type = GATE;
     Lowered L;
     TilePass tile{};
     RegPass reg{};
     FusedBlock fused{};
     size_t host_gate = 0;  // index into the caller's gate list (HOST)
+    int32_t op0 = 0, nops = 0;  // slice of the plan's small_ops (SMALL)
     static ExecStep gate(const Lowered &l) { ExecStep s; s.type = GATE; s.L = l; return s; }
     static ExecStep tile_step(const TilePass &p) { ExecStep s; s.type = TILE; s.tile = p; return s; }
     static ExecStep fused_step(const FusedBlock &b) { ExecStep s; s.type = FUSED; s.fused = b; return s; }
@@ -146,8 +147,10 @@ struct ExecPlan {
     std::vector<TileOp> tile_ops;          // LDS passes (batched engine; uploaded by it)
     std::vector<RegOp> reg_ops;            // uploaded first in the blob
     std::vector<unsigned char> mats;       // fused matrices, after the register-pass ops
+    std::vector<SmallOp> small_ops;        // last in the blob
     size_t mats_offset() const { return (reg_ops.size() * sizeof(RegOp) + 255) & ~size_t(255); }
-    size_t blob_bytes() const { return mats_offset() + mats.size(); }
+    size_t small_offset() const { return (mats_offset() + mats.size() + 255) & ~size_t(255); }
+    size_t blob_bytes() const { return small_offset() + small_ops.size() * sizeof(SmallOp); }
 };
 
 // Coefficients of a parametric op (RegOp::param > 0) for the angle theta, in

@@ -123,6 +123,16 @@ struct Lowered {
 Status validate_gate(uint32_t n, const qi_gate &g);
 Status lower_gate(uint32_t n, const qi_gate &g, Lowered &out);
 Status launch_gate(State &s, const Lowered &L, hipStream_t st);
+// States of at most this many qubits fit one workgroup's LDS: a gate list runs
+// as one launch (launch_small_gates).
+constexpr uint32_t kSmallQubits = 11;
+struct SmallOp {      // a lowered gate's index sets (GateK in gates.hip), for a state of at most kSmallQubits
+    int32_t kind;     // LoweredKind
+    uint32_t items, fixed, set, pmask, tb, tb2, cmask;
+    double c[8];
+};
+SmallOp small_op(const Lowered &L, uint32_t n);
+Status launch_small_gates(State &s, const SmallOp *dops, int nops, hipStream_t st);
 
 // ------------------------------------------------------- misc kernels ------
 Status launch_init(State &s, int kind, uint64_t basis, hipStream_t st);
