@@ -557,8 +557,10 @@ __global__ __launch_bounds__(512) void k_small_gates(typename V2<R>::T *__restri
         for (int w = threadIdx.x; w < cnt * W; w += blockDim.x)
             reinterpret_cast<f32x4 *>(sops)[w] = reinterpret_cast<const f32x4 *>(ops + o0)[w];
         __syncthreads();
+        SmallOp nxt = sops[0];
         for (int o = 0; o < cnt; o++) {
-            const SmallOp &op = sops[o];
+            const SmallOp op = nxt;
+            nxt = sops[o + 1 < cnt ? o + 1 : o];  // read while this op runs
             auto u = [](uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); };
             const uint32_t items = u(op.items), fixed = u(op.fixed), set = u(op.set), pmask = u(op.pmask);
             GateK<R> g;

@@ -15,6 +15,7 @@
 #include <cmath>
 #include <memory>
 #include <random>
+#include <type_traits>
 #include <vector>
 
 #include "qi_internal.h"
@@ -577,14 +578,11 @@ __device__ __forceinline__ void store_angle_pair(bf16 *row, int nang, int j, flo
 // padding. The inputs are rounded to BF16, so the trigonometry runs in FP32
 // (the host regenerates the kept candidates' angles in FP64 for the exact
 // evaluation).
-__global__ __launch_bounds__(256) void k_ansatz_features(uint64_t seed, uint64_t draw0, uint64_t count, uint64_t c0, int rows,
-                                                         int nang, int k_in, bf16 *__restrict__ X) {
-    const uint32_t pairs = (uint32_t(nang) + 1) / 2, per = pairs + 1, items = uint32_t(rows) * per;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < items; i += gridDim.x * blockDim.x) {
-        const uint32_t r = i / per, p = i - r * per;
-        const uint64_t c = c0 + r;
-        bf16 *row = X + size_t(r) * k_in;
-        if (p < pairs) {
+struct UniformCandidates {
+    uint64_t seed, draw0, count;
+    int nang;
+    __device__ __forceinline__ void item(uint64_t c, uint32_t p, bf16 *row, int width) const {
+        if (p < (uint32_t(nang) + 1) / 2) {
             const int j = 2 * int(p);
             const bool two = j + 1 < nang;
             float sa, ca, sb = 0.f, cb = 0.f;
@@ -594,10 +592,10 @@ __global__ __launch_bounds__(256) void k_ansatz_features(uint64_t seed, uint64_t
         } else {
             for (int q = 0; q < 3; q++)
                 row[2 * nang + q] = f2bf((float)(0.5 + sm64_uniform(seed, draw0 + count * nang + 3 * c + q + 1) - 1.0));
-            for (int k = 2 * nang + 3; k < k_in; k++) row[k] = f2bf(0.f);
+            for (int k = 2 * nang + 3; k < width; k++) row[k] = f2bf(0.f);
         }
     }
-}
+};
 
 // Candidates of an optimisation round around a centre theta0 (a local
 // proposal): theta_j = theta0_j + sigma z_j with standard normals from the
@@ -606,15 +604,14 @@ __global__ __launch_bounds__(256) void k_ansatz_features(uint64_t seed, uint64_t
 // d = draw0 + 2 (c P + p), P = ceil(nang / 2), rho = sqrt(-2 ln(1 - u1)),
 // z_2p = rho cos(2 pi u2), z_2p+1 = rho sin(2 pi u2); the couplings are the
 // fixed J of the round. Same row layout and items as k_ansatz_features.
-__global__ __launch_bounds__(256) void k_ansatz_features_local(uint64_t seed, uint64_t draw0, uint64_t c0, int rows, int nang,
-                                                               int k_in, const double *__restrict__ theta0, double sigma,
-                                                               double j0, double j1, double j2, bf16 *__restrict__ X) {
-    const uint32_t pairs = (uint32_t(nang) + 1) / 2, per = pairs + 1, items = uint32_t(rows) * per;
-    const float inv2pi = 0.15915494309189535f, sg = (float)sigma;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < items; i += gridDim.x * blockDim.x) {
-        const uint32_t r = i / per, p = i - r * per;
-        const uint64_t c = c0 + r;
-        bf16 *row = X + size_t(r) * k_in;
+struct LocalCandidates {
+    uint64_t seed, draw0;
+    int nang;
+    const double *theta0;
+    double sigma, j0, j1, j2;
+    __device__ __forceinline__ void item(uint64_t c, uint32_t p, bf16 *row, int width) const {
+        const uint32_t pairs = (uint32_t(nang) + 1) / 2;
+        const float inv2pi = 0.15915494309189535f, sg = (float)sigma;
         if (p < pairs) {
             const int j = 2 * int(p);
             const bool two = j + 1 < nang;
@@ -631,8 +628,172 @@ __global__ __launch_bounds__(256) void k_ansatz_features_local(uint64_t seed, ui
             row[2 * nang] = f2bf((float)(j0 - 1.0));
             row[2 * nang + 1] = f2bf((float)(j1 - 1.0));
             row[2 * nang + 2] = f2bf((float)(j2 - 1.0));
-            for (int k = 2 * nang + 3; k < k_in; k++) row[k] = f2bf(0.f);
+            for (int k = 2 * nang + 3; k < width; k++) row[k] = f2bf(0.f);
         }
+    }
+};
+
+// The features of candidates c0 .. c0 + rows as a matrix (rows x k_in).
+template <typename F>
+__global__ __launch_bounds__(256) void k_ansatz_features(F f, uint64_t c0, int rows, int k_in, bf16 *__restrict__ X) {
+    const uint32_t per = (uint32_t(f.nang) + 1) / 2 + 1, items = uint32_t(rows) * per;
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < items; i += gridDim.x * blockDim.x) {
+        const uint32_t r = i / per, p = i - r * per;
+        f.item(c0 + r, p, X + size_t(r) * k_in, k_in);
+    }
+}
+
+// ------------------------------------------------------ fused prediction --
+// Inputs already in memory (rows x k_in).
+struct StagedRows {
+    const bf16 *X;
+    int k_in;
+};
+
+// W1^T, W2^T, W3^T (rows = outputs, K contiguous) as the matrix instruction's
+// first operand, one contiguous 1 KiB per 32 x 16 fragment: fragment (k step,
+// column tile), lane l holds column l % 16, k = 8 (l / 16) .. + 7; K padded
+// with zeros to whole steps.
+struct PackLayers {
+    size_t off[3];  // of W^T in wt
+    int k_in, H;
+};
+__global__ __launch_bounds__(256) void k_pack_weights(const bf16 *__restrict__ wt, PackLayers L, bf16 *__restrict__ out) {
+    const int l = blockIdx.y, H = L.H, ld = l ? H : L.k_in, steps = (ld + 31) / 32;
+    const int chunk = blockIdx.x * 256 + threadIdx.x, tiles = H / 16;
+    if (chunk >= steps * tiles * 64) return;
+    wt += L.off[l];
+    if (l) out += (size_t((L.k_in + 31) / 32 * 32) + size_t(l - 1) * H) * H;
+    const int lane = chunk & 63, ct = (chunk >> 6) % tiles, ks = (chunk >> 6) / tiles;
+    const int n = ct * 16 + (lane & 15), k = ks * 32 + 8 * (lane >> 4);
+    uint4 v = make_uint4(0, 0, 0, 0);
+    if (k < ld) v = *reinterpret_cast<const uint4 *>(wt + size_t(n) * ld + k);
+    reinterpret_cast<uint4 *>(out)[chunk] = v;
+}
+
+// acc += A (64 rows in LDS, stride lda) times this wave's 16 NJ columns of a
+// packed layer of `steps` k steps over `tiles` column tiles. A step's weights
+// are loaded one step ahead; k runs in ascending order, as in k_gemm.
+template <int NJ>
+__device__ __forceinline__ void mlp_layer(floatx4 (&acc)[4][NJ], const bf16 *A, int lda, const bf16 *__restrict__ wp, int steps) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint4 *w = reinterpret_cast<const uint4 *>(wp) + size_t(wave) * NJ * 64 + lane;
+    constexpr int step_words = 4 * NJ * 64;
+    const bf16 *a0 = A + (lane & 15) * lda + 8 * (lane >> 4);
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++) acc[i][j] = floatx4{0, 0, 0, 0};
+    auto load = [&](uint4 (&b)[NJ], int ks) {
+#pragma unroll
+        for (int j = 0; j < NJ; j++) b[j] = w[size_t(ks) * step_words + j * 64];
+    };
+    auto step = [&](const uint4 (&b)[NJ], int ks) {
+        bf16x8 a[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) a[i] = *reinterpret_cast<const bf16x8 *>(a0 + i * 16 * lda + ks * 32);
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int j = 0; j < NJ; j++)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, b[j]), a[i], acc[i][j], 0, 0, 0);
+    };
+    uint4 b0[NJ], b1[NJ];
+    load(b0, 0);
+    int ks = 0;
+    for (; ks + 2 <= steps; ks += 2) {
+        load(b1, ks + 1);
+        step(b0, ks);
+        if (ks + 2 < steps) load(b0, ks + 2);
+        step(b1, ks + 1);
+    }
+    if (ks < steps) step(b0, ks);
+}
+
+// The whole network for 64 rows per workgroup: inputs generated or loaded into
+// LDS, three layers through LDS (a wave owns 16 NJ of the H = 64 NJ columns and
+// keeps their 64 x 16 NJ outputs in registers until every wave has read the
+// layer's inputs), the head from the third layer's registers. Activations never
+// reach HBM; the weights come from L2 once per workgroup. Two workgroups per CU,
+// so one's GELU and input arithmetic runs under the other's matrix
+// instructions; matrix and vector issue are about even. Sums run in the order
+// of the layer-by-layer path (the same bits), which wrote and read 0.5 GB of
+// activations per layer. 2^19 candidates, 387 inputs, width 512: 1.05 ms
+// (724 TFLOP/s), layer by layer 1.98 ms; 4096 candidates: 101 against 115 us
+// with the call around it, so every size of these widths takes this kernel.
+template <int NJ, typename F>
+__global__ __launch_bounds__(256, 2) void k_mlp_rows(F f, uint64_t c0, uint64_t rows, int k_in, int lda, const bf16 *__restrict__ wp,
+                                                     const float *__restrict__ b1, const float *__restrict__ b2,
+                                                     const float *__restrict__ b3, const float *__restrict__ w4,
+                                                     const float *__restrict__ b4, float *__restrict__ y) {
+    constexpr int H = 64 * NJ;
+    extern __shared__ __attribute__((aligned(16))) unsigned char mlp_lds[];
+    bf16 *const A = reinterpret_cast<bf16 *>(mlp_lds);
+    float *const head = reinterpret_cast<float *>(mlp_lds + size_t(64) * lda * sizeof(bf16));  // 4 x 64
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint64_t r0 = uint64_t(blockIdx.x) * 64;
+    const int steps1 = (k_in + 31) / 32, width = 32 * steps1;
+    if constexpr (std::is_same<F, StagedRows>::value) {
+        for (int i = tid; i < 64 * (width / 8); i += 256) {
+            const int r = i / (width / 8), k = 8 * (i - r * (width / 8));
+            uint4 v = make_uint4(0, 0, 0, 0);
+            if (r0 + r < rows && k < k_in) v = *reinterpret_cast<const uint4 *>(f.X + (r0 + r) * k_in + k);
+            *reinterpret_cast<uint4 *>(A + r * lda + k) = v;
+        }
+    } else {
+        const uint32_t per = (uint32_t(f.nang) + 1) / 2 + 1;
+        for (uint32_t i = tid; i < 64 * per; i += 256) {
+            const uint32_t r = i / per, p = i - r * per;
+            f.item(c0 + r0 + r, p, A + r * lda, width);
+        }
+    }
+    __syncthreads();
+    floatx4 acc[4][NJ];
+#pragma unroll
+    for (int l = 0; l < 2; l++) {
+        mlp_layer<NJ>(acc, A, lda, wp, l ? H / 32 : steps1);
+        wp += size_t(l ? H : width) * H;
+        __syncthreads();
+        const float *bias = l ? b2 : b1;
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+            const int col = wave * 16 * NJ + j * 16 + 4 * (lane >> 4);
+            const float4 bb = *reinterpret_cast<const float4 *>(bias + col);
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                float v[4] = {acc[i][j][0] + bb.x, acc[i][j][1] + bb.y, acc[i][j][2] + bb.z, acc[i][j][3] + bb.w};
+#pragma unroll
+                for (int r = 0; r < 4; r++) v[r] = gelu_fwd(v[r]);
+                *reinterpret_cast<uint2 *>(A + (i * 16 + (lane & 15)) * lda + col) = pack_bf16x4(v);
+            }
+        }
+        __syncthreads();
+    }
+    mlp_layer<NJ>(acc, A, lda, wp, H / 32);
+    float hs[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < NJ; j++) {
+        const int col = wave * 16 * NJ + j * 16 + 4 * (lane >> 4);
+        const float4 bb = *reinterpret_cast<const float4 *>(b3 + col), w = *reinterpret_cast<const float4 *>(w4 + col);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            hs[i] += gelu_fwd(acc[i][j][0] + bb.x) * w.x;
+            hs[i] += gelu_fwd(acc[i][j][1] + bb.y) * w.y;
+            hs[i] += gelu_fwd(acc[i][j][2] + bb.z) * w.z;
+            hs[i] += gelu_fwd(acc[i][j][3] + bb.w) * w.w;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        hs[i] += __shfl_xor(hs[i], 16);
+        hs[i] += __shfl_xor(hs[i], 32);
+        if (lane < 16) head[wave * 64 + i * 16 + lane] = hs[i];
+    }
+    __syncthreads();
+    if (tid < 64 && r0 + tid < rows) {
+        float s = 0.f;
+        for (int k = 0; k < 4; k++) s += head[k * 64 + tid];
+        y[r0 + tid] = s + *b4;
     }
 }
 
@@ -649,6 +810,7 @@ struct Mlp {
     float *w = nullptr, *m = nullptr, *v = nullptr, *g = nullptr;  // FP32 masters, Adam moments, grads
     bf16 *wb = nullptr;                                            // BF16 copies (W1, W2, W3)
     bf16 *wt = nullptr;                                            // BF16 W1^T, W2^T, W3^T (same offsets)
+    bf16 *wp = nullptr;                                            // the same as matrix-instruction fragments (prediction)
     int step = 0;
     // activations for a batch of up to cap rows
     size_t cap = 0;
@@ -669,7 +831,7 @@ struct Mlp {
     uint32_t *perm = nullptr;
     size_t ndata = 0;
     ~Mlp() {
-        void *ps[] = {w, m, v, g, wb, wt, X, H[0], H[1], H[2], dZb[0], dZb[1], dZb[2], Z[0], Z[1], Z[2], dZf[0], dZf[1], dZf[2],
+        void *ps[] = {w, m, v, g, wb, wt, wp, X, H[0], H[1], H[2], dZb[0], dZb[1], dZb[2], Z[0], Z[1], Z[2], dZf[0], dZf[1], dZf[2],
                       y, t, dy, part, lossp, T1, T2, ws, dataX, dataT, perm, lacc, yall, theta0};
         for (void *p : ps)
             if (p) (void)hipFree(p);
@@ -791,6 +953,47 @@ static void refresh_bf16(Mlp &N, hipStream_t st) {
     }
 }
 
+// Hidden widths the fused prediction kernel is built for (16 NJ columns per
+// wave), and inputs that fit its LDS rows beside a second workgroup.
+static bool fused_predict(const Mlp &N) { return (N.hid == 512 || N.hid == 256) && N.k_in <= 576; }
+// Dynamic LDS above 64 KiB has to be allowed per kernel (and device).
+template <typename F> static Status allow_lds() {
+    QI_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(k_mlp_rows<8, F>), hipFuncAttributeMaxDynamicSharedMemorySize, 81920));
+    QI_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(k_mlp_rows<4, F>), hipFuncAttributeMaxDynamicSharedMemorySize, 81920));
+    return Status{};
+}
+
+static size_t packed_words(const Mlp &N) { return size_t((N.k_in + 31) / 32 * 32 + 2 * N.hid) * N.hid; }
+static Status alloc_packed(Mlp &N) {
+    if (N.wp) return Status{};
+    Status e = allow_lds<StagedRows>();
+    if (e.ok()) e = allow_lds<UniformCandidates>();
+    if (e.ok()) e = allow_lds<LocalCandidates>();
+    if (!e.ok()) return e;
+    const hipError_t he = hipMalloc(&N.wp, packed_words(N) * sizeof(bf16));
+    if (he != hipSuccess) { N.wp = nullptr; return oom_err(he); }
+    return Status{};
+}
+// The packed weights of the current parameters (once per call: a few microseconds).
+static void pack_weights(Mlp &N, hipStream_t st) {
+    const PackLayers L{{N.off[0], N.off[2], N.off[4]}, N.k_in, N.hid};
+    const int steps = (std::max(N.k_in, N.hid) + 31) / 32;
+    hipLaunchKernelGGL(k_pack_weights, dim3((unsigned)((steps * (N.hid / 16) * 64 + 255) / 256), 3), dim3(256), 0, st,
+                       (const bf16 *)N.wt, L, N.wp);
+}
+// Predictions of `rows` rows of the source f (candidates from c0).
+template <typename F> static void predict_fused(Mlp &N, hipStream_t st, const F &f, uint64_t c0, uint64_t rows, float *y) {
+    const int lda = std::max((N.k_in + 31) / 32 * 32, N.hid) + 8;
+    const size_t lds = size_t(64) * lda * sizeof(bf16) + 4 * 64 * sizeof(float);
+    const float *b1 = N.w + N.off[1], *b2 = N.w + N.off[3], *b3 = N.w + N.off[5], *w4 = N.w + N.off[6], *b4 = N.w + N.off[7];
+    auto *const kernel = N.hid == 512 ? k_mlp_rows<8, F> : k_mlp_rows<4, F>;
+    const uint64_t per = uint64_t(1) << 22;  // workgroups per launch (2^30 work items)
+    for (uint64_t g0 = 0; g0 * 64 < rows; g0 += per) {
+        const uint64_t left = rows - g0 * 64, blocks = std::min<uint64_t>(per, (left + 63) / 64);
+        hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), lds, st, f, c0 + g0 * 64, left, N.k_in, lda,
+                           (const bf16 *)N.wp, b1, b2, b3, w4, b4, y + g0 * 64);
+    }
+}
 // Forward over rows already staged in N.X; keeps Z (pre-activations) when training.
 // C = X W with B^T = W^T stored K-contiguous (the fast operand layout).
 // Predictions y for `rows` staged rows: layers 1 and 2, then layer 3 with the
@@ -1062,6 +1265,7 @@ qi_status qi_mlp_predict(qi_mlp_t m, const float *x, size_t rows, float *y, qi_e
     hipStream_t st = N.ctx->stream;
     const size_t chunk = 65536;
     QM_TRY(mlp_alloc(N, std::min(chunk, std::max<size_t>(rows, 1))));
+    if (fused_predict(N)) QM_TRY(alloc_packed(N));
     hipError_t e = hipSuccess;
     double dev_ms = 0.0;
     for (size_t r0 = 0; r0 < rows; r0 += chunk) {
@@ -1069,7 +1273,12 @@ qi_status qi_mlp_predict(qi_mlp_t m, const float *x, size_t rows, float *y, qi_e
         QM_TRY(stage_rows(N, st, x + r0 * N.n_in, nullptr, nr));
         hipEvent_t a = N.ctx->ev0, b = N.ctx->ev1;
         (void)hipEventRecord(a, st);
-        predict_rows(N, st, (int)nr, N.y);
+        if (fused_predict(N)) {
+            pack_weights(N, st);
+            predict_fused(N, st, StagedRows{N.X, N.k_in}, 0, nr, N.y);
+        } else {
+            predict_rows(N, st, (int)nr, N.y);
+        }
         (void)hipEventRecord(b, st);
         if ((e = hipMemcpyAsync(y + r0, N.y, nr * 4, hipMemcpyDeviceToHost, st))) break;
         if ((e = hipStreamSynchronize(st))) break;
@@ -1093,7 +1302,9 @@ qi_status qi_mlp_predict_ansatz(qi_mlp_t m, uint64_t seed, uint64_t draw0, uint6
     std::lock_guard<std::mutex> lk(N.ctx->mu);
     hipStream_t st = N.ctx->stream;
     const size_t chunk = std::min<size_t>(kScreenChunk, (size_t(1) << 31) / (size_t(nang) + 1));  // 32-bit item indices
-    QM_TRY(mlp_alloc(N, std::min<size_t>(chunk, count)));
+    const bool fused = fused_predict(N);
+    if (fused) QM_TRY(alloc_packed(N));
+    else QM_TRY(mlp_alloc(N, std::min<size_t>(chunk, count)));
     hipError_t e;
     if (count > N.ycap) {
         if (N.yall) (void)hipFree(N.yall);
@@ -1102,12 +1313,17 @@ qi_status qi_mlp_predict_ansatz(qi_mlp_t m, uint64_t seed, uint64_t draw0, uint6
         if ((e = hipMalloc(&N.yall, count * sizeof(float)))) QM_RET(oom_err(e));
         N.ycap = count;
     }
+    const UniformCandidates f{seed, draw0, count, (int)nang};
     (void)hipEventRecord(N.ctx->ev0, st);
-    for (uint64_t c0 = 0; c0 < count; c0 += chunk) {
+    if (fused) {
+        pack_weights(N, st);
+        predict_fused(N, st, f, 0, count, N.yall);
+    }
+    for (uint64_t c0 = 0; !fused && c0 < count; c0 += chunk) {
         const int nr = (int)std::min<uint64_t>(chunk, count - c0);
         const size_t items = size_t(nr) * ((nang + 1) / 2 + 1);
-        hipLaunchKernelGGL(k_ansatz_features, dim3((unsigned)std::min<size_t>((items + 255) / 256, 16384)), dim3(256), 0, st, seed,
-                           draw0, count, c0, nr, (int)nang, N.k_in, N.X);
+        hipLaunchKernelGGL(k_ansatz_features<UniformCandidates>, dim3((unsigned)std::min<size_t>((items + 255) / 256, 16384)),
+                           dim3(256), 0, st, f, c0, nr, N.k_in, N.X);
         predict_rows(N, st, nr, N.yall + c0);
     }
     (void)hipEventRecord(N.ctx->ev1, st);
@@ -1130,7 +1346,9 @@ qi_status qi_mlp_predict_ansatz_local(qi_mlp_t m, uint64_t seed, uint64_t draw0,
     std::lock_guard<std::mutex> lk(N.ctx->mu);
     hipStream_t st = N.ctx->stream;
     const size_t chunk = std::min<size_t>(kScreenChunk, (size_t(1) << 31) / (size_t(nang) + 1));  // 32-bit item indices
-    QM_TRY(mlp_alloc(N, std::min<size_t>(chunk, count)));
+    const bool fused = fused_predict(N);
+    if (fused) QM_TRY(alloc_packed(N));
+    else QM_TRY(mlp_alloc(N, std::min<size_t>(chunk, count)));
     hipError_t e;
     if (count > N.ycap) {
         if (N.yall) (void)hipFree(N.yall);
@@ -1148,12 +1366,17 @@ qi_status qi_mlp_predict_ansatz_local(qi_mlp_t m, uint64_t seed, uint64_t draw0,
     }
     if ((e = hipMemcpyAsync(N.theta0, theta0, nang * sizeof(double), hipMemcpyHostToDevice, st)))
         QM_RET(make_err(QI_ERR_DEVICE, 0, 0, 0, 0, hipGetErrorString(e)));
+    const LocalCandidates f{seed, draw0, (int)nang, N.theta0, sigma, J[0], J[1], J[2]};
     (void)hipEventRecord(N.ctx->ev0, st);
-    for (uint64_t c0 = 0; c0 < count; c0 += chunk) {
+    if (fused) {
+        pack_weights(N, st);
+        predict_fused(N, st, f, 0, count, N.yall);
+    }
+    for (uint64_t c0 = 0; !fused && c0 < count; c0 += chunk) {
         const int nr = (int)std::min<uint64_t>(chunk, count - c0);
         const size_t items = size_t(nr) * ((nang + 1) / 2 + 1);
-        hipLaunchKernelGGL(k_ansatz_features_local, dim3((unsigned)std::min<size_t>((items + 255) / 256, 16384)), dim3(256), 0, st,
-                           seed, draw0, c0, nr, (int)nang, N.k_in, (const double *)N.theta0, sigma, J[0], J[1], J[2], N.X);
+        hipLaunchKernelGGL(k_ansatz_features<LocalCandidates>, dim3((unsigned)std::min<size_t>((items + 255) / 256, 16384)),
+                           dim3(256), 0, st, f, c0, nr, N.k_in, N.X);
         predict_rows(N, st, nr, N.yall + c0);
     }
     (void)hipEventRecord(N.ctx->ev1, st);
