@@ -1,6 +1,7 @@
 // api.hip — the C ABI (include/qiron.h): validation, error payloads, state
 // handles and the host-side orchestration of the kernels. Every entry point
 // locks its context's mutex and runs on the context's single in-order stream.
+#include <algorithm>
 #include <cfloat>
 #include <cmath>
 #include <cstdio>
@@ -21,6 +22,73 @@ void fill_err(qi_error *err, const Status &st) {
     snprintf(err->msg, sizeof err->msg, "%s", st.msg.c_str());
 }
 
+// ----------------------------------------------------------- state buffers --
+void *IdleBuffers::take(size_t want) {
+    std::lock_guard<std::mutex> lk(mu);
+    for (size_t k = idle.size(); k-- > 0;)
+        if (idle[k].bytes == want) {
+            void *p = idle[k].p;
+            idle.erase(idle.begin() + (ptrdiff_t)k);
+            bytes -= want;
+            return p;
+        }
+    return nullptr;
+}
+void IdleBuffers::put(void *p, size_t size) {
+    if (!p) return;
+    std::lock_guard<std::mutex> lk(mu);
+    if (size > kIdleBytes) { (void)hipFree(p); return; }
+    while (!idle.empty() && (bytes + size > kIdleBytes || idle.size() >= kIdleBuffers)) {
+        (void)hipFree(idle.front().p);
+        bytes -= idle.front().bytes;
+        idle.erase(idle.begin());
+    }
+    idle.push_back(DevBuf{p, size});
+    bytes += size;
+}
+void IdleBuffers::release() {
+    std::lock_guard<std::mutex> lk(mu);
+    for (DevBuf &b : idle) (void)hipFree(b.p);
+    idle.clear();
+    bytes = 0;
+}
+size_t IdleBuffers::held() {
+    std::lock_guard<std::mutex> lk(mu);
+    return bytes;
+}
+
+// The live contexts, for dev_malloc.
+static std::mutex g_contexts_mu;
+static std::vector<Ctx *> g_contexts;
+
+hipError_t dev_malloc(void **p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipErrorOutOfMemory) return e;
+    int dev = -1;
+    (void)hipGetLastError();
+    (void)hipGetDevice(&dev);
+    {
+        std::lock_guard<std::mutex> lk(g_contexts_mu);
+        for (Ctx *c : g_contexts)
+            if (c->device == dev) c->idle.release();
+    }
+    return hipMalloc(p, bytes);
+}
+
+static Status alloc_state(Ctx &C, uint32_t n, int prec, State &out) {
+    out.ctx = &C; out.n = n; out.prec = prec;
+    out.d = C.idle.take(out.bytes());
+    if (out.d) return Status{};
+    hipError_t e = dev_malloc(&out.d, out.bytes());
+    if (e != hipSuccess) { out.d = nullptr; return oom_err(e); }
+    return Status{};
+}
+// The caller has waited for the context's stream.
+static void free_state(State &s) {
+    if (s.d) s.ctx->idle.put(s.d, s.bytes());
+    s.d = nullptr;
+}
+
 Status ensure(DevBuf &b, size_t bytes) {
     if (b.bytes >= bytes && b.p) return Status{};
     if (b.p) {
@@ -29,7 +97,7 @@ Status ensure(DevBuf &b, size_t bytes) {
         b.p = nullptr; b.bytes = 0;
     }
     size_t want = bytes < 4096 ? 4096 : bytes;
-    hipError_t e = hipMalloc(&b.p, want);
+    hipError_t e = dev_malloc(&b.p, want);
     if (e != hipSuccess) { b.p = nullptr; return oom_err(e); }
     b.bytes = want;
     return Status{};
@@ -184,16 +252,13 @@ static Status check_normalised(State &s) {
     return Status{};
 }
 
-static Status alloc_state(Ctx &C, uint32_t n, int prec, State &out) {
-    out.ctx = &C; out.n = n; out.prec = prec; out.d = nullptr;
-    hipError_t e = hipMalloc(&out.d, out.bytes());
-    if (e != hipSuccess) { out.d = nullptr; return oom_err(e); }
-    return Status{};
-}
-
 struct TmpState {
     State s;
-    ~TmpState() { if (s.d) (void)hipFree(s.d); }
+    ~TmpState() {
+        if (!s.d) return;
+        (void)hipStreamSynchronize(s.ctx->stream);
+        free_state(s);
+    }
 };
 
 static Status apply_1q_list(State &s, int kind, const uint64_t *q, uint32_t m, const double *mat) {
@@ -471,7 +536,7 @@ static Status apply_gates(State &s, uint32_t n_circuit, const qi_gate *gates, si
             allow_oop = true;
         } else if (swaps) {
             size_t fr = 0, tot = 0;
-            if (hipMemGetInfo(&fr, &tot) == hipSuccess && fr > s.bytes() + (size_t(16) << 30))
+            if (hipMemGetInfo(&fr, &tot) == hipSuccess && fr + C.idle.held() > s.bytes() + (size_t(16) << 30))
                 allow_oop = ensure(C.alt, s.bytes()).ok();
         }
     }
@@ -619,6 +684,10 @@ qi_status qi_ctx_create(int device, qi_ctx_t *out, qi_error *err) {
     }
     // an unseeded context draws from an OS-seeded stream, as rand::rng() does
     C.rng = (uint64_t(std::random_device{}()) << 32) ^ uint64_t(std::random_device{}());
+    {
+        std::lock_guard<std::mutex> lk(g_contexts_mu);
+        g_contexts.push_back(&C);
+    }
     *out = c.release();
     QI_RET(Status{});
 }
@@ -628,6 +697,11 @@ qi_status qi_ctx_destroy(qi_ctx_t ctx) {
     Ctx &C = ctx->c;
     (void)hipSetDevice(C.device);
     (void)hipStreamSynchronize(C.stream);
+    {
+        std::lock_guard<std::mutex> lk(g_contexts_mu);
+        g_contexts.erase(std::remove(g_contexts.begin(), g_contexts.end(), &C), g_contexts.end());
+    }
+    C.idle.release();
     if (C.graph_exec) (void)hipGraphExecDestroy(C.graph_exec);
     for (DevBuf *b : {&C.red, &C.red_out, &C.ops, &C.probs, &C.aux, &C.plan, &C.trot, &C.alt})
         if (b->p) (void)hipFree(b->p);
@@ -683,7 +757,7 @@ qi_status qi_state_destroy(qi_state_t s) {
     {
         QI_LOCK(s->s.ctx);
         (void)hipStreamSynchronize(s->s.ctx->stream);
-        if (s->s.d) (void)hipFree(s->s.d);
+        free_state(s->s);
     }
     delete s;
     return QI_OK;
@@ -696,8 +770,8 @@ qi_status qi_state_clone(qi_state_t src, qi_state_t *out, qi_error *err) {
     std::unique_ptr<qi_state_s> s(new qi_state_s());
     Status e = alloc_state(*src->s.ctx, src->s.n, src->s.prec, s->s);
     if (!e.ok()) QI_RET(e);
-    if (!(e = launch_copy(s->s, src->s, src->s.ctx->stream)).ok()) { (void)hipFree(s->s.d); QI_RET(e); }
-    if (!(e = device_check(src->s.ctx->stream)).ok()) { (void)hipFree(s->s.d); QI_RET(e); }
+    if (!(e = launch_copy(s->s, src->s, src->s.ctx->stream)).ok()) { (void)hipStreamSynchronize(src->s.ctx->stream); free_state(s->s); QI_RET(e); }
+    if (!(e = device_check(src->s.ctx->stream)).ok()) { free_state(s->s); QI_RET(e); }
     *out = s.release();
     QI_RET(Status{});
 }

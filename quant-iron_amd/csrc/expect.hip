@@ -32,6 +32,29 @@ __device__ __forceinline__ double flip_sign(double x, uint32_t odd) {
     return __longlong_as_double((long long)b);
 }
 
+// The index of tile t's first amplitude: t with a zero inserted at each of the
+// K tile qubits. (The positions sit in scalar registers: loaded from memory a
+// position per trip is a wait per trip.)
+struct TilePos {
+    uint64_t lo, hi;
+    __device__ __forceinline__ explicit TilePos(const uint32_t *pos)
+        : lo(pos[0] | uint64_t(pos[1]) << 32), hi(pos[2] | uint64_t(pos[3]) << 32) {}
+    __device__ __forceinline__ uint32_t operator()(int k) const { return uint32_t((k < 8 ? lo : hi) >> (8 * (k & 7))) & 255u; }
+};
+__device__ __forceinline__ uint64_t tile_base(uint64_t t, const TilePos &pos, int K) {
+    for (int k = 0; k < K; k++) {
+        const uint32_t b = pos(k);
+        t = ((t >> b) << (b + 1)) | (t & ((uint64_t(1) << b) - 1));
+    }
+    return t;
+}
+// The low `bits` of tid on the qubits of the tile-local bits from `first` on.
+__device__ __forceinline__ uint64_t thread_offset(uint32_t tid, const TilePos &pos, int bits, int first) {
+    uint64_t at = 0;
+    for (int i = 0; i < bits; i++) at |= uint64_t((tid >> i) & 1u) << pos(i + first);
+    return at;
+}
+
 // u = Re w (IM 0) or Im w (IM 1), w = conj(a) b, of the 8 pairs (s, s ^ M) of
 // the register bits, s with the highest bit of M clear, in ascending order of s.
 template <int M, int IM>
@@ -68,15 +91,11 @@ __global__ __launch_bounds__(512, CPLX ? 2 : 4) void k_expect_tiles(const T *__r
     // Loads: 16-byte units, thread t takes units t, t + nt, ...: the low K - 4
     // unit bits are the thread's, the rest the unit counter's (uniform).
     constexpr int UB = F32 ? 1 : 0, NU = kExpSlots >> UB, JB = 4 - UB;  // local bits in a unit, units per thread, counter bits
-    uint64_t at = 0;
-    for (int i = 0; i < K - 4; i++) at |= uint64_t((tid >> i) & 1u) << exp_pos(ps.pos, i + UB);
+    const TilePos pos4(ps.pos);
+    const uint64_t at = thread_offset(tid, pos4, K - 4, UB);
     DD acc[2] = {dd_zero(), dd_zero()};
     for (uint64_t t = blockIdx.x % per_pass; t < tiles; t += per_pass) {
-        uint64_t base = t;
-        for (int k = 0; k < K; k++) {
-            const uint32_t b = exp_pos(ps.pos, k);
-            base = ((base >> b) << (b + 1)) | (base & ((uint64_t(1) << b) - 1));
-        }
+        const uint64_t base = tile_base(t, pos4, K);
         if (act) {
             typedef float F4 __attribute__((ext_vector_type(4)));
             F4 u[NU];
@@ -85,7 +104,7 @@ __global__ __launch_bounds__(512, CPLX ? 2 : 4) void k_expect_tiles(const T *__r
                 uint64_t o = 0;
 #pragma unroll
                 for (int b = 0; b < JB; b++)
-                    if ((j >> b) & 1) o |= uint64_t(1) << exp_pos(ps.pos, K - JB + b);
+                    if ((j >> b) & 1) o |= uint64_t(1) << pos4(K - JB + b);
                 u[j] = __builtin_nontemporal_load(reinterpret_cast<const F4 *>(psi + (base | at | o)));
             }
             const uint32_t l0 = exp_slot<T>(tid << UB);
@@ -173,6 +192,7 @@ __global__ __launch_bounds__(512, CPLX ? 2 : 4) void k_expect_tiles(const T *__r
 #pragma unroll
                 for (int p = 0; p < kExpSlots; p++) {
                     double cr = 0.0, ci = 0.0;
+#pragma unroll 4  // (four terms' scalar loads in flight)
                     for (uint32_t d = st.doff[p]; d < st.doff[p + 1]; d++) {
                         const ExpDiag &t1 = diags[d];
                         const uint32_t odd = __popcll(base & t1.zo) + __popc(tl & t1.zl);
@@ -255,6 +275,183 @@ __global__ __launch_bounds__(256) void k_expect_group(const T *__restrict__ psi,
     if (threadIdx.x == 0) {
         part[size_t(blockIdx.x) * 4 + 0] = v[0].s; part[size_t(blockIdx.x) * 4 + 1] = v[0].c;
         part[size_t(blockIdx.x) * 4 + 2] = v[1].s; part[size_t(blockIdx.x) * 4 + 3] = v[1].c;
+    }
+}
+
+// ---------------------------------------------------------- SumOp::apply --
+// acc[s] += h[s] part(s) for the real (IM 0) or imaginary parts of a unit's
+// coefficients, signed, with fused multiply-adds; part: the partner of slot s.
+__device__ __forceinline__ float flip_sign(float x, uint32_t odd) {
+    return __uint_as_float(__float_as_uint(x) ^ (odd << 31));
+}
+
+template <bool IM, typename T, typename R, int NS>
+__device__ __forceinline__ void apply_part(T (&acc)[NS], const R *__restrict__ h, uint32_t odd, const T (&b)[NS]) {
+    R c[NS];
+#pragma unroll
+    for (int s = 0; s < NS; s++) c[s] = h[s];  // one run of scalar loads
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+        const R k = flip_sign(c[s], odd);
+        if (IM) {
+            acc[s].x = fma(-k, b[s].y, acc[s].x);
+            acc[s].y = fma(k, b[s].x, acc[s].y);
+        } else {
+            acc[s].x = fma(k, b[s].x, acc[s].x);
+            acc[s].y = fma(k, b[s].y, acc[s].y);
+        }
+    }
+}
+
+// One tile of one pass (expect_plan.h): the input tile goes to LDS, each thread
+// keeps the results of its loads' places in registers and takes a partner
+// per unit and slot from LDS, or from memory for remote masks. FIRST: the pass
+// starts the result, later passes add to it.
+// Bound by HBM (a pass moves two or three states: 146 us per later pass of a
+// 256 MiB state, 5.5 TB/s) and, where the diagonal terms run, by the latency of
+// their scalar loads. 24 qubits, complex128, a 4 x 6 lattice (138 terms, 38
+// masks): 0.65 ms in four passes, 1.86 ms as 138 gathers per amplitude.
+template <typename T, typename R, bool FIRST, bool CPLX>
+__global__ __launch_bounds__(512, 4) void k_apply_tiles(const T *__restrict__ psi, T *__restrict__ res, ApplyPass ps,
+                                                     const ApplyUnit<R> *__restrict__ units, const ExpDiag *__restrict__ diags, int K) {
+    constexpr bool F32 = sizeof(T) == 8;
+    constexpr int SB = apply_slot_bits(!F32), NS = 1 << SB, UB = F32 ? 1 : 0, NU = NS >> UB, JB = SB - UB, U = 1 << UB;
+    typedef float F4 __attribute__((ext_vector_type(4)));
+    extern __shared__ __attribute__((aligned(16))) unsigned char exp_lds[];
+    T *const tile = reinterpret_cast<T *>(exp_lds);
+    const uint32_t tid = threadIdx.x;
+    const TilePos pos4(ps.pos);
+    const uint64_t base = tile_base(blockIdx.x, pos4, K), at = base | thread_offset(tid, pos4, K - SB, UB);
+    // the slot bits' steps in memory and in LDS
+    uint64_t go[JB];
+    uint32_t so[SB];
+#pragma unroll
+    for (int b = 0; b < JB; b++) {
+        go[b] = uint64_t(1) << pos4(K - JB + b);
+        so[UB + b] = exp_slot<T>(1u << (K - JB + b));
+    }
+    if (F32) so[0] = exp_slot<T>(1u);
+    const uint32_t tl = tid << UB, ls = exp_slot<T>(tl);
+    T acc[NS];
+    {
+        F4 u[NU];
+#pragma unroll
+        for (int j = 0; j < NU; j++) {
+            uint64_t g = at;
+#pragma unroll
+            for (int b = 0; b < JB; b++)
+                if ((j >> b) & 1) g |= go[b];
+            u[j] = *reinterpret_cast<const F4 *>(psi + g);
+            if (!FIRST) {
+                const F4 r = __builtin_nontemporal_load(reinterpret_cast<const F4 *>(res + g));
+                if constexpr (F32) {
+                    acc[2 * j].x = r.x; acc[2 * j].y = r.y;
+                    acc[2 * j + 1].x = r.z; acc[2 * j + 1].y = r.w;
+                } else {
+                    acc[j] = __builtin_bit_cast(T, r);
+                }
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < NU; j++) {
+            uint32_t o = ls;
+#pragma unroll
+            for (int b = 0; b < JB; b++)
+                if ((j >> b) & 1) o ^= so[UB + b];
+            *reinterpret_cast<F4 *>(tile + o) = u[j];
+        }
+    }
+    if (FIRST)
+#pragma unroll
+        for (int s = 0; s < NS; s++) { acc[s].x = 0; acc[s].y = 0; }
+    __syncthreads();
+    for (uint32_t ui = ps.u0; ui < ps.u0 + ps.nu; ui++) {
+        const ApplyUnit<R> &un = units[ui];
+        const uint32_t flags = un.flags, odd = (__popcll(base & un.zo) + __popc(tl & un.zl)) & 1u;
+        T b[NS];
+        if (flags & kApplyRemote) {
+            const uint64_t x = un.x;
+#pragma unroll
+            for (int j = 0; j < NU; j++) {
+                uint64_t g = at;
+#pragma unroll
+                for (int k = 0; k < JB; k++)
+                    if ((j >> k) & 1) g |= go[k];
+                const F4 v = *reinterpret_cast<const F4 *>(psi + ((g ^ x) & ~uint64_t(U - 1)));
+                if constexpr (F32) {
+                    const bool odd_x = x & 1;
+                    b[2 * j].x = odd_x ? v.z : v.x; b[2 * j].y = odd_x ? v.w : v.y;
+                    b[2 * j + 1].x = odd_x ? v.x : v.z; b[2 * j + 1].y = odd_x ? v.y : v.w;
+                } else {
+                    b[j] = __builtin_bit_cast(T, v);
+                }
+            }
+        } else {
+            const uint32_t lx = ls ^ exp_slot<T>(un.xl);
+#pragma unroll
+            for (int s = 0; s < NS; s++) {
+                uint32_t o = lx;
+#pragma unroll
+                for (int k = 0; k < SB; k++)
+                    if ((s >> k) & 1) o ^= so[k];
+                b[s] = tile[o];
+            }
+        }
+        if (flags & kApplyRe) apply_part<false>(acc, un.re, odd, b);
+        if (flags & kApplyIm) apply_part<true>(acc, un.im, odd, b);
+    }
+    if (ps.diag) {
+        // the signed sums of the coefficients by slot-bit pattern, then their
+        // Walsh transform: the factor of each slot
+        double dr[NS], di[NS];
+#pragma unroll
+        for (int p = 0; p < NS; p++) {
+            double cr = 0.0, ci = 0.0;
+#pragma unroll 4  // (four terms' scalar loads in flight)
+            for (uint32_t d = ps.doff[p]; d < ps.doff[p + 1]; d++) {
+                const ExpDiag &t = diags[d];
+                const uint32_t odd = (__popcll(base & t.zo) + __popc(tl & t.zl)) & 1u;
+                cr += flip_sign(t.re, odd);
+                if (CPLX) ci += flip_sign(t.im, odd);
+            }
+            dr[p] = cr;
+            di[p] = ci;
+        }
+#pragma unroll
+        for (int b = 1; b < NS; b <<= 1)
+#pragma unroll
+            for (int s = 0; s < NS; s++)
+                if (!(s & b)) {
+                    const double x = dr[s], y = dr[s | b], z = di[s], w = di[s | b];
+                    dr[s] = x + y; dr[s | b] = x - y;
+                    if (CPLX) { di[s] = z + w; di[s | b] = z - w; }
+                }
+#pragma unroll
+        for (int s = 0; s < NS; s++) {
+            uint32_t o = ls;
+#pragma unroll
+            for (int b = 0; b < SB; b++)
+                if ((s >> b) & 1) o ^= so[b];
+            const T b = tile[o];
+            const R hr = R(dr[s]), hi = R(di[s]);
+            acc[s].x = fma(hr, b.x, acc[s].x);
+            acc[s].y = fma(hr, b.y, acc[s].y);
+            if (CPLX) {
+                acc[s].x = fma(-hi, b.y, acc[s].x);
+                acc[s].y = fma(hi, b.x, acc[s].y);
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < NU; j++) {
+        uint64_t g = at;
+#pragma unroll
+        for (int b = 0; b < JB; b++)
+            if ((j >> b) & 1) g |= go[b];
+        F4 r;
+        if constexpr (F32) r = F4{acc[2 * j].x, acc[2 * j].y, acc[2 * j + 1].x, acc[2 * j + 1].y};
+        else r = __builtin_bit_cast(F4, acc[j]);
+        __builtin_nontemporal_store(r, reinterpret_cast<F4 *>(res + g));
     }
 }
 
@@ -374,6 +571,39 @@ Status expect_run(State &s, const qi_pauli_term *terms, size_t nt, const ExpPlan
 }
 
 }  // namespace
+
+namespace {
+template <typename T, typename R>
+Status apply_tiles(const State &in, State &out, const qi_pauli_term *terms, size_t nt, hipStream_t st) {
+    Ctx &C = *in.ctx;
+    ApplyPlan<R> p;
+    plan_apply<R>(in.n, terms, nt, p);
+    const size_t diags = up16(p.units.size() * sizeof(ApplyUnit<R>)), bytes = diags + p.diags.size() * sizeof(ExpDiag);
+    Status s = ensure(C.ops, bytes);
+    if (s.ok()) s = ensure_stage(C, bytes);
+    if (!s.ok()) return s;
+    memcpy(C.stage, p.units.data(), p.units.size() * sizeof(ApplyUnit<R>));
+    memcpy(C.stage + diags, p.diags.data(), p.diags.size() * sizeof(ExpDiag));
+    if (bytes) QI_HIP_TRY(hipMemcpyAsync(C.ops.p, C.stage, bytes, hipMemcpyHostToDevice, st));
+    const uint64_t tiles = (uint64_t(1) << in.n) >> p.K;
+    const unsigned threads = 1u << (p.K - apply_slot_bits(sizeof(R) == 8));  // one slot set each: 512
+    for (size_t k = 0; k < p.passes.size(); k++) {
+        // (the diagonal terms run in the first pass)
+        auto *const kernel = k ? k_apply_tiles<T, R, false, false>
+                               : p.complex_diag ? k_apply_tiles<T, R, true, true> : k_apply_tiles<T, R, true, false>;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)tiles), dim3(threads), sizeof(T) << p.K, st, (const T *)in.d, (T *)out.d,
+                           p.passes[k], (const ApplyUnit<R> *)C.ops.p, (const ExpDiag *)((const unsigned char *)C.ops.p + diags), p.K);
+    }
+    QI_HIP_TRY(hipGetLastError());
+    QI_HIP_TRY(hipStreamSynchronize(st));  // the tables and the staging buffer are reused by the next call
+    return Status{};
+}
+}  // namespace
+
+Status sumop_apply_tiles(const State &in, State &out, const qi_pauli_term *terms, size_t nt, hipStream_t st) {
+    return in.prec == QI_C128 ? apply_tiles<double2, double>(in, out, terms, nt, st)
+                              : apply_tiles<float2, float>(in, out, terms, nt, st);
+}
 
 size_t expect_stage_bytes(size_t nt) { return exp_plan_bytes(nt) + nt * sizeof(TermK) + 256; }
 

@@ -3,6 +3,7 @@
 #include "expect_plan.h"
 
 #include <cstring>
+#include <unordered_map>
 
 namespace qi {
 
@@ -24,10 +25,25 @@ uint32_t reg_bits(uint32_t l, const ExpSet &s) {
     return r;
 }
 
-// Union growth: adds to `u` every mask of take[] that fits into `cap` bits,
-// the ones that need the fewest new bits first; above kGreedyMax masks simply
-// in list order (the search is quadratic).
+// The qubits of a tile of K: `q`, then the masks that need the fewest new ones
+// while they fit; above kGreedyMax masks simply in list order (the search is
+// quadratic).
 constexpr size_t kGreedyMax = 256;
+uint64_t grow_tile(uint64_t q, const uint64_t *xs, size_t count, int K) {
+    for (bool grown = true; grown;) {
+        grown = false;
+        size_t best = SIZE_MAX;
+        int least = 64;
+        for (size_t g = 0; g < count; g++) {
+            const int add = popc(xs[g] & ~q);
+            if (!add || popc(q) + add > K || add >= least) continue;
+            best = g; least = add;
+            if (count > kGreedyMax || add == 1) break;
+        }
+        if (best != SIZE_MAX) { q |= xs[best]; grown = true; }
+    }
+    return q;
+}
 
 }  // namespace
 
@@ -93,20 +109,7 @@ void plan_expect(uint32_t n, bool c128, const qi_pauli_term *terms, size_t nt, E
     while (at < nleft || diag_todo) {
         ExpPass &ps = p.passes[p.npasses++];
         memset(&ps, 0, sizeof ps);
-        // the tile: the low qubits, then masks that need the fewest new qubits
-        uint64_t q = lowmask;
-        for (bool grown = true; grown;) {
-            grown = false;
-            size_t best = SIZE_MAX;
-            int least = 64;
-            for (size_t g = at; g < nleft; g++) {
-                const int add = popc(p.xs[g] & ~q);
-                if (!add || popc(q) + add > K || add >= least) continue;
-                best = g; least = add;
-                if (nleft - at > kGreedyMax || add == 1) break;
-            }
-            if (best != SIZE_MAX) { q |= p.xs[best]; grown = true; }
-        }
+        uint64_t q = grow_tile(lowmask, p.xs + at, nleft - at, K);
         for (uint32_t b = 0; b < n && popc(q) < K; b++) q |= uint64_t(1) << b;
         ps.qmask = q;
         for (int k = 0, b = 0; k < K; b++)
@@ -216,5 +219,131 @@ void plan_expect(uint32_t n, bool c128, const qi_pauli_term *terms, size_t nt, E
     }
     memset(&p.units[p.nunits], 0, sizeof(ExpUnit));
 }
+
+// A pass reads and writes the result as well as the input, a remote mask reads
+// the input once more: passes of fewer masks than this are not worth it.
+constexpr size_t kApplyPassMasks = 3;
+
+template <typename R> void plan_apply(uint32_t n, const qi_pauli_term *terms, size_t nt, ApplyPlan<R> &p) {
+    const bool c128 = sizeof(R) == 8;
+    const int K = exp_tile_qubits(n, c128);
+    p.K = K;
+    const bool whole = (int)n == K;
+    const uint64_t lowmask = whole ? (uint64_t(1) << n) - 1 : (uint64_t(1) << exp_low_qubits(c128)) - 1;
+    std::vector<uint64_t> xs;
+    std::unordered_map<uint64_t, std::vector<uint32_t>> of;  // terms of each mask
+    bool diag = false;
+    for (size_t k = 0; k < nt; k++) {
+        if (!terms[k].x_mask) { diag = true; continue; }
+        std::vector<uint32_t> &v = of[terms[k].x_mask];
+        if (v.empty()) xs.push_back(terms[k].x_mask);
+        v.push_back((uint32_t)k);
+    }
+    const uint32_t slots = apply_slots(K, c128);
+    constexpr int SB = apply_slot_bits(sizeof(R) == 8), NS = 1 << SB;
+    uint32_t sm = 0;
+    for (int j = 0; j < SB; j++) sm |= 1u << exp_pos(&slots, j);
+    auto slot_bits = [&](uint32_t l) {
+        uint32_t r = 0;
+        for (int j = 0; j < SB; j++) r |= ((l >> exp_pos(&slots, j)) & 1u) << j;
+        return r;
+    };
+    std::vector<std::vector<uint64_t>> local;  // the masks of each pass; the rest (left) are remote
+    std::vector<uint64_t> tiles, left = xs;
+    for (;;) {
+        const uint64_t q0 = grow_tile(lowmask, left.data(), left.size(), K);
+        std::vector<uint64_t> in, out;
+        for (uint64_t x : left) ((x & ~q0) ? out : in).push_back(x);
+        if (!tiles.empty() && in.size() < kApplyPassMasks) break;
+        uint64_t q = q0;
+        for (uint32_t b = 0; b < n && popc(q) < K; b++) q |= uint64_t(1) << b;
+        tiles.push_back(q);
+        local.push_back(in);
+        left = out;
+        if (left.empty()) break;
+    }
+    for (size_t ip = 0; ip < tiles.size(); ip++) {
+        const uint64_t q = tiles[ip];
+        ExpPass ps{};  // positions for local_bits
+        ps.qmask = q;
+        for (int k = 0, b = 0; k < K; b++)
+            if ((q >> b) & 1) { ps.pos[k >> 2] |= (uint32_t)b << (8 * (k & 3)); k++; }
+        ApplyPass pass{};
+        pass.qmask = q;
+        memcpy(pass.pos, ps.pos, sizeof ps.pos);
+        pass.u0 = (uint32_t)p.units.size();
+        const bool last = ip + 1 == tiles.size();  // takes the remote masks
+        const size_t nlocal = local[ip].size(), total = nlocal + (last ? left.size() : 0);
+        for (size_t m = 0; m < total; m++) {
+            const bool remote = m >= nlocal;
+            const uint64_t x = remote ? left[m - nlocal] : local[ip][m];
+            const size_t e0 = p.units.size();
+            for (uint32_t t : of[x]) {
+                const qi_pauli_term &tm = terms[t];
+                const uint32_t zl = local_bits(tm.z_mask, ps, K);
+                const uint64_t zo = tm.z_mask & ~q;
+                size_t e = e0;
+                while (e < p.units.size() && !(p.units[e].zo == zo && p.units[e].zl == (zl & ~sm))) e++;
+                if (e == p.units.size()) {
+                    ApplyUnit<R> un{};
+                    un.zo = zo; un.x = x; un.zl = zl & ~sm;
+                    un.xl = remote ? 0 : local_bits(x, ps, K);
+                    un.flags = remote ? (uint32_t)kApplyRemote : 0u;
+                    p.units.push_back(un);
+                }
+            }
+            // the unit's coefficients, summed in FP64: c (-i)^ny (-1)^{popcount(slot & z)}
+            for (size_t e = e0; e < p.units.size(); e++) {
+                ApplyUnit<R> &un = p.units[e];
+                double hr[NS] = {0}, hi[NS] = {0};
+                for (uint32_t t : of[x]) {
+                    const qi_pauli_term &tm = terms[t];
+                    const uint32_t zl = local_bits(tm.z_mask, ps, K), zr = slot_bits(zl);
+                    if (un.zo != (tm.z_mask & ~q) || un.zl != (zl & ~sm)) continue;
+                    double cr = tm.c_re, ci = tm.c_im, r;
+                    switch (popc(tm.x_mask & tm.z_mask) & 3) {
+                    case 1: r = cr; cr = ci; ci = -r; break;   // times -i
+                    case 2: cr = -cr; ci = -ci; break;
+                    case 3: r = cr; cr = -ci; ci = r; break;   // times i
+                    default: break;
+                    }
+                    for (uint32_t s = 0; s < (uint32_t)NS; s++) {
+                        const bool odd = popc(s & zr) & 1;
+                        hr[s] += odd ? -cr : cr;
+                        hi[s] += odd ? -ci : ci;
+                    }
+                }
+                for (int s = 0; s < NS; s++) {
+                    un.re[s] = (R)hr[s];
+                    un.im[s] = (R)hi[s];
+                    if (hr[s] != 0.0) un.flags |= kApplyRe;
+                    if (hi[s] != 0.0) un.flags |= kApplyIm;
+                }
+                if (!(un.flags & (kApplyRe | kApplyIm))) un.flags |= kApplyRe;  // zero times NaN stays NaN
+            }
+        }
+        pass.nu = (uint32_t)p.units.size() - pass.u0;
+        if (ip == 0 && diag) {
+            pass.diag = 1;
+            uint32_t cnt[kExpSlots + 1] = {0};
+            for (size_t k = 0; k < nt; k++)
+                if (!terms[k].x_mask) cnt[slot_bits(local_bits(terms[k].z_mask, ps, K)) + 1]++;
+            for (int b = 0; b < kExpSlots; b++) cnt[b + 1] += cnt[b];
+            memcpy(pass.doff, cnt, sizeof cnt);
+            p.diags.resize(cnt[kExpSlots]);
+            for (size_t k = 0; k < nt; k++) {
+                if (terms[k].x_mask) continue;
+                const uint32_t zl = local_bits(terms[k].z_mask, ps, K);
+                ExpDiag &d = p.diags[cnt[slot_bits(zl)]++];
+                d.zo = terms[k].z_mask & ~q; d.zl = zl & ~sm; d.pad = 0;
+                d.re = terms[k].c_re; d.im = terms[k].c_im;
+                p.complex_diag = p.complex_diag || d.im != 0.0;
+            }
+        }
+        p.passes.push_back(pass);
+    }
+}
+template void plan_apply<float>(uint32_t, const qi_pauli_term *, size_t, ApplyPlan<float> &);
+template void plan_apply<double>(uint32_t, const qi_pauli_term *, size_t, ApplyPlan<double> &);
 
 }  // namespace qi

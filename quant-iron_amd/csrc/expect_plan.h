@@ -1,5 +1,6 @@
 // expect_plan.h — how the expectation of a SumOp is cut into tile passes
-// (planned on the host in expect_plan.cpp, run by expect.hip).
+// (planned on the host in expect_plan.cpp, run by expect.hip), and a SumOp's
+// product with a state on the same tiles.
 //
 // A tile is the 2^K amplitudes spanned by a set of K qubits. A term whose X
 // and Y factors lie inside that set needs only amplitudes of one tile, so one
@@ -13,6 +14,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <vector>
 
 #include "../../include/qiron.h"
 
@@ -93,5 +95,44 @@ int exp_tile_qubits(uint32_t n, bool c128);
 // Qubits 0 .. low-1 are always in a tile: 128-byte runs in memory.
 inline int exp_low_qubits(bool c128) { return c128 ? 3 : 4; }
 void plan_expect(uint32_t n, bool c128, const qi_pauli_term *terms, size_t nt, ExpPlan &p);
+
+// ---- SumOp::apply on the same tiles ----
+// A thread owns 16 (complex64) or 8 (complex128) amplitudes of the result
+// (slots: the tile-local bits of apply_slots) and adds, per unit, sign * h[slot] * in[i ^ x]: one unit per x
+// mask and Z support outside the slot bits. The partner comes from the tile in
+// LDS, or from memory for masks the pass's tile does not hold ("remote").
+constexpr int apply_slot_bits(bool c128) { return c128 ? 3 : 4; }
+template <typename R> struct ApplyUnit {
+    uint64_t zo;     // Z bits outside the tile
+    uint64_t x;      // the mask
+    uint32_t zl;     // Z bits inside the tile, outside the slot bits (tile-local)
+    uint32_t xl;     // the mask in tile-local bits (not remote)
+    uint32_t flags;  // kApplyRe | kApplyIm | kApplyRemote
+    uint32_t pad;
+    static constexpr int slots = 1 << apply_slot_bits(sizeof(R) == 8);
+    R re[slots], im[slots];
+};
+enum : uint32_t { kApplyRe = 1, kApplyIm = 2, kApplyRemote = 4 };
+struct ApplyPass {
+    uint64_t qmask;
+    uint32_t u0, nu;
+    uint32_t pos[4];     // as ExpPass
+    uint32_t diag;       // 1: the diagonal terms run here
+    uint32_t doff[kExpSlots + 1];
+};
+template <typename R> struct ApplyPlan {
+    int K = 0;
+    std::vector<ApplyPass> passes;
+    std::vector<ApplyUnit<R>> units;
+    std::vector<ExpDiag> diags;  // sorted by slot-bit pattern
+    bool complex_diag = false;   // a diagonal coefficient has an imaginary part
+};
+// Tile-local positions of the slot bits, ascending, a byte each: the bits a
+// thread's loads step over (complex64: bit 0 inside a 16-byte unit, then the top three).
+inline uint32_t apply_slots(int K, bool c128) {
+    const uint32_t k = (uint32_t)K;
+    return c128 ? (k - 3) | (k - 2) << 8 | (k - 1) << 16 : 0u | (k - 3) << 8 | (k - 2) << 16 | (k - 1) << 24;
+}
+template <typename R> void plan_apply(uint32_t n, const qi_pauli_term *terms, size_t nt, ApplyPlan<R> &p);
 
 }  // namespace qi

@@ -848,23 +848,23 @@ static Status mlp_alloc(Mlp &N, size_t rows) {
     for (void **p : ps)
         if (*p) { (void)hipFree(*p); *p = nullptr; }
     const size_t H = N.hid;
-    QI_HIP_TRY(hipMalloc(&N.X, rows * N.k_in * sizeof(bf16)));
+    QI_HIP_TRY(dev_malloc(&N.X, rows * N.k_in * sizeof(bf16)));
     for (int l = 0; l < 3; l++) {
-        QI_HIP_TRY(hipMalloc(&N.H[l], rows * H * sizeof(bf16)));
-        QI_HIP_TRY(hipMalloc(&N.dZb[l], rows * H * sizeof(bf16)));
-        QI_HIP_TRY(hipMalloc(&N.Z[l], rows * H * sizeof(float)));
-        QI_HIP_TRY(hipMalloc(&N.dZf[l], rows * H * sizeof(float)));
+        QI_HIP_TRY(dev_malloc(&N.H[l], rows * H * sizeof(bf16)));
+        QI_HIP_TRY(dev_malloc(&N.dZb[l], rows * H * sizeof(bf16)));
+        QI_HIP_TRY(dev_malloc(&N.Z[l], rows * H * sizeof(float)));
+        QI_HIP_TRY(dev_malloc(&N.dZf[l], rows * H * sizeof(float)));
     }
-    QI_HIP_TRY(hipMalloc(&N.y, rows * sizeof(float)));
-    QI_HIP_TRY(hipMalloc(&N.t, rows * sizeof(float)));
-    QI_HIP_TRY(hipMalloc(&N.dy, rows * sizeof(float)));
-    QI_HIP_TRY(hipMalloc(&N.part, ((rows + 255) / 256) * std::max<size_t>(H, N.k_in) * sizeof(float)));
-    QI_HIP_TRY(hipMalloc(&N.lossp, ((rows + 3) / 4) * sizeof(float)));
+    QI_HIP_TRY(dev_malloc(&N.y, rows * sizeof(float)));
+    QI_HIP_TRY(dev_malloc(&N.t, rows * sizeof(float)));
+    QI_HIP_TRY(dev_malloc(&N.dy, rows * sizeof(float)));
+    QI_HIP_TRY(dev_malloc(&N.part, ((rows + 255) / 256) * std::max<size_t>(H, N.k_in) * sizeof(float)));
+    QI_HIP_TRY(dev_malloc(&N.lossp, ((rows + 3) / 4) * sizeof(float)));
     const size_t wide = std::max<size_t>(H, N.k_in);
-    QI_HIP_TRY(hipMalloc(&N.T1, rows * wide * sizeof(bf16)));
-    QI_HIP_TRY(hipMalloc(&N.T2, rows * H * sizeof(bf16)));
-    QI_HIP_TRY(hipMalloc(&N.ws, size_t(kMaxSplits) * wide * H * sizeof(float)));
-    if (!N.lacc) QI_HIP_TRY(hipMalloc(&N.lacc, sizeof(double)));
+    QI_HIP_TRY(dev_malloc(&N.T1, rows * wide * sizeof(bf16)));
+    QI_HIP_TRY(dev_malloc(&N.T2, rows * H * sizeof(bf16)));
+    QI_HIP_TRY(dev_malloc(&N.ws, size_t(kMaxSplits) * wide * H * sizeof(float)));
+    if (!N.lacc) QI_HIP_TRY(dev_malloc(&N.lacc, sizeof(double)));
     N.cap = rows;
     return Status{};
 }
@@ -970,7 +970,7 @@ static Status alloc_packed(Mlp &N) {
     if (e.ok()) e = allow_lds<UniformCandidates>();
     if (e.ok()) e = allow_lds<LocalCandidates>();
     if (!e.ok()) return e;
-    const hipError_t he = hipMalloc(&N.wp, packed_words(N) * sizeof(bf16));
+    const hipError_t he = dev_malloc(&N.wp, packed_words(N) * sizeof(bf16));
     if (he != hipSuccess) { N.wp = nullptr; return oom_err(he); }
     return Status{};
 }
@@ -1117,8 +1117,8 @@ qi_status qi_mlp_create(qi_ctx_t ctx, uint32_t n_in, uint32_t hidden, uint64_t s
     std::lock_guard<std::mutex> lk(N.ctx->mu);
     hipStream_t st = N.ctx->stream;
     hipError_t e;
-    if ((e = hipMalloc(&N.w, N.nparam * 4)) || (e = hipMalloc(&N.m, N.nparam * 4)) || (e = hipMalloc(&N.v, N.nparam * 4)) ||
-        (e = hipMalloc(&N.g, N.nparam * 4)) || (e = hipMalloc(&N.wb, N.nparam * 2)) || (e = hipMalloc(&N.wt, N.nparam * 2)))
+    if ((e = dev_malloc(&N.w, N.nparam * 4)) || (e = dev_malloc(&N.m, N.nparam * 4)) || (e = dev_malloc(&N.v, N.nparam * 4)) ||
+        (e = dev_malloc(&N.g, N.nparam * 4)) || (e = dev_malloc(&N.wb, N.nparam * 2)) || (e = dev_malloc(&N.wt, N.nparam * 2)))
         QM_RET(oom_err(e));
     if ((e = hipMemcpy(N.w, w.data(), N.nparam * 4, hipMemcpyHostToDevice)) || (e = hipMemset(N.m, 0, N.nparam * 4)) ||
         (e = hipMemset(N.v, 0, N.nparam * 4)) || (e = hipMemset(N.g, 0, N.nparam * 4)))
@@ -1193,8 +1193,8 @@ qi_status qi_mlp_set_data(qi_mlp_t m, const float *x, const float *t, size_t row
     std::lock_guard<std::mutex> lk(N.ctx->mu);
     if (N.dataX) { (void)hipFree(N.dataX); (void)hipFree(N.dataT); (void)hipFree(N.perm); N.dataX = nullptr; }
     hipError_t e;
-    if ((e = hipMalloc(&N.dataX, rows * N.k_in * sizeof(bf16))) || (e = hipMalloc(&N.dataT, rows * 4)) ||
-        (e = hipMalloc(&N.perm, rows * 4)))
+    if ((e = dev_malloc(&N.dataX, rows * N.k_in * sizeof(bf16))) || (e = dev_malloc(&N.dataT, rows * 4)) ||
+        (e = dev_malloc(&N.perm, rows * 4)))
         QM_RET(oom_err(e));
     const size_t chunk = 65536;
     std::vector<bf16> hx(chunk * N.k_in);
@@ -1310,7 +1310,7 @@ qi_status qi_mlp_predict_ansatz(qi_mlp_t m, uint64_t seed, uint64_t draw0, uint6
         if (N.yall) (void)hipFree(N.yall);
         N.yall = nullptr;
         N.ycap = 0;
-        if ((e = hipMalloc(&N.yall, count * sizeof(float)))) QM_RET(oom_err(e));
+        if ((e = dev_malloc(&N.yall, count * sizeof(float)))) QM_RET(oom_err(e));
         N.ycap = count;
     }
     const UniformCandidates f{seed, draw0, count, (int)nang};
@@ -1354,14 +1354,14 @@ qi_status qi_mlp_predict_ansatz_local(qi_mlp_t m, uint64_t seed, uint64_t draw0,
         if (N.yall) (void)hipFree(N.yall);
         N.yall = nullptr;
         N.ycap = 0;
-        if ((e = hipMalloc(&N.yall, count * sizeof(float)))) QM_RET(oom_err(e));
+        if ((e = dev_malloc(&N.yall, count * sizeof(float)))) QM_RET(oom_err(e));
         N.ycap = count;
     }
     if (nang > N.th0cap) {
         if (N.theta0) (void)hipFree(N.theta0);
         N.theta0 = nullptr;
         N.th0cap = 0;
-        if ((e = hipMalloc(&N.theta0, nang * sizeof(double)))) QM_RET(oom_err(e));
+        if ((e = dev_malloc(&N.theta0, nang * sizeof(double)))) QM_RET(oom_err(e));
         N.th0cap = nang;
     }
     if ((e = hipMemcpyAsync(N.theta0, theta0, nang * sizeof(double), hipMemcpyHostToDevice, st)))

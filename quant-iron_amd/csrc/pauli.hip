@@ -92,7 +92,8 @@ __global__ __launch_bounds__(256) void k_pauli_exp(typename V2<R>::T *psi, uint6
     }
 }
 
-// out_i = sum_t (P_t in)_i * c_t, folded in term order (SumOp::apply).
+// out_i = sum_t (P_t in)_i * c_t, folded in term order (SumOp::apply of states
+// up to 20 qubits).
 template <typename R>
 __global__ __launch_bounds__(256) void k_sumop_apply(const typename V2<R>::T *__restrict__ in,
                                                      typename V2<R>::T *__restrict__ out, uint64_t dim,
@@ -191,6 +192,11 @@ Status launch_diag_tables(State &s, const DiagPass &p, const double2 *dtables, h
 }
 
 Status launch_sumop_apply(const State &in, State &out, const qi_pauli_term *terms, size_t nt, hipStream_t st) {
+    // Gathers of a state that the caches hold are cheaper than tile passes of few
+    // workgroups; the crossover lies between 20 and 21 qubits in both precisions
+    // (us, one chain or lattice of each size): 4 x 5 qubits 112 / 145 (complex64),
+    // 125 / 136 (complex128), 3 x 7: 198 / 156 and 224 / 162.
+    if (in.n > 20) return sumop_apply_tiles(in, out, terms, nt, st);
     Ctx &C = *in.ctx;
     std::vector<TermK> h(nt);
     for (size_t k = 0; k < nt; k++) h[k] = make_term(terms[k]);

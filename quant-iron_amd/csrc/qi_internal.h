@@ -51,10 +51,36 @@ struct DevBuf {
 // Scratch that grows on demand (reductions, histograms, schedules).
 Status ensure(DevBuf &b, size_t bytes);
 
+// hipMalloc that, when memory runs out, gives back the idle state buffers of
+// every context on the current device and tries once more. Every device
+// allocation of the library goes through it.
+hipError_t dev_malloc(void **p, size_t bytes);
+template <typename T> hipError_t dev_malloc(T **p, size_t bytes) { return dev_malloc(reinterpret_cast<void **>(p), bytes); }
+
+// Buffers of destroyed states, kept for the next state of the same size: the
+// reference's API returns a new state from every operation, and mapping and
+// unmapping 256 MiB costs more than a pass over it (a 24-qubit complex128
+// SumOp product takes 0.66 ms, with hipMalloc and hipFree around it 0.8 to
+// 5 ms). Bounded (kIdleBytes and kIdleBuffers per context, the oldest go
+// first), given back when an allocation fails and when the context ends. A
+// buffer is idle only after the context's stream has been waited for.
+constexpr size_t kIdleBytes = size_t(2) << 30;
+constexpr size_t kIdleBuffers = 32;
+struct IdleBuffers {
+    std::mutex mu;
+    std::vector<DevBuf> idle;  // oldest first
+    size_t bytes = 0;
+    void *take(size_t want);       // null: none of that size
+    void put(void *p, size_t bytes);
+    void release();
+    size_t held();
+};
+
 struct Ctx {
     int device = 0;
     hipStream_t stream = nullptr;
     std::mutex mu;
+    IdleBuffers idle;
     DevBuf red;      // reduction partials
     DevBuf red_out;  // reduction results (device)
     DevBuf ops;      // per-call op tables (tiles, Pauli terms)
@@ -154,6 +180,8 @@ Status launch_pauli_exp(State &s, const qi_pauli_term &t, double ch_re, double c
                         double sh_im, hipStream_t st);
 Status launch_sumop_apply(const State &in, State &out, const qi_pauli_term *terms, size_t nt,
                           hipStream_t st);
+// The same in tile passes (expect.hip), states of at least 13 qubits.
+Status sumop_apply_tiles(const State &in, State &out, const qi_pauli_term *terms, size_t nt, hipStream_t st);
 // A run of diagonal Pauli-string exponentials in one pass: per-amplitude
 // factors looked up in tables over at most kDiagTabBits qubits each.
 constexpr int kDiagTabBits = 10;
