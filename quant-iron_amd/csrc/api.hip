@@ -540,17 +540,22 @@ static Status apply_gates(State &s, uint32_t n_circuit, const qi_gate *gates, si
                 allow_oop = ensure(C.alt, s.bytes()).ok();
         }
     }
-    // plan key: options, gates, state shape and the buffer choice; the same gate
-    // list again reuses the last plan and its op tables in the plan buffer (no
-    // planning, no upload)
-    std::vector<unsigned char> key(sizeof(qi_exec_opts) + ng * sizeof(qi_gate) + 9);
-    memcpy(key.data(), &o, sizeof o);
-    if (ng) memcpy(key.data() + sizeof o, gates, ng * sizeof(qi_gate));
-    const uint64_t np = (uint64_t)s.n | ((uint64_t)s.prec << 32);
-    memcpy(key.data() + sizeof o + ng * sizeof(qi_gate), &np, 8);
-    key[sizeof o + ng * sizeof(qi_gate) + 8] = allow_oop ? 1 : 0;
+    // plan key: options, state shape and the buffer choice, then the gates; the
+    // same gate list again reuses the last plan and its op tables in the plan
+    // buffer (no planning, no upload). Compared in place: a copy is made for a
+    // new plan only.
+    struct PlanHead {
+        qi_exec_opts o;
+        uint32_t n, prec, oop;
+    } head;
+    memset(&head, 0, sizeof head);
+    head.o = o; head.n = s.n; head.prec = (uint32_t)s.prec; head.oop = allow_oop ? 1 : 0;
+    const size_t gate_bytes = ng * sizeof(qi_gate);
+    const bool same = C.cached_plan && C.plan_key.size() == sizeof head + gate_bytes &&
+                      memcmp(C.plan_key.data(), &head, sizeof head) == 0 &&
+                      (ng == 0 || memcmp(C.plan_key.data() + sizeof head, gates, gate_bytes) == 0);
     std::shared_ptr<ExecPlan> plan;
-    if (C.cached_plan && C.plan_key == key) {
+    if (same) {
         plan = std::static_pointer_cast<ExecPlan>(C.cached_plan);
     } else {
         plan = std::make_shared<ExecPlan>();
@@ -572,15 +577,17 @@ static Status apply_gates(State &s, uint32_t n_circuit, const qi_gate *gates, si
             QI_HIP_TRY(hipMemcpyAsync(C.plan.p, C.stage, plan->blob_bytes(), hipMemcpyHostToDevice, C.stream));
         }
         C.cached_plan = plan;
-        C.plan_key = key;
+        C.plan_key.resize(sizeof head + gate_bytes);
+        memcpy(C.plan_key.data(), &head, sizeof head);
+        if (ng) memcpy(C.plan_key.data() + sizeof head, gates, gate_bytes);
+        C.plan_serial++;
     }
     C.last_plan_steps = plan->steps.size();
-    // graph key: the plan key and the op-table and second-state buffers the graph reads
-    const uint64_t pp[2] = {(uint64_t)(uintptr_t)C.plan.p, (uint64_t)(uintptr_t)(allow_oop ? C.alt.p : nullptr)};
-    key.insert(key.end(), (const unsigned char *)pp, (const unsigned char *)pp + sizeof pp);
+    // graph key: the plan and the op-table and second-state buffers the graph reads
+    const uint64_t key[3] = {C.plan_serial, (uint64_t)(uintptr_t)C.plan.p, (uint64_t)(uintptr_t)(allow_oop ? C.alt.p : nullptr)};
     void *alt = allow_oop ? C.alt.p : nullptr;
     auto launch = [&]() -> Status { return launch_plan(s, *plan, gates, C.plan.p, alt); };
-    return run_maybe_graph(C, s, use_graph, key.data(), key.size(), launch);
+    return run_maybe_graph(C, s, use_graph, key, sizeof key, launch);
 }
 
 static Status check_pair(const State &a, const State &b) {

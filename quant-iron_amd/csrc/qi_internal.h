@@ -112,6 +112,7 @@ struct Ctx {
     // the last gate-list plan (an ExecPlan), whose op tables are in `plan`, and its key
     std::shared_ptr<void> cached_plan;
     std::vector<unsigned char> plan_key;
+    uint64_t plan_serial = 0;  // of cached_plan: a new number for every plan made
 };
 
 struct State {
