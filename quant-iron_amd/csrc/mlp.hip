@@ -365,9 +365,9 @@ __global__ __launch_bounds__(256) void k_head(const bf16 *__restrict__ H, const 
     }
 }
 
-// Column sums of X (rows x cols, FP32) into out[cols]: grid (ceil(cols/64), row chunks of 256).
-__global__ __launch_bounds__(256) void k_colsum_part(const float *__restrict__ X, int rows, int cols, float *__restrict__ part) {
-    __shared__ float sh[4][64];
+// Column sums of X (rows x cols, FP32) over 256-row chunks: workgroup (64
+// columns, chunk).
+__device__ __forceinline__ void colsum_chunk(const float *__restrict__ X, int rows, int cols, float *__restrict__ part, float (*sh)[64]) {
     const int c = blockIdx.x * 64 + (threadIdx.x & 63), g = threadIdx.x >> 6;
     const int r0 = blockIdx.y * 256;
     float s = 0.f;
@@ -379,6 +379,10 @@ __global__ __launch_bounds__(256) void k_colsum_part(const float *__restrict__ X
     sh[g][threadIdx.x & 63] = s;
     __syncthreads();
     if (g == 0 && c < cols) part[size_t(blockIdx.y) * cols + c] = sh[0][threadIdx.x] + sh[1][threadIdx.x] + sh[2][threadIdx.x] + sh[3][threadIdx.x];
+}
+__global__ __launch_bounds__(256) void k_colsum_part(const float *__restrict__ X, int rows, int cols, float *__restrict__ part) {
+    __shared__ float sh[4][64];
+    colsum_chunk(X, rows, cols, part, sh);
 }
 __global__ __launch_bounds__(256) void k_colsum_fold(const float *__restrict__ part, int chunks, int cols, float *__restrict__ out) {
     const int c = blockIdx.x * 256 + threadIdx.x;
@@ -400,9 +404,8 @@ __global__ __launch_bounds__(256) void k_head_fold(const float *__restrict__ par
 
 // Partial sums of dw[k] = sum_r H[r,k] dy[r] (head weights) over chunks of 256
 // rows, as k_colsum_part (folded by k_colsum_fold).
-__global__ __launch_bounds__(256) void k_head_grad_part(const bf16 *__restrict__ H, const float *__restrict__ dy, int rows,
-                                                        int hid, float *__restrict__ part) {
-    __shared__ float sh[4][64];
+__device__ __forceinline__ void head_grad_chunk(const bf16 *__restrict__ H, const float *__restrict__ dy, int rows, int hid,
+                                                float *__restrict__ part, float (*sh)[64]) {
     const int c = blockIdx.x * 64 + (threadIdx.x & 63), g = threadIdx.x >> 6;
     const int r0 = blockIdx.y * 256;
     float s = 0.f;
@@ -414,19 +417,31 @@ __global__ __launch_bounds__(256) void k_head_grad_part(const bf16 *__restrict__
     if (g == 0 && c < hid)
         part[size_t(blockIdx.y) * hid + c] = sh[0][threadIdx.x] + sh[1][threadIdx.x] + sh[2][threadIdx.x] + sh[3][threadIdx.x];
 }
+__global__ __launch_bounds__(256) void k_head_grad_part(const bf16 *__restrict__ H, const float *__restrict__ dy, int rows,
+                                                        int hid, float *__restrict__ part) {
+    __shared__ float sh[4][64];
+    head_grad_chunk(H, dy, rows, hid, part, sh);
+}
 
+// Adam on one FP32 master parameter; returns its new value.
+struct AdamStep {
+    float lr, b1, b2, eps, c1, c2;
+};
+__device__ __forceinline__ float adam_update(float *__restrict__ w, float *__restrict__ m, float *__restrict__ v, size_t i, float gi,
+                                             const AdamStep &a) {
+    const float mi = a.b1 * m[i] + (1.f - a.b1) * gi;
+    const float vi = a.b2 * v[i] + (1.f - a.b2) * gi * gi;
+    m[i] = mi;
+    v[i] = vi;
+    const float wi = w[i] - a.lr * (mi / a.c1) / (sqrtf(vi / a.c2) + a.eps);
+    w[i] = wi;
+    return wi;
+}
 // Adam on FP32 masters; refreshes the BF16 copy (nullable) of each parameter.
 __global__ __launch_bounds__(256) void k_adam(float *__restrict__ w, float *__restrict__ m, float *__restrict__ v,
-                                              const float *__restrict__ g, bf16 *__restrict__ wb, size_t n, float lr,
-                                              float b1, float b2, float eps, float c1, float c2) {
+                                              const float *__restrict__ g, bf16 *__restrict__ wb, size_t n, AdamStep a) {
     for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += size_t(gridDim.x) * blockDim.x) {
-        const float gi = g[i];
-        const float mi = b1 * m[i] + (1.f - b1) * gi;
-        const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-        m[i] = mi;
-        v[i] = vi;
-        const float wi = w[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-        w[i] = wi;
+        const float wi = adam_update(w, m, v, i, g[i], a);
         if (wb) wb[i] = f2bf(wi);
     }
 }
@@ -515,8 +530,7 @@ __global__ __launch_bounds__(256) void k_gather_rows(const bf16 *__restrict__ X,
 }  // namespace
 
 // acc += sum of the loss partials of one batch (one workgroup, fixed order)
-__global__ __launch_bounds__(256) void k_loss_accum(const float *__restrict__ part, int n, double *__restrict__ acc) {
-    __shared__ double sh[256];
+__device__ __forceinline__ void loss_accum(const float *__restrict__ part, int n, double *__restrict__ acc, double *sh) {
     double s = 0.0;
     for (int i = threadIdx.x; i < n; i += 256) s += part[i];
     sh[threadIdx.x] = s;
@@ -526,6 +540,272 @@ __global__ __launch_bounds__(256) void k_loss_accum(const float *__restrict__ pa
         __syncthreads();
     }
     if (threadIdx.x == 0) *acc += sh[0];
+}
+__global__ __launch_bounds__(256) void k_loss_accum(const float *__restrict__ part, int n, double *__restrict__ acc) {
+    __shared__ double sh[256];
+    loss_accum(part, n, acc, sh);
+}
+
+// ------------------------------------------------ small-batch training --
+// A training step on a batch whose layers have too few 128 x 128 tiles to fill
+// the chip is a chain of short dependent kernels (bounded by launches and load
+// round trips, not by bytes or operations), so it runs as nine launches (three
+// layers, head, two backward layers, the three weight gradients in one, all
+// column sums and the loss in one, Adam with every copy of the weights and the
+// next batch's rows in one) where the large-batch path takes 37. Each producer also writes the
+// transposed copy that a weight gradient reads. Every sum keeps the order of
+// the large-batch path's kernels (same K slices, slice order, row groups and
+// chunks): the same bits. Per step of 1024 rows at 195 -> 512 x 3 -> 1 the
+// large-batch kernels take 188 us, these 67.
+
+// C[M x N] = A[M x K] B[N x K]^T, both K-contiguous: one 32 x 32 tile per
+// workgroup, one wave per K slice of kper (blockDim / 64 slices), the slices
+// summed in order through LDS, then the epilogue. Fragments go from memory to
+// registers, four k steps (16 loads per lane) in flight.
+struct SmallGemm {
+    const bf16 *A, *B;
+    int lda, ldb, M, N, K, kper;
+    float *Cf;         // FP32 result (ldc = N)
+    bf16 *Cb, *Ct;     // BF16 result, and transposed (N x M)
+    const float *bias, *Zin;
+};
+struct SmallGemms {
+    SmallGemm g[3];
+};
+constexpr int kSlicesMax = kMaxSplits;
+template <int EPI> __global__ __launch_bounds__(64 * kSlicesMax) void k_small_gemm(SmallGemms gs) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char sg_lds[];
+    float(*const red)[32][36] = reinterpret_cast<float(*)[32][36]>(sg_lds);  // a slice's tile, padded rows
+    __shared__ __attribute__((aligned(16))) bf16 tr[32][40];
+    const SmallGemm &g = gs.g[blockIdx.z];
+    const int m0 = blockIdx.y * 32, n0 = blockIdx.x * 32;
+    if (m0 >= g.M || n0 >= g.N) return;  // whole workgroups (several problems in one grid)
+    const int lane = threadIdx.x & 63, slice = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kb = slice * g.kper, ke = min(g.K, kb + g.kper);
+    const int fr = lane & 15, fk = 8 * (lane >> 4);
+    floatx4 acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) acc[i][j] = floatx4{0, 0, 0, 0};
+    auto frag = [&](const bf16 *P, int ld, int rows, int r, int k) {
+        uint4 v = make_uint4(0, 0, 0, 0);
+        if (r < rows && k < ke) v = *reinterpret_cast<const uint4 *>(P + size_t(r) * ld + k);
+        return __builtin_bit_cast(bf16x8, v);
+    };
+    for (int k0 = kb; k0 < ke; k0 += 128) {
+        bf16x8 a[4][2], b[4][2];
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                a[s][i] = frag(g.A, g.lda, g.M, m0 + 16 * i + fr, k0 + 32 * s + fk);
+                b[s][i] = frag(g.B, g.ldb, g.N, n0 + 16 * i + fr, k0 + 32 * s + fk);
+            }
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[s][j], a[s][i], acc[i][j], 0, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+            *reinterpret_cast<floatx4 *>(&red[slice][16 * i + fr][16 * j + 4 * (lane >> 4)]) = acc[i][j];
+    __syncthreads();
+    const int slices = blockDim.x >> 6;
+    for (int it = threadIdx.x; it < 256; it += blockDim.x) {
+        const int row = it >> 3, col = 4 * (it & 7);
+        float4 x = *reinterpret_cast<const float4 *>(&red[0][row][col]);
+        for (int z = 1; z < slices; z++) {
+            const float4 q = *reinterpret_cast<const float4 *>(&red[z][row][col]);
+            x.x += q.x; x.y += q.y; x.z += q.z; x.w += q.w;
+        }
+        const bool in = m0 + row < g.M;
+        const size_t o = size_t(m0 + row) * g.N + n0 + col;
+        float v[4] = {x.x, x.y, x.z, x.w};
+        if (EPI == EPI_STORE) {
+            if (in) *reinterpret_cast<float4 *>(g.Cf + o) = x;
+            continue;
+        }
+        if (EPI == EPI_GELU) {
+            const float4 bb = *reinterpret_cast<const float4 *>(g.bias + n0 + col);
+            v[0] += bb.x; v[1] += bb.y; v[2] += bb.z; v[3] += bb.w;
+            if (in) *reinterpret_cast<float4 *>(g.Cf + o) = make_float4(v[0], v[1], v[2], v[3]);
+#pragma unroll
+            for (int r = 0; r < 4; r++) v[r] = gelu_fwd(v[r]);
+        } else {
+            const float4 z = in ? *reinterpret_cast<const float4 *>(g.Zin + o) : make_float4(0.f, 0.f, 0.f, 0.f);
+            v[0] *= gelu_grad(z.x); v[1] *= gelu_grad(z.y); v[2] *= gelu_grad(z.z); v[3] *= gelu_grad(z.w);
+            if (in) *reinterpret_cast<float4 *>(g.Cf + o) = make_float4(v[0], v[1], v[2], v[3]);
+        }
+        const uint2 h = pack_bf16x4(v);
+        if (in) *reinterpret_cast<uint2 *>(g.Cb + o) = h;
+        tr[col][row] = (bf16)h.x; tr[col + 1][row] = (bf16)(h.x >> 16);
+        tr[col + 2][row] = (bf16)h.y; tr[col + 3][row] = (bf16)(h.y >> 16);
+    }
+    if (EPI == EPI_STORE || !g.Ct) return;
+    __syncthreads();
+    for (int it = threadIdx.x; it < 128; it += blockDim.x) {  // 8 rows of a column (M % 16 == 0)
+        const int col = it >> 2, row = 8 * (it & 3);
+        if (m0 + row < g.M)
+            *reinterpret_cast<uint4 *>(g.Ct + size_t(n0 + col) * g.M + m0 + row) = *reinterpret_cast<const uint4 *>(&tr[col][row]);
+    }
+}
+
+// k_head for eight rows per workgroup (a wave each), with the transposed dZ.
+__global__ __launch_bounds__(512) void k_head_rows8(const bf16 *__restrict__ H, const float *__restrict__ w, const float *__restrict__ bp,
+                                                    int rows, int hid, float *__restrict__ y, const float *__restrict__ t, float inv_b,
+                                                    const float *__restrict__ Z, float *__restrict__ dZf, bf16 *__restrict__ dZb,
+                                                    bf16 *__restrict__ dZt, float *__restrict__ dy, float *__restrict__ loss_part) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char hr_lds[];
+    bf16 *const tr = reinterpret_cast<bf16 *>(hr_lds);  // hid x 8
+    __shared__ float lsum[8];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int r = blockIdx.x * 8 + wave;  // rows % 16 == 0
+    float s = 0.f;
+#pragma unroll 8
+    for (int k = lane; k < hid; k += 64) s += bf2f(H[size_t(r) * hid + k]) * w[k];
+    for (int m = 32; m >= 1; m >>= 1) s += __shfl_xor(s, m);
+    s += *bp;
+    const float d = 2.f * (s - t[r]) * inv_b;
+    if (lane == 0) {
+        y[r] = s;
+        dy[r] = d;
+        lsum[wave] = (s - t[r]) * (s - t[r]);
+    }
+#pragma unroll 8
+    for (int k = lane; k < hid; k += 64) {
+        const size_t o = size_t(r) * hid + k;
+        const float g = d * w[k] * gelu_grad(Z[o]);
+        const bf16 b = f2bf(g);
+        dZf[o] = g;
+        dZb[o] = b;
+        tr[k * 8 + wave] = b;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2)
+        loss_part[2 * blockIdx.x + threadIdx.x] =
+            lsum[4 * threadIdx.x] + lsum[4 * threadIdx.x + 1] + lsum[4 * threadIdx.x + 2] + lsum[4 * threadIdx.x + 3];
+    for (int k = threadIdx.x; k < hid; k += 512)
+        *reinterpret_cast<uint4 *>(dZt + size_t(k) * rows + 8 * blockIdx.x) = *reinterpret_cast<const uint4 *>(tr + k * 8);
+}
+
+// k_gather_rows for eight rows per workgroup, with the transposed block.
+struct GatherRows {
+    const bf16 *X;
+    const uint32_t *idx;
+    const float *t;
+    bf16 *out, *outt;
+    float *tout;
+    int rows, cols;
+};
+__device__ __forceinline__ void gather_rows8(const GatherRows &g, int block, bf16 *tr) {
+    const int r0 = block * 8, words = g.cols / 8;  // cols % 16 == 0, rows % 16 == 0; tr: cols x 8
+    for (int i = threadIdx.x; i < 8 * words; i += 256) {
+        const int r = i / words, c = i - r * words;
+        const uint4 v = *reinterpret_cast<const uint4 *>(g.X + size_t(g.idx[r0 + r]) * g.cols + 8 * c);
+        *reinterpret_cast<uint4 *>(g.out + size_t(r0 + r) * g.cols + 8 * c) = v;
+        const uint32_t q[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int k = 0; k < 8; k++) tr[(8 * c + k) * 8 + r] = (bf16)(q[k >> 1] >> (16 * (k & 1)));
+    }
+    if (threadIdx.x < 8) g.tout[r0 + threadIdx.x] = g.t[g.idx[r0 + threadIdx.x]];
+    __syncthreads();
+    for (int c = threadIdx.x; c < g.cols; c += 256)
+        *reinterpret_cast<uint4 *>(g.outt + size_t(c) * g.rows + r0) = *reinterpret_cast<const uint4 *>(tr + c * 8);
+}
+__global__ __launch_bounds__(256) void k_gather_rows8(GatherRows g) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char gr_lds[];
+    gather_rows8(g, blockIdx.x, reinterpret_cast<bf16 *>(gr_lds));
+}
+
+// Chunk sums of the bias gradients (dZ of the three layers), the head's weight
+// and bias gradients, and the batch's loss: workgroup (64 columns, chunk, which).
+struct StepSums {
+    const float *dZ[3], *dy, *lossp;
+    const bf16 *H;
+    float *part[5];  // b1, b2, b3, w4, b4: chunks x width
+    double *lacc;    // null: no loss
+    int rows, hid, nloss;
+};
+__global__ __launch_bounds__(256) void k_step_sums(StepSums s) {
+    __shared__ float sh[4][64];
+    __shared__ double shd[256];
+    const int w = blockIdx.z;
+    if (w < 3) colsum_chunk(s.dZ[w], s.rows, s.hid, s.part[w], sh);
+    else if (w == 3) head_grad_chunk(s.H, s.dy, s.rows, s.hid, s.part[3], sh);
+    else if (blockIdx.x == 0) colsum_chunk(s.dy, s.rows, 1, s.part[4], sh);
+    else if (blockIdx.x == 1 && blockIdx.y == 0 && s.lacc) loss_accum(s.lossp, s.nloss, s.lacc, shd);
+}
+
+// The gradients folded from those chunks in order.
+__device__ __forceinline__ float fold_chunks(const float *__restrict__ part, int chunks, int cols, int c) {
+    float s = 0.f;
+    for (int k = 0; k < chunks; k++) s += part[size_t(k) * cols + c];
+    return s;
+}
+struct VecParams {
+    const float *part[5];
+    size_t off[5];
+    int width[5], chunks;
+};
+__global__ __launch_bounds__(256) void k_fold_vectors(VecParams p, float *__restrict__ g) {
+    const int w = blockIdx.y, c = blockIdx.x * 256 + threadIdx.x;
+    if (c < p.width[w]) g[p.off[w] + c] = fold_chunks(p.part[w], p.chunks, p.width[w], c);
+}
+
+// Adam on all parameters: 32 x 32 tiles of the three matrices (FP32 master,
+// BF16 copy and its transpose through LDS), then 256 entries per workgroup of
+// the vectors, whose gradients are folded here, and the next batch's rows
+// (the step's last launch: nothing reads this batch's any more).
+struct AdamAll {
+    float *w, *m, *v;
+    const float *g;
+    bf16 *wb, *wt;
+    size_t off[3];
+    int rows[3], hid, tiles[3];  // tiles of each matrix
+    VecParams vec;
+    int vblocks[5];
+    GatherRows next;
+};
+__global__ __launch_bounds__(256) void k_adam_all(AdamAll p, AdamStep a) {
+    int b = blockIdx.x;
+#pragma unroll
+    for (int l = 0; l < 3; l++) {
+        if (b < p.tiles[l]) {
+            __shared__ bf16 t[32][34];
+            const int tc = p.hid / 32, c0 = (b % tc) * 32, r0 = (b / tc) * 32, tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+            for (int k = ty; k < 32; k += 8) {
+                if (r0 + k >= p.rows[l]) continue;
+                const size_t i = p.off[l] + size_t(r0 + k) * p.hid + c0 + tx;
+                const bf16 h = f2bf(adam_update(p.w, p.m, p.v, i, p.g[i], a));
+                p.wb[i] = h;
+                t[k][tx] = h;
+            }
+            __syncthreads();
+            for (int k = ty; k < 32; k += 8)
+                if (r0 + tx < p.rows[l]) p.wt[p.off[l] + size_t(c0 + k) * p.rows[l] + r0 + tx] = t[tx][k];
+            return;
+        }
+        b -= p.tiles[l];
+    }
+    for (int w = 0; w < 5; w++) {
+        if (b < p.vblocks[w]) {
+            const int c = b * 256 + threadIdx.x;
+            if (c < p.vec.width[w]) {
+                const size_t i = p.vec.off[w] + c;
+                p.wb[i] = f2bf(adam_update(p.w, p.m, p.v, i, fold_chunks(p.vec.part[w], p.vec.chunks, p.vec.width[w], c), a));
+            }
+            return;
+        }
+        b -= p.vblocks[w];
+    }
+    extern __shared__ __attribute__((aligned(16))) unsigned char ad_lds[];
+    gather_rows8(p.next, b, reinterpret_cast<bf16 *>(ad_lds));
 }
 
 // SplitMix64 draw k (1-based) of the stream seeded with `seed` (Steele, Lea &
@@ -821,6 +1101,10 @@ struct Mlp {
     float *ws = nullptr;                                           // split-K partials
     size_t ws_floats() const { return ws ? size_t(kMaxSplits) * size_t(std::max(hid, k_in)) * size_t(hid) : 0; }
     double *lacc = nullptr;                                        // epoch loss accumulator
+    // small-batch steps: transposed inputs, activations and gradients, chunk sums
+    bf16 *XT = nullptr, *HT[2] = {nullptr, nullptr}, *dZT[3] = {nullptr, nullptr, nullptr};
+    float *vpart = nullptr;
+    size_t tcap = 0;
     float *yall = nullptr;                                         // predictions of a candidate screen
     size_t ycap = 0;
     double *theta0 = nullptr;                                      // centre of a local candidate round
@@ -831,7 +1115,7 @@ struct Mlp {
     uint32_t *perm = nullptr;
     size_t ndata = 0;
     ~Mlp() {
-        void *ps[] = {w, m, v, g, wb, wt, wp, X, H[0], H[1], H[2], dZb[0], dZb[1], dZb[2], Z[0], Z[1], Z[2], dZf[0], dZf[1], dZf[2],
+        void *ps[] = {XT, HT[0], HT[1], dZT[0], dZT[1], dZT[2], vpart, w, m, v, g, wb, wt, wp, X, H[0], H[1], H[2], dZb[0], dZb[1], dZb[2], Z[0], Z[1], Z[2], dZf[0], dZf[1], dZf[2],
                       y, t, dy, part, lossp, T1, T2, ws, dataX, dataT, perm, lacc, yall, theta0};
         for (void *p : ps)
             if (p) (void)hipFree(p);
@@ -1054,6 +1338,156 @@ static void backward(Mlp &N, hipStream_t st, int rows) {
     colsum(N, st, N.dZf[0], rows, H, N.g + N.off[1]);
 }
 
+// ------------------------------------------------ small-batch training --
+// K slices that the large-batch path gives a layer GEMM of M x N x K (gemm)
+// and a weight gradient (gemm_at_b): the small-batch kernels take the same, so
+// that both sum in the same order.
+static int layer_slices(int M, int Nn, int K, size_t ws_floats, int &kper) {
+    const int tiles = ((M + TM - 1) / TM) * ((Nn + TN - 1) / TN);
+    int splits = std::min({kMaxSplits, 256 / std::max(tiles, 1), K / (2 * TK), int(ws_floats / (size_t(M) * Nn))});
+    kper = K;
+    if (splits < 2) return 1;
+    kper = ((K + splits - 1) / splits + 2 * TK - 1) / (2 * TK) * (2 * TK);
+    return (K + kper - 1) / kper;
+}
+static int gradient_slices(int M, int Nn, int K, int &kper) {
+    const int tiles = ((M + TM - 1) / TM) * ((Nn + TN - 1) / TN);
+    const int splits = std::max(1, std::min({kMaxSplits, 256 / std::max(tiles, 1), K / (2 * TK)}));
+    kper = ((K + splits - 1) / splits + 2 * TK - 1) / (2 * TK) * (2 * TK);
+    return (K + kper - 1) / kper;
+}
+// Batches whose layers have fewer than kSplitBelowTiles 128 x 128 tiles (at
+// that line the large-batch path stops splitting K), up to widths where the
+// two meet: us per step, large-batch kernels -> these, at 195 inputs: width 512
+// batch 128 137 -> 46, 3072 226 -> 130; width 1024 batch 1024 233 -> 158; width
+// 2048 batch 256 248 -> 198; 4000 inputs, width and batch 1024 291 -> 288.
+static bool small_step(const Mlp &N, size_t rows) {
+    const size_t tiles = ((rows + TM - 1) / TM) * size_t((N.hid + TN - 1) / TN);
+    return tiles < (size_t)kSplitBelowTiles && N.hid <= 2048 && N.k_in <= 2048;
+}
+static Status small_alloc(Mlp &N, size_t rows) {
+    if (rows <= N.tcap) return Status{};
+    void **ps[] = {(void **)&N.XT, (void **)&N.HT[0], (void **)&N.HT[1], (void **)&N.dZT[0], (void **)&N.dZT[1], (void **)&N.dZT[2],
+                   (void **)&N.vpart};
+    QI_HIP_TRY(hipDeviceSynchronize());
+    N.tcap = 0;
+    for (void **p : ps)
+        if (*p) { (void)hipFree(*p); *p = nullptr; }
+    const size_t H = N.hid;
+    QI_HIP_TRY(dev_malloc(&N.XT, rows * N.k_in * sizeof(bf16)));
+    for (int l = 0; l < 2; l++) QI_HIP_TRY(dev_malloc(&N.HT[l], rows * H * sizeof(bf16)));
+    for (int l = 0; l < 3; l++) QI_HIP_TRY(dev_malloc(&N.dZT[l], rows * H * sizeof(bf16)));
+    QI_HIP_TRY(dev_malloc(&N.vpart, (rows + 255) / 256 * (4 * H + 1) * sizeof(float)));
+    const int lds = kSlicesMax * 32 * 36 * (int)sizeof(float);
+    QI_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(k_small_gemm<EPI_GELU>), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    QI_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(k_small_gemm<EPI_STORE>), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    QI_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(k_small_gemm<EPI_GELU_BWD>), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    N.tcap = rows;
+    return Status{};
+}
+template <int EPI> static void small_gemm(hipStream_t st, const SmallGemms &gs, int count, int slices) {
+    int mx = 0, nx = 0;
+    for (int k = 0; k < count; k++) { mx = std::max(mx, gs.g[k].M); nx = std::max(nx, gs.g[k].N); }
+    hipLaunchKernelGGL(k_small_gemm<EPI>, dim3((unsigned)(nx / 32), (unsigned)((mx + 31) / 32), (unsigned)count), dim3(64 * slices),
+                       size_t(slices) * 32 * 36 * sizeof(float), st, gs);
+}
+static void small_forward(Mlp &N, hipStream_t st, int rows) {
+    const bf16 *in[3] = {N.X, N.H[0], N.H[1]};
+    for (int l = 0; l < 3; l++) {
+        const int K = l ? N.hid : N.k_in;
+        SmallGemms gs{};
+        SmallGemm &g = gs.g[0];
+        g.A = in[l]; g.lda = K; g.B = N.wt + N.off[2 * l]; g.ldb = K;
+        g.M = rows; g.N = N.hid; g.K = K;
+        const int slices = layer_slices(rows, N.hid, K, N.ws_floats(), g.kper);
+        g.Cf = N.Z[l]; g.Cb = N.H[l]; g.Ct = l < 2 ? N.HT[l] : nullptr; g.bias = N.w + N.off[2 * l + 1];
+        small_gemm<EPI_GELU>(st, gs, 1, slices);
+    }
+}
+static VecParams vec_params(const Mlp &N, int rows) {
+    VecParams p{};
+    p.chunks = (rows + 255) / 256;
+    const int which[5] = {1, 3, 5, 6, 7};  // b1, b2, b3, w4, b4
+    for (int k = 0; k < 5; k++) {
+        p.part[k] = N.vpart + size_t(k) * p.chunks * N.hid;
+        p.off[k] = N.off[which[k]];
+        p.width[k] = k < 4 ? N.hid : 1;
+    }
+    return p;
+}
+// Gradients: the matrices' into N.g, the vectors' as chunk sums in N.vpart;
+// lacc (may be null) gains the batch's loss.
+static void small_backward(Mlp &N, hipStream_t st, int rows, double *lacc) {
+    const int H = N.hid;
+    hipLaunchKernelGGL(k_head_rows8, dim3(rows / 8), dim3(512), size_t(H) * 8 * sizeof(bf16), st, (const bf16 *)N.H[2],
+                       (const float *)(N.w + N.off[6]), (const float *)(N.w + N.off[7]), rows, H, N.y, (const float *)N.t, 1.0f / rows,
+                       (const float *)N.Z[2], N.dZf[2], N.dZb[2], N.dZT[2], N.dy, N.lossp);
+    for (int l = 1; l >= 0; l--) {  // dZ_l = (dZ_{l+1} W_{l+1}^T) * gelu'(Z_l)
+        SmallGemms gs{};
+        SmallGemm &g = gs.g[0];
+        g.A = N.dZb[l + 1]; g.lda = H; g.B = N.wb + N.off[2 * (l + 1)]; g.ldb = H;
+        g.M = rows; g.N = H; g.K = H;
+        const int slices = layer_slices(rows, H, H, N.ws_floats(), g.kper);
+        g.Cf = N.dZf[l]; g.Cb = N.dZb[l]; g.Ct = N.dZT[l]; g.Zin = N.Z[l];
+        small_gemm<EPI_GELU_BWD>(st, gs, 1, slices);
+    }
+    // the weight gradients X^T dZ1, H1^T dZ2, H2^T dZ3: one launch where their slice counts agree
+    SmallGemms gs{};
+    int slices[3];
+    const bf16 *left[3] = {N.XT, N.HT[0], N.HT[1]};
+    for (int l = 0; l < 3; l++) {
+        SmallGemm &g = gs.g[l];
+        g.A = left[l]; g.lda = rows; g.B = N.dZT[l]; g.ldb = rows;
+        g.M = l ? H : N.k_in; g.N = H; g.K = rows;
+        slices[l] = gradient_slices(g.M, H, rows, g.kper);
+        g.Cf = N.g + N.off[2 * l];
+    }
+    if (slices[0] == slices[1] && slices[1] == slices[2]) {
+        small_gemm<EPI_STORE>(st, gs, 3, slices[0]);
+    } else {
+        for (int l = 0; l < 3; l++) {
+            SmallGemms one{};
+            one.g[0] = gs.g[l];
+            small_gemm<EPI_STORE>(st, one, 1, slices[l]);
+        }
+    }
+    const VecParams v = vec_params(N, rows);
+    StepSums s{};
+    for (int l = 0; l < 3; l++) s.dZ[l] = N.dZf[l];
+    s.dy = N.dy; s.lossp = N.lossp; s.H = N.H[2]; s.lacc = lacc;
+    for (int k = 0; k < 5; k++) s.part[k] = const_cast<float *>(v.part[k]);
+    s.rows = rows; s.hid = H; s.nloss = (rows + 3) / 4;
+    // (x: 64-column blocks; the last z takes two single workgroups)
+    hipLaunchKernelGGL(k_step_sums, dim3((unsigned)std::max(2, (H + 63) / 64), (unsigned)v.chunks, 5), dim3(256), 0, st, s);
+}
+static GatherRows gather_of(const Mlp &N, const uint32_t *idx, int rows) {
+    return GatherRows{N.dataX, idx, N.dataT, N.X, N.XT, N.t, rows, N.k_in};
+}
+// next: the index list of the next batch (null: none).
+static void small_adam(Mlp &N, hipStream_t st, int rows, const AdamStep &ad, const uint32_t *next) {
+    AdamAll p{};
+    p.w = N.w; p.m = N.m; p.v = N.v; p.g = N.g; p.wb = N.wb; p.wt = N.wt; p.hid = N.hid;
+    int blocks = 0;
+    for (int l = 0; l < 3; l++) {
+        p.off[l] = N.off[2 * l];
+        p.rows[l] = l ? N.hid : N.k_in;
+        p.tiles[l] = (N.hid / 32) * ((p.rows[l] + 31) / 32);
+        blocks += p.tiles[l];
+    }
+    p.vec = vec_params(N, rows);
+    for (int k = 0; k < 5; k++) {
+        p.vblocks[k] = (p.vec.width[k] + 255) / 256;
+        blocks += p.vblocks[k];
+    }
+    size_t lds = 0;
+    if (next) {
+        p.next = gather_of(N, next, rows);
+        blocks += rows / 8;
+        lds = size_t(N.k_in) * 8 * sizeof(bf16);
+    }
+    hipLaunchKernelGGL(k_adam_all, dim3((unsigned)blocks), dim3(256), lds, st, p, ad);
+}
+
 static Status stage_rows(Mlp &N, hipStream_t st, const float *x, const float *t, size_t rows) {
     // host FP32 rows (n_in wide) -> device BF16 rows (k_in wide, zero padded)
     std::vector<bf16> hx(rows * N.k_in, 0);
@@ -1175,8 +1609,17 @@ qi_status qi_mlp_gradients(qi_mlp_t m, const float *x, const float *t, size_t ro
     hipStream_t st = N.ctx->stream;
     QM_TRY(mlp_alloc(N, rows));
     QM_TRY(stage_rows(N, st, x, t, rows));
-    forward(N, st, (int)rows, true);
-    backward(N, st, (int)rows);
+    if (small_step(N, rows)) {
+        QM_TRY(small_alloc(N, rows));
+        hipLaunchKernelGGL(k_transpose_b16, dim3((N.k_in + 31) / 32, (unsigned)((rows + 31) / 32)), dim3(256), 0, st, (const bf16 *)N.X,
+                           (int)rows, N.k_in, N.XT);
+        small_forward(N, st, (int)rows);
+        small_backward(N, st, (int)rows, nullptr);
+        hipLaunchKernelGGL(k_fold_vectors, dim3((unsigned)((N.hid + 255) / 256), 5), dim3(256), 0, st, vec_params(N, (int)rows), N.g);
+    } else {
+        forward(N, st, (int)rows, true);
+        backward(N, st, (int)rows);
+    }
     std::vector<float> lp((rows + 3) / 4);
     hipError_t e = hipMemcpyAsync(grads, N.g, N.nparam * 4, hipMemcpyDeviceToHost, st);
     if (!e) e = hipMemcpyAsync(lp.data(), N.lossp, lp.size() * 4, hipMemcpyDeviceToHost, st);
@@ -1226,21 +1669,32 @@ qi_status qi_mlp_train_epoch(qi_mlp_t m, uint32_t batch, float lr, uint64_t shuf
     hipError_t e = hipMemcpy(N.perm, perm.data(), perm.size() * 4, hipMemcpyHostToDevice);
     if (e) QM_RET(make_err(QI_ERR_DEVICE, 0, 0, 0, 0, hipGetErrorString(e)));
     const size_t nb = N.ndata / batch;  // full batches only
+    const bool small = small_step(N, batch);
+    if (small) QM_TRY(small_alloc(N, batch));
     if ((e = hipMemsetAsync(N.lacc, 0, sizeof(double), st))) QM_RET(make_err(QI_ERR_DEVICE, 0, 0, 0, 0, hipGetErrorString(e)));
     (void)hipEventRecord(N.ctx->ev0, st);
     // no host round trip inside the epoch: the head bias is read on the
     // device and the loss accumulates on the device
     for (size_t b = 0; b < nb; b++) {
-        hipLaunchKernelGGL(k_gather_rows, dim3(batch), dim3(256), 0, st, (const bf16 *)N.dataX, (const uint32_t *)N.perm + b * batch,
+        const uint32_t *idx = (const uint32_t *)N.perm + b * batch;
+        N.step++;
+        const float b1 = 0.9f, b2 = 0.999f;
+        const AdamStep ad{lr, b1, b2, 1e-8f, 1.f - std::pow(b1, (float)N.step), 1.f - std::pow(b2, (float)N.step)};
+        if (small) {
+            if (b == 0)
+                hipLaunchKernelGGL(k_gather_rows8, dim3(batch / 8), dim3(256), size_t(N.k_in) * 8 * sizeof(bf16), st,
+                                   gather_of(N, idx, (int)batch));
+            small_forward(N, st, (int)batch);
+            small_backward(N, st, (int)batch, N.lacc);
+            small_adam(N, st, (int)batch, ad, b + 1 < nb ? idx + batch : nullptr);
+            continue;
+        }
+        hipLaunchKernelGGL(k_gather_rows, dim3(batch), dim3(256), 0, st, (const bf16 *)N.dataX, idx,
                            (int)batch, N.k_in, N.X, (const float *)N.dataT, N.t);
         forward(N, st, (int)batch, true);
         backward(N, st, (int)batch);
         hipLaunchKernelGGL(k_loss_accum, dim3(1), dim3(256), 0, st, (const float *)N.lossp, (int)((batch + 3) / 4), N.lacc);
-        N.step++;
-        const float b1 = 0.9f, b2 = 0.999f;
-        const float c1 = 1.f - std::pow(b1, (float)N.step), c2 = 1.f - std::pow(b2, (float)N.step);
-        hipLaunchKernelGGL(k_adam, dim3(1024), dim3(256), 0, st, N.w, N.m, N.v, (const float *)N.g, N.wb, N.nparam, lr, b1, b2,
-                           1e-8f, c1, c2);
+        hipLaunchKernelGGL(k_adam, dim3(1024), dim3(256), 0, st, N.w, N.m, N.v, (const float *)N.g, N.wb, N.nparam, ad);
         const int rows[3] = {N.k_in, N.hid, N.hid};
         for (int l = 0; l < 3; l++)
             hipLaunchKernelGGL(k_transpose_bf16, dim3((N.hid + 31) / 32, (rows[l] + 31) / 32), dim3(256), 0, st,
