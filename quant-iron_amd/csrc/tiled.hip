@@ -17,6 +17,8 @@
 // Arithmetic: both precisions use fused multiply-adds in the register ops
 // (complex128 tiles agree with the reference's unfused products to about
 // 1e-15 per gate); the LDS gates keep the reference's products.
+#include <type_traits>
+
 #include "qi_internal.h"
 #include "exec_plan.h"
 
@@ -43,6 +45,7 @@ template <typename T> __device__ __forceinline__ T cadd(T a, T b) { return mk<T>
 template <typename T> __device__ __forceinline__ T csub(T a, T b) { return mk<T>(a.x - b.x, a.y - b.y); }
 template <typename T, typename R> __device__ __forceinline__ T cscale(R f, T a) { return mk<T>(f * a.x, f * a.y); }
 
+__host__ __device__ constexpr uint32_t ins0_const(uint32_t k, unsigned p) { return ((k >> p) << (p + 1)) | (k & ((1u << p) - 1)); }
 __device__ __forceinline__ uint32_t ins0(uint32_t k, unsigned p) { return ((k >> p) << (p + 1)) | (k & ((1u << p) - 1)); }
 
 __device__ __forceinline__ uint64_t insert_zeros64(uint64_t k, uint64_t fixed) {
@@ -101,6 +104,99 @@ __device__ __forceinline__ double xlane(int addr, double x) {
     return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
 }
 template <typename T> __device__ __forceinline__ T xlane2(int addr, T x) { return mk<T>(xlane(addr, x.x), xlane(addr, x.y)); }
+
+// Lane bits 0-3 stay inside a row of 16 lanes, so values cross them as data
+// parallel operands of VALU moves. Measured on one MI355X (cycles at 2.4 GHz
+// per instruction and SIMD, three waves): a ds_bpermute 25 (the four SIMDs
+// share the LDS crossbar), a DPP move 4.6, v_cndmask with a scalar mask 4.2
+// (17 and more through VCC), v_bitop3 2.7, v_fma_f32 2.6, v_permlane*_swap
+// 8.7 (11.2 with a wait of its own). A VALU result needs two wait states
+// before a DPP operand reads it: every block below starts with them or with
+// four unrelated instructions, and spaces its own results by three.
+#define QI_DPP_X1 "quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf"     // lane ^ 1
+#define QI_DPP_X2 "quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf"     // lane ^ 2
+#define QI_DPP_X3 "quad_perm:[3,2,1,0] row_mask:0xf bank_mask:0xf"     // lane ^ 3
+#define QI_DPP_X7 "row_half_mirror row_mask:0xf bank_mask:0xf"         // lane ^ 7
+#define QI_DPP_X8 "row_ror:8 row_mask:0xf bank_mask:0xf"               // lane ^ 8
+#define QI_MOV4(D) "v_mov_b32_dpp %0, %4 " D "\n\tv_mov_b32_dpp %1, %5 " D "\n\tv_mov_b32_dpp %2, %6 " D "\n\tv_mov_b32_dpp %3, %7 " D
+#define QI_MOV4_SELF(D) "v_mov_b32_dpp %0, %0 " D "\n\tv_mov_b32_dpp %1, %1 " D "\n\tv_mov_b32_dpp %2, %2 " D "\n\tv_mov_b32_dpp %3, %3 " D
+// y = x of lane ^ 2^I, four words
+template <int I> __device__ __forceinline__ void partner4(uint32_t (&y)[4], const uint32_t (&x)[4]) {
+#define QI_P4(CODE)                                                                                                       \
+    asm("s_nop 1\n\t" CODE : "=&v"(y[0]), "=&v"(y[1]), "=&v"(y[2]), "=&v"(y[3]) : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]))
+    if constexpr (I == 0) QI_P4(QI_MOV4(QI_DPP_X1));
+    else if constexpr (I == 1) QI_P4(QI_MOV4(QI_DPP_X2));
+    else if constexpr (I == 2) QI_P4(QI_MOV4(QI_DPP_X7) "\n\t" QI_MOV4_SELF(QI_DPP_X3));  // 7 ^ 3 = 4
+    else QI_P4(QI_MOV4(QI_DPP_X8));
+#undef QI_P4
+}
+// x = x of lane ^ 2^I in place, four words
+template <int I> __device__ __forceinline__ void flip4(uint32_t &x0, uint32_t &x1, uint32_t &x2, uint32_t &x3) {
+#define QI_F4(CODE) asm("s_nop 1\n\t" CODE : "+v"(x0), "+v"(x1), "+v"(x2), "+v"(x3))
+    if constexpr (I == 0) QI_F4(QI_MOV4_SELF(QI_DPP_X1));
+    else if constexpr (I == 1) QI_F4(QI_MOV4_SELF(QI_DPP_X2));
+    else if constexpr (I == 2) QI_F4(QI_MOV4_SELF(QI_DPP_X7) "\n\t" QI_MOV4_SELF(QI_DPP_X3));
+    else QI_F4(QI_MOV4_SELF(QI_DPP_X8));
+#undef QI_F4
+}
+// The lanes with bit I set trade a with the b of their partners (lane ^ 2^I),
+// four word pairs. Bits 2 and 3 select the written lanes by the moves' bank
+// masks (a copy of a, two moves), bits 0 and 1 by the lane mask hi (all ones
+// where the bit is set): select what to send, move it, select twice.
+#define QI_MOV8(D0, D1)                                                                                                   \
+    "v_mov_b32 %8, %0\n\tv_mov_b32 %9, %1\n\tv_mov_b32 %10, %2\n\tv_mov_b32 %11, %3\n\t"                                  \
+    "v_mov_b32_dpp %0, %4 " D0 "\n\tv_mov_b32_dpp %1, %5 " D0 "\n\tv_mov_b32_dpp %2, %6 " D0 "\n\tv_mov_b32_dpp %3, %7 " D0  \
+    "\n\tv_mov_b32_dpp %4, %8 " D1 "\n\tv_mov_b32_dpp %5, %9 " D1 "\n\tv_mov_b32_dpp %6, %10 " D1 "\n\tv_mov_b32_dpp %7, %11 " D1
+#define QI_SEL8(D)                                                                                                        \
+    "v_bitop3_b32 %8, %4, %0, %12 bitop3:0xd8\n\tv_bitop3_b32 %9, %5, %1, %12 bitop3:0xd8\n\t"                            \
+    "v_bitop3_b32 %10, %6, %2, %12 bitop3:0xd8\n\tv_bitop3_b32 %11, %7, %3, %12 bitop3:0xd8\n\t"                          \
+    "v_mov_b32_dpp %8, %8 " D "\n\tv_mov_b32_dpp %9, %9 " D "\n\tv_mov_b32_dpp %10, %10 " D "\n\tv_mov_b32_dpp %11, %11 " D \
+    "\n\tv_bitop3_b32 %0, %0, %8, %12 bitop3:0xd8\n\tv_bitop3_b32 %1, %1, %9, %12 bitop3:0xd8\n\t"                        \
+    "v_bitop3_b32 %2, %2, %10, %12 bitop3:0xd8\n\tv_bitop3_b32 %3, %3, %11, %12 bitop3:0xd8\n\t"                          \
+    "v_bitop3_b32 %4, %4, %8, %12 bitop3:0xe4\n\tv_bitop3_b32 %5, %5, %9, %12 bitop3:0xe4\n\t"                            \
+    "v_bitop3_b32 %6, %6, %10, %12 bitop3:0xe4\n\tv_bitop3_b32 %7, %7, %11, %12 bitop3:0xe4"
+template <int I> __device__ __forceinline__ void trade4(uint32_t (&a)[4], uint32_t (&b)[4], uint32_t hi) {
+    uint32_t t[4];
+#define QI_T4(CODE)                                                                                                       \
+    asm(CODE                                                                                                              \
+        : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3]), "=&v"(t[0]),    \
+          "=&v"(t[1]), "=&v"(t[2]), "=&v"(t[3])                                                                           \
+        : "v"(hi))
+    if constexpr (I == 0) QI_T4(QI_SEL8(QI_DPP_X1));
+    else if constexpr (I == 1) QI_T4(QI_SEL8(QI_DPP_X2));
+    else if constexpr (I == 2) QI_T4(QI_MOV8("row_shr:4 row_mask:0xf bank_mask:0xa", "row_shl:4 row_mask:0xf bank_mask:0x5"));
+    else QI_T4(QI_MOV8("row_ror:8 row_mask:0xf bank_mask:0xc", "row_ror:8 row_mask:0xf bank_mask:0x3"));
+#undef QI_T4
+}
+// The components of a tile as 32-bit words (a complex128 component is two).
+__device__ __forceinline__ void to_words(float x, uint32_t *w) { w[0] = __float_as_uint(x); }
+__device__ __forceinline__ void to_words(double x, uint32_t *w) {
+    const uint64_t b = (uint64_t)__double_as_longlong(x);
+    w[0] = (uint32_t)b;
+    w[1] = (uint32_t)(b >> 32);
+}
+__device__ __forceinline__ void from_words(const uint32_t *w, float &x) { x = __uint_as_float(w[0]); }
+__device__ __forceinline__ void from_words(const uint32_t *w, double &x) {
+    x = __longlong_as_double((long long)(((uint64_t)w[1] << 32) | w[0]));
+}
+template <typename R> constexpr int kWords = sizeof(R) / 4;
+// (a, b) trade places on the lanes whose mask word is all ones (a controlled
+// swap: difference under the mask, added to both)
+__device__ __forceinline__ void ip_cswap32(uint32_t &a, uint32_t &b, uint32_t m) {
+    uint32_t t;
+    asm("v_bitop3_b32 %0, %1, %2, %3 bitop3:0x28" : "=v"(t) : "v"(a), "v"(b), "v"(m));  // (a ^ b) & m
+    asm("v_xor_b32 %0, %0, %1" : "+v"(a) : "v"(t));
+    asm("v_xor_b32 %0, %0, %1" : "+v"(b) : "v"(t));
+}
+template <typename R> __device__ __forceinline__ void ip_cswap(R &a, R &b, uint32_t m) {
+    uint32_t x[kWords<R>], y[kWords<R>];
+    to_words(a, x);
+    to_words(b, y);
+#pragma unroll
+    for (int w = 0; w < kWords<R>; w++) ip_cswap32(x[w], y[w], m);
+    from_words(x, a);
+    from_words(y, b);
+}
 
 // ------------------------------------------------------ in-place updates --
 // A tile lives in registers across a loop whose body dispatches on
@@ -272,6 +368,26 @@ __device__ __forceinline__ void pairs_reg(Regs<R, E> &v, const R *k, uint32_t rc
     R nk[8];
 #pragma unroll
     for (int q = 0; q < 8; q++) nk[q] = -k[q];
+    if constexpr (CT && KIND == RO_X) {  // controlled swap under the lane mask (and the register's)
+        const uint32_t m = tok ? ~0u : 0u;
+        if (rcm == 0) {
+#pragma unroll
+            for (int r = 0; r < E; r++) {
+                if (r & (1 << B)) continue;
+                ip_cswap(v.d[2 * r], v.d[2 * (r | (1 << B))], m);
+                ip_cswap(v.d[2 * r + 1], v.d[2 * (r | (1 << B)) + 1], m);
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < E; r++) {
+                if (r & (1 << B)) continue;
+                const uint32_t mr = (uint32_t(r) & rcm) == rcm ? m : 0u;
+                ip_cswap(v.d[2 * r], v.d[2 * (r | (1 << B))], mr);
+                ip_cswap(v.d[2 * r + 1], v.d[2 * (r | (1 << B)) + 1], mr);
+            }
+        }
+        return;
+    }
     const uint64_t tokm = CT ? __builtin_amdgcn_ballot_w64(tok) : 0;
 #pragma unroll
     for (int r = 0; r < E; r++) {
@@ -288,12 +404,6 @@ __device__ __forceinline__ void pairs_reg(Regs<R, E> &v, const R *k, uint32_t rc
             } else ip_gen(ax, ay, bx, by, k, nk);
         } else {
             const uint64_t m = (uint32_t(r) & rcm) == rcm ? tokm : 0;  // uniform per register
-            if constexpr (KIND == RO_X) {  // controlled swap: new b first, then a and b in place
-                const R tx = selm(m, ax, bx), ty = selm(m, ay, by);
-                ip_sel(ax, bx, m); ip_sel(ay, by, m);
-                ip_set(bx, tx); ip_set(by, ty);
-                continue;
-            }
             if constexpr (KIND == RO_Y) {  // all four new values first, then in place
                 const R n0 = selm(m, by, ax), n1 = selm(m, -bx, ay), n2 = selm(m, -ay, bx), n3 = selm(m, ax, by);
                 ip_set(ax, n0); ip_set(ay, n1); ip_set(bx, n2); ip_set(by, n3);
@@ -318,8 +428,44 @@ __device__ __forceinline__ void pairs_reg(Regs<R, E> &v, const R *k, uint32_t rc
 
 // Lane pairs: s = own amplitude, p = partner's; k holds this lane's row of
 // the matrix (own coefficient first).
-template <int KIND, bool CT, int E, typename T, typename R>
+// The partners (lane ^ 2^I, I < 4) of G components by DPP.
+template <int I, typename R, int G> __device__ __forceinline__ void fetch_partners(R (&p)[G], const R (&own)[G]) {
+    constexpr int W = kWords<R>, N = 4 / W;
+    static_assert(G % N == 0, "whole blocks of four words");
+#pragma unroll
+    for (int g = 0; g < G; g += N) {
+        uint32_t x[4], y[4];
+#pragma unroll
+        for (int q = 0; q < N; q++) to_words(own[g + q], x + W * q);
+        partner4<I>(y, x);
+#pragma unroll
+        for (int q = 0; q < N; q++) from_words(y + W * q, p[g + q]);
+    }
+}
+// Four words' worth of components (flat indices idx) flipped across lane bit I < 4 in place.
+template <int I, int E, typename R> __device__ __forceinline__ void flip_block(Regs<R, E> &v, const int *idx) {
+    constexpr int W = kWords<R>, N = 4 / W;
+    uint32_t x[4];
+#pragma unroll
+    for (int q = 0; q < N; q++) to_words(v.d[idx[q]], x + W * q);
+    flip4<I>(x[0], x[1], x[2], x[3]);
+#pragma unroll
+    for (int q = 0; q < N; q++) from_words(x + W * q, v.d[idx[q]]);
+}
+// I: the lane bit when it is below 4 (partners by DPP), else -1 (ds_bpermute from addr).
+template <int KIND, bool CT, int I, int E, typename T, typename R>
 __device__ __forceinline__ void pairs_lane(Regs<R, E> &v, int addr, const R *k, uint32_t rcm, bool tok) {
+    if constexpr (!CT && KIND == RO_X && I >= 0) {  // every amplitude moves: in place
+        constexpr int N = 4 / kWords<R>;
+#pragma unroll
+        for (int q = 0; q < 2 * E; q += N) {
+            int idx[N];
+#pragma unroll
+            for (int j = 0; j < N; j++) idx[j] = q + j;
+            flip_block<I, E, R>(v, idx);
+        }
+        return;
+    }
     const R nk1 = -k[1], nk3 = -k[3];
     const uint64_t tokm = CT ? __builtin_amdgcn_ballot_w64(tok) : 0;
     // partners fetched a group of registers ahead: the exchange latency
@@ -328,8 +474,17 @@ __device__ __forceinline__ void pairs_lane(Regs<R, E> &v, int addr, const R *k, 
 #pragma unroll
     for (int r0 = 0; r0 < E; r0 += G) {
         R px[G], py[G];
+        if constexpr (I >= 0) {
+            R own[2 * G], p[2 * G];
 #pragma unroll
-        for (int g = 0; g < G; g++) { px[g] = xlane(addr, v.d[2 * (r0 + g)]); py[g] = xlane(addr, v.d[2 * (r0 + g) + 1]); }
+            for (int g = 0; g < 2 * G; g++) own[g] = v.d[2 * r0 + g];
+            fetch_partners<I>(p, own);
+#pragma unroll
+            for (int g = 0; g < G; g++) { px[g] = p[2 * g]; py[g] = p[2 * g + 1]; }
+        } else {
+#pragma unroll
+            for (int g = 0; g < G; g++) { px[g] = xlane(addr, v.d[2 * (r0 + g)]); py[g] = xlane(addr, v.d[2 * (r0 + g) + 1]); }
+        }
 #pragma unroll
         for (int g = 0; g < G; g++) {
             const int r = r0 + g;
@@ -387,7 +542,16 @@ __device__ __forceinline__ void pair_op(Regs<R, E> &v, const RegOp &op, uint32_t
             k[2] = bit ? coef<R>(op, 4) : coef<R>(op, 2);
             k[3] = bit ? coef<R>(op, 5) : coef<R>(op, 3);
         }
-        pairs_lane<KIND, CT, E, T, R>(v, addr, k, rcm, tok);
+        if constexpr (!CT) {  // (controlled lane targets are rare: one form)
+            switch (i) {
+            case 0: pairs_lane<KIND, CT, 0, E, T, R>(v, addr, k, rcm, tok); return;
+            case 1: pairs_lane<KIND, CT, 1, E, T, R>(v, addr, k, rcm, tok); return;
+            case 2: pairs_lane<KIND, CT, 2, E, T, R>(v, addr, k, rcm, tok); return;
+            case 3: pairs_lane<KIND, CT, 3, E, T, R>(v, addr, k, rcm, tok); return;
+            default: break;
+            }
+        }
+        pairs_lane<KIND, CT, -1, E, T, R>(v, addr, k, rcm, tok);
         return;
     }
     R k[8];
@@ -404,6 +568,7 @@ __device__ __forceinline__ void pair_op(Regs<R, E> &v, const RegOp &op, uint32_t
 template <int B, int KIND, bool CT, int E, typename T, typename R>
 __device__ __forceinline__ void diag_reg(Regs<R, E> &v, T p0, T p1, uint32_t rcm, bool tok) {
     const R n0 = -p0.y, n1 = -p1.y;
+    const uint32_t tsgn = tok ? 0x80000000u : 0u;  // controlled Z: sign flip on the lanes whose controls hold
     const uint64_t tokm = CT ? __builtin_amdgcn_ballot_w64(tok) : 0;
 #pragma unroll
     for (int r = 0; r < E; r++) {
@@ -416,8 +581,11 @@ __device__ __forceinline__ void diag_reg(Regs<R, E> &v, T p0, T p1, uint32_t rcm
             else ip_cmul(ax, ay, p.x, p.y, one ? n1 : n0);
         } else {
             const uint64_t m = (uint32_t(r) & rcm) == rcm ? tokm : 0;
-            if constexpr (KIND == RO_Z) { ip_sel(ax, -ax, m); ip_sel(ay, -ay, m); }
-            else {
+            if constexpr (KIND == RO_Z) {
+                const uint32_t sgn = (uint32_t(r) & rcm) == rcm ? tsgn : 0u;
+                ip_xor(ax, sgn);
+                ip_xor(ay, sgn);
+            } else {
                 const T n = cmul(mk<T>(ax, ay), p);
                 ip_sel(ax, n.x, m); ip_sel(ay, n.y, m);
             }
@@ -439,8 +607,9 @@ __device__ __forceinline__ void diag_thr(Regs<R, E> &v, T f, bool one, uint32_t 
         } else {
             const uint64_t m = (uint32_t(r) & rcm) == rcm ? tokm : 0;
             if constexpr (KIND == RO_Z) {
-                ip_sel(ax, xor_sign(ax, sgn), m);
-                ip_sel(ay, xor_sign(ay, sgn), m);
+                const uint32_t rs = (uint32_t(r) & rcm) == rcm && tok ? sgn : 0u;
+                ip_xor(ax, rs);
+                ip_xor(ay, rs);
             } else {
                 const T n = cmul(mk<T>(ax, ay), f);
                 ip_sel(ax, n.x, m); ip_sel(ay, n.y, m);
@@ -478,13 +647,30 @@ __device__ __forceinline__ void x_reg_c1(Regs<R, E> &v) {
     }
 }
 template <int C, int E, typename R>
-__device__ __forceinline__ void x_lane_c1(Regs<R, E> &v, int addr) {
+__device__ __forceinline__ void x_lane_c1(Regs<R, E> &v, int i, int addr) {
     constexpr int G0 = sizeof(R) == 4 ? 4 : 2, H = E / 2, G = H < G0 ? H : G0;
     int rs[H];
     {
         int n = 0;
 #pragma unroll
         for (int r = 0; r < E; r++) if ((r >> C) & 1) rs[n++] = r;
+    }
+    constexpr int N = 4 / kWords<R>;  // components per block of four words
+    const auto flip = [&](auto bit) {
+#pragma unroll
+        for (int q = 0; q < 2 * H; q += N) {
+            int idx[N];
+#pragma unroll
+            for (int j = 0; j < N; j++) idx[j] = 2 * rs[(q + j) / 2] + (q + j) % 2;
+            flip_block<decltype(bit)::value, E, R>(v, idx);
+        }
+    };
+    switch (i) {
+    case 0: flip(std::integral_constant<int, 0>{}); return;
+    case 1: flip(std::integral_constant<int, 1>{}); return;
+    case 2: flip(std::integral_constant<int, 2>{}); return;
+    case 3: flip(std::integral_constant<int, 3>{}); return;
+    default: break;
     }
 #pragma unroll
     for (int g0 = 0; g0 < H; g0 += G) {
@@ -535,14 +721,14 @@ template <int E, typename R> __device__ __forceinline__ void xc1_op(Regs<R, E> &
     constexpr int RB = __builtin_ctz(E);
     const int c = op.lp0;
     if (op.tgt >= kLaneTarget) {
-        const int addr = int((lane ^ (1u << (op.tgt - kLaneTarget))) << 2);
+        const int i = op.tgt - kLaneTarget, addr = int((lane ^ (1u << i)) << 2);
         switch (c) {
-        case 0: if constexpr (0 < RB) x_lane_c1<0, E, R>(v, addr); break;
-        case 1: if constexpr (1 < RB) x_lane_c1<1, E, R>(v, addr); break;
-        case 2: if constexpr (2 < RB) x_lane_c1<2, E, R>(v, addr); break;
-        case 3: if constexpr (3 < RB) x_lane_c1<3, E, R>(v, addr); break;
-        case 4: if constexpr (4 < RB) x_lane_c1<4, E, R>(v, addr); break;
-        case 5: if constexpr (5 < RB) x_lane_c1<5, E, R>(v, addr); break;
+        case 0: if constexpr (0 < RB) x_lane_c1<0, E, R>(v, i, addr); break;
+        case 1: if constexpr (1 < RB) x_lane_c1<1, E, R>(v, i, addr); break;
+        case 2: if constexpr (2 < RB) x_lane_c1<2, E, R>(v, i, addr); break;
+        case 3: if constexpr (3 < RB) x_lane_c1<3, E, R>(v, i, addr); break;
+        case 4: if constexpr (4 < RB) x_lane_c1<4, E, R>(v, i, addr); break;
+        case 5: if constexpr (5 < RB) x_lane_c1<5, E, R>(v, i, addr); break;
         default: break;
         }
         return;
@@ -582,20 +768,27 @@ __device__ __forceinline__ void zc1_op(Regs<R, E> &v, const RegOp &op, uint32_t 
 template <int B, bool XS, int E>
 __device__ __forceinline__ void shear_reg(Regs<float, E> &v, float a, float b) {
     const float na = -a, nb = -b;
+    // two register pairs (four chains of three) interleaved: 545 cycles per
+    // 64 amplitudes against 618 one pair at a time
+    constexpr int G = 2;
 #pragma unroll
-    for (int r = 0; r < E; r++) {
-        if ((r >> B) & 1) continue;
-        const int s = r | (1 << B);
-        float &p0 = v.d[2 * r], &q0 = v.d[2 * s + (XS ? 1 : 0)];   // first pair, angle phi
-        float &p1 = v.d[2 * r + 1], &q1 = v.d[2 * s + (XS ? 0 : 1)];  // second pair, angle +-phi
-        const float a1 = XS ? na : a, b1 = XS ? nb : b;
-        ip_fmac(p0, a, q0);
-        ip_fmac(p1, a1, q1);
-        ip_fmac(q0, b, p0);
-        ip_fmac(q1, b1, p1);
-        ip_fmac(p0, a, q0);
-        ip_fmac(p1, a1, q1);
-    }
+    for (int n0 = 0; n0 < E / 2; n0 += G)
+#pragma unroll
+        for (int st = 0; st < 3; st++)
+#pragma unroll
+            for (int g = 0; g < G; g++) {
+                const int r = int(ins0_const(n0 + g, B)), q = r | (1 << B);
+                float &p0 = v.d[2 * r], &q0 = v.d[2 * q + (XS ? 1 : 0)];      // first pair, angle phi
+                float &p1 = v.d[2 * r + 1], &q1 = v.d[2 * q + (XS ? 0 : 1)];  // second pair, angle +-phi
+                const float a1 = XS ? na : a, b1 = XS ? nb : b;
+                if (st != 1) {
+                    ip_fmac(p0, a, q0);
+                    ip_fmac(p1, a1, q1);
+                } else {
+                    ip_fmac(q0, b, p0);
+                    ip_fmac(q1, b1, p1);
+                }
+            }
 }
 template <bool XS, int E> __device__ __forceinline__ void shear_op(Regs<float, E> &v, const RegOp &op) {
     constexpr int RB = __builtin_ctz(E);
@@ -648,68 +841,50 @@ template <int E> __device__ __forceinline__ void hs_op(Regs<float, E> &v, const 
 }
 
 // ------------------------------------------------------- exchange ops --
-// a's lanes with lane bit 4 (5) set trade with b's lanes where it is clear:
-// v_permlane16_swap / v_permlane32_swap, one VALU instruction per 32-bit
-// component, both registers updated in place (tied operands, like the other
-// in-place ops). A VALU write of a register that a permlane swap reads needs
-// two wait states before the swap: each swap carries its own s_nop 1, so no
-// instruction the compiler places in between can break that.
-__device__ __forceinline__ void swap_rows32(uint32_t &a, uint32_t &b, bool b5) {
-    if (b5) asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
-    else asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+// Lane bits 4 and 5: v_permlane16_swap / v_permlane32_swap trade a's lanes
+// with the bit set for b's lanes where it is clear, one VALU instruction per
+// word, both registers in place. A VALU result needs two wait states before a
+// swap reads it: one s_nop 1 per block of four.
+#define QI_SWAP4(OP) "s_nop 1\n\t" OP " %0, %4\n\t" OP " %1, %5\n\t" OP " %2, %6\n\t" OP " %3, %7"
+template <int I> __device__ __forceinline__ void swap_rows4(uint32_t (&a)[4], uint32_t (&b)[4]) {
+#define QI_S4(OP)                                                                                                         \
+    asm volatile(QI_SWAP4(OP)                                                                                             \
+                 : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3]))
+    if constexpr (I == 5) QI_S4("v_permlane32_swap_b32");
+    else QI_S4("v_permlane16_swap_b32");
+#undef QI_S4
 }
-__device__ __forceinline__ void swap_rows(float &a, float &b, bool b5) {
-    uint32_t x = __float_as_uint(a), y = __float_as_uint(b);
-    swap_rows32(x, y, b5);
-    a = __uint_as_float(x);
-    b = __uint_as_float(y);
-}
-__device__ __forceinline__ void swap_rows(double &a, double &b, bool b5) {
-    uint32_t al = lo32(a), ah = hi32(a), bl = lo32(b), bh = hi32(b);
-    swap_rows32(al, bl, b5);
-    swap_rows32(ah, bh, b5);
-    a = mk64(al, ah);
-    b = mk64(bl, bh);
+template <int B, int I, int E, typename R> __device__ __forceinline__ void xlr_bits(Regs<R, E> &v, uint32_t lane) {
+    constexpr int W = kWords<R>, N = 4 / W;
+    const uint32_t hi = I < 2 && ((lane >> I) & 1u) ? ~0u : 0u;
+#pragma unroll
+    for (int n = 0; n < E; n += N) {  // n: component n % 2 of register pair n / 2
+        uint32_t a[4], b[4];
+#pragma unroll
+        for (int q = 0; q < N; q++) {
+            const int r = int(ins0_const((n + q) / 2, B)), c = (n + q) % 2;
+            to_words(v.d[2 * r + c], a + W * q);
+            to_words(v.d[2 * (r | (1 << B)) + c], b + W * q);
+        }
+        if constexpr (I >= 4) swap_rows4<I>(a, b);
+        else trade4<I>(a, b, hi);
+#pragma unroll
+        for (int q = 0; q < N; q++) {
+            const int r = int(ins0_const((n + q) / 2, B)), c = (n + q) % 2;
+            from_words(a + W * q, v.d[2 * r + c]);
+            from_words(b + W * q, v.d[2 * (r | (1 << B)) + c]);
+        }
+    }
 }
 template <int B, int E, typename R>
 __device__ __forceinline__ void xlr_reg(Regs<R, E> &v, uint32_t lane, int i) {
-    if (i >= 4) {  // lane bits 4 and 5: one cross-row swap per component pair, no lane addressing
-        const bool b5 = i == 5;
-#pragma unroll
-        for (int r = 0; r < E; r++) {
-            if (r & (1 << B)) continue;
-#pragma unroll
-            for (int c = 0; c < 2; c++) swap_rows(v.d[2 * r + c], v.d[2 * (r | (1 << B)) + c], b5);
-        }
-        return;
-    }
-    const int addr = int((lane ^ (1u << i)) << 2);
-    const uint64_t hi = __builtin_amdgcn_ballot_w64(((lane >> i) & 1u) != 0), lo = ~hi;
-    constexpr int G = sizeof(R) == 4 ? 4 : 2;  // exchanges issued a group ahead of their use
-    int rs[E / 2];
-    {
-        int n = 0;
-#pragma unroll
-        for (int r = 0; r < E; r++) if (!(r & (1 << B))) rs[n++] = r;
-    }
-#pragma unroll
-    for (int g0 = 0; g0 < E / 2; g0 += G) {
-        R y[G][2];
-#pragma unroll
-        for (int g = 0; g < G && g0 + g < E / 2; g++)
-#pragma unroll
-            for (int c = 0; c < 2; c++) {
-                const int r = rs[g0 + g];
-                y[g][c] = xlane(addr, selm(hi, v.d[2 * r + c], v.d[2 * (r | (1 << B)) + c]));
-            }
-#pragma unroll
-        for (int g = 0; g < G && g0 + g < E / 2; g++)
-#pragma unroll
-            for (int c = 0; c < 2; c++) {
-                const int r = rs[g0 + g];
-                ip_sel(v.d[2 * (r | (1 << B)) + c], y[g][c], lo);
-                ip_sel(v.d[2 * r + c], y[g][c], hi);
-            }
+    switch (i) {
+    case 0: xlr_bits<B, 0, E, R>(v, lane); break;
+    case 1: xlr_bits<B, 1, E, R>(v, lane); break;
+    case 2: xlr_bits<B, 2, E, R>(v, lane); break;
+    case 3: xlr_bits<B, 3, E, R>(v, lane); break;
+    case 4: xlr_bits<B, 4, E, R>(v, lane); break;
+    default: xlr_bits<B, 5, E, R>(v, lane); break;
     }
 }
 template <int E, typename R>
