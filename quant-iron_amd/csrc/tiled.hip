@@ -103,7 +103,6 @@ __device__ __forceinline__ double xlane(int addr, double x) {
     const int hi = __builtin_amdgcn_ds_bpermute(addr, (int)(b >> 32));
     return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
 }
-template <typename T> __device__ __forceinline__ T xlane2(int addr, T x) { return mk<T>(xlane(addr, x.x), xlane(addr, x.y)); }
 
 // Lane bits 0-3 stay inside a row of 16 lanes, so values cross them as data
 // parallel operands of VALU moves. Measured on one MI355X (cycles at 2.4 GHz
@@ -1166,6 +1165,10 @@ __global__ __launch_bounds__(64) void k_wave_pass(const typename V2<R>::T *src_p
     using T = typename V2<R>::T;
     constexpr int TB = kLaneBits, RB = K - TB, E = 1 << RB;
     const uint32_t lane = threadIdx.x;
+    // A wave that still has loads to issue goes first: its data is on the way
+    // while the SIMD's other waves compute (25-qubit Trotter steps 7.55 -> 7.35
+    // ms complex64, 27-qubit random circuit 9.83 -> 9.65 ms complex128).
+    __builtin_amdgcn_s_setprio(3);
     const uint64_t base = insert_zeros64(xcd_block_order(blockIdx.x, pass.chunk_log2), pass.qmask);
     uint64_t at_in = 0, at_out = 0, tmask = 0;
 #pragma unroll
@@ -1186,6 +1189,7 @@ __global__ __launch_bounds__(64) void k_wave_pass(const typename V2<R>::T *src_p
             v.set(r, ld_stream(src + o));
         }
     }
+    __builtin_amdgcn_s_setprio(0);
     // The op table of a pass ends with a no-op, so op o + 1 can be fetched
     // while op o runs. One-wave passes hold no LDS ops (the planner streams them).
     R ph[2] = {R(1), R(0)};  // the lane's pending phase
