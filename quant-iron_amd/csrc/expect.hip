@@ -68,13 +68,14 @@ __device__ __forceinline__ void pair_products(const double (&ar)[kExpSlots], con
     }
 }
 
-// What bounds it: FP64 issue and one read of the state per pass, about evenly
-// (two 64 KiB tiles per CU, so one loads while the other computes). The
+// What bounds it: FP64 issue (VALU busy 44% of the time) and one read of the
+// state per pass (2.6 TB/s), neither hidden well behind the other: a CU holds
+// 16 waves (128 VGPRs), in two workgroups at 64 KiB tiles, four at 32 KiB. The
 // four-bit register sets share the LDS reads (16 per thread and set) and the
 // FP64 conversions among the masks of the set; a Heisenberg bond costs a
 // multiply-add pair and one multiply-add per amplitude pair, whatever its
 // number of terms. 29 qubits, complex64, a chain with fields (113 terms, 29 x
-// masks): 67.1 ms with one read of the state per mask, 4.9 ms in three passes.
+// masks): 67.1 ms with one read of the state per mask, 5.0 ms in four passes.
 // The imaginary sums (complex coefficients) take registers that cost half the
 // waves, so they have an instance of their own.
 template <typename T, bool CPLX>

@@ -71,12 +71,9 @@ int exp_tile_qubits(uint32_t n, bool c128) {
 }
 
 void plan_expect(uint32_t n, bool c128, const qi_pauli_term *terms, size_t nt, ExpPlan &p) {
-    const int K = exp_tile_qubits(n, c128), low = exp_low_qubits(c128);
-    p.K = K;
+    const int low = exp_low_qubits(c128);
     p.npasses = p.nsets = p.nunits = p.ndiags = p.nfar = 0;
     p.complex_out = false;
-    const bool whole = (int)n == K;
-    const uint64_t lowmask = whole ? (uint64_t(1) << n) - 1 : (uint64_t(1) << low) - 1;
     // distinct nonzero x masks in order of appearance; next term of the same mask in gid[nt + k]
     size_t nx = 0;
     uint32_t *const head = p.gid, *const next = p.gid + nt;  // head: first term of mask g
@@ -97,6 +94,21 @@ void plan_expect(uint32_t n, bool c128, const qi_pauli_term *terms, size_t nt, E
             next[t] = (uint32_t)k;
         }
     }
+    // A complex64 state of more qubits than its widest tile takes tiles of one
+    // qubit less, unless a mask needs that one: at half the LDS, four
+    // workgroups per CU load and compute out of step instead of two. 28 qubits,
+    // 4 x 7 lattice: 3.76 -> 3.48 ms; 24-qubit chain 232 -> 207 us; 29-qubit chain
+    // 5.09 -> 5.01 ms (11 qubits: 3.86 ms, 211 us, 5.07 ms; complex128 with 11
+    // instead of 12: 1.92 -> 2.16 ms at 27 qubits).
+    int K = exp_tile_qubits(n, c128);
+    const bool whole = (int)n == K;
+    const uint64_t lowmask = whole ? (uint64_t(1) << n) - 1 : (uint64_t(1) << low) - 1;
+    if (!c128 && !whole) {
+        K--;
+        for (size_t g = 0; g < nx; g++)
+            if (popc(p.xs[g] | lowmask) == K + 1) { K++; break; }
+    }
+    p.K = K;
     // masks that no tile holds go to the streaming kernel
     size_t nleft = 0;
     for (size_t g = 0; g < nx; g++) {

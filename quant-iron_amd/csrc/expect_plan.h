@@ -89,8 +89,8 @@ struct ExpPlan {
 size_t exp_plan_bytes(size_t nt);
 // Carves the arrays out of `arena` (exp_plan_bytes(nt) bytes, 16-byte aligned).
 void exp_plan_carve(ExpPlan &p, void *arena, size_t nt);
-// Tile width for n qubits (n >= 4): the whole state up to kExpMaxK - 1 = 12
-// qubits, else 13 (complex64) or 12 (complex128) of them.
+// Widest tile for n qubits (n >= 4): the whole state, at most 13 (complex64) or
+// 12 (complex128) qubits of it.
 int exp_tile_qubits(uint32_t n, bool c128);
 // Qubits 0 .. low-1 are always in a tile: 128-byte runs in memory.
 inline int exp_low_qubits(bool c128) { return c128 ? 3 : 4; }
