@@ -554,6 +554,7 @@ struct Batch {
     std::vector<uint32_t> level_blocks;
     std::vector<std::pair<size_t, size_t>> wlevels;  // the same for one-wave passes
     std::vector<uint32_t> wlevel_blocks;
+    std::vector<char> wsparse;                       // the level has tasks whose state is still partly known to be zero
     std::vector<std::pair<size_t, size_t>> elevels;
     std::vector<uint32_t> elevel_blocks;
     size_t nsmall = 0, nfold = 0;
@@ -858,6 +859,7 @@ Status batch_plan(Batch &B) {
     std::vector<std::vector<WaveTask>> per_wlevel;
     std::vector<FoldTask> folds;
     B.eterms.clear();
+    B.wsparse.clear();
     uint64_t arena_elems = 0;
     uint32_t nparts = 0;
     for (size_t ci = 0; ci < B.circs.size(); ci++) {
@@ -880,12 +882,19 @@ Status batch_plan(Batch &B) {
         arena_elems += uint64_t(1) << P.n;
         const uint32_t tiles = uint32_t(1) << (P.n - B.K);
         if (on_waves(P)) {
+            const uint64_t all = (uint64_t(1) << P.n) - 1;
+            uint64_t known = 0;
             for (size_t p = 0; p < P.wpasses.size(); p++) {
                 WaveTask wt{};
                 wt.off = off; wt.pass = P.wpass_base + (uint32_t)p; wt.slot_base = C.slot_base;
-                wt.block0 = uint32_t(1) << (P.n - kw);  // tile count; turned into offsets per level below
-                if (per_wlevel.size() <= p) per_wlevel.resize(p + 1);
+                wt.known = known;
+                wt.last = p + 1 == P.wpasses.size();
+                // tile count (a first pass has one that is not zero); turned into offsets per level below
+                wt.block0 = p == 0 && !wt.last ? 1u : uint32_t(1) << (P.n - kw);
+                if (per_wlevel.size() <= p) { per_wlevel.resize(p + 1); B.wsparse.resize(p + 1); }
+                if (known != all) B.wsparse[p] = 1;
                 per_wlevel[p].push_back(wt);
+                known |= P.wpasses[p].qmask;
             }
         }
         size_t level = 0;
@@ -1011,7 +1020,7 @@ template <typename R, int K> static Status launch_levels(Batch &B, hipStream_t s
         }
         if (l < B.wlevels.size()) {
             auto r = B.wlevels[l];
-            Status e = launch_batch_wave(B.prec, l == 0, B.wlevel_blocks[l], st, B.d_arena.p, wt + r.first,
+            Status e = launch_batch_wave(B.prec, B.wsparse[l] != 0, B.wlevel_blocks[l], st, B.d_arena.p, wt + r.first,
                                          (int)(r.second - r.first), (const RegPass *)B.d_wpasses.p,
                                          (const RegOp *)B.d_wops.p, B.d_ptab.p);
             if (!e.ok()) return e;

@@ -185,11 +185,11 @@ struct WaveTask {
     uint32_t block0;    // first workgroup of this task in the launch
     uint32_t pass;      // index of its RegPass in the pass table
     int32_t slot_base;  // first angle slot of the circuit (RegOp::param counts from it)
-    uint32_t pad;
+    uint32_t last;      // the circuit's last pass: tiles outside `known` are written as zeros
+    uint64_t known;     // qubits the earlier passes' tiles spanned: amplitudes with another bit set are zero (0: |0..0>)
 };
-// init: the launch holds the first pass of each of its circuits (the state is
-// |0..0>, the pass loads nothing).
-Status launch_batch_wave(int prec, bool init, uint32_t blocks, hipStream_t st, void *arena, const WaveTask *tasks,
+// sparse: some task's `known` is not all of its circuit's qubits.
+Status launch_batch_wave(int prec, bool sparse, uint32_t blocks, hipStream_t st, void *arena, const WaveTask *tasks,
                          int ntasks, const RegPass *passes, const RegOp *ops, const void *ptab);
 
 Status plan_fused(const State &s, const std::vector<Lowered> &gates, int kb, ExecPlan &plan);
