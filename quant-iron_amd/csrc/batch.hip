@@ -417,24 +417,14 @@ struct BigTask {
     uint8_t pos[48];
 };
 
-__device__ __forceinline__ int find_task(const BigTask *__restrict__ tasks, int ntasks, uint32_t b) {
-    int lo = 0, hi = ntasks - 1;
-    while (lo < hi) {
-        int mid = (lo + hi + 1) >> 1;
-        if (tasks[mid].block0 <= b) lo = mid; else hi = mid - 1;
-    }
-    return lo;
-}
-
 template <typename R, int K>
 __global__ __launch_bounds__(kPT) void k_batch_pass(typename V2<R>::T *__restrict__ arena, const BigTask *__restrict__ tasks,
-                                                    int ntasks, const TileOp *__restrict__ ops,
+                                                    const uint32_t *__restrict__ index, const TileOp *__restrict__ ops,
                                                     const double *__restrict__ coef) {
     using T = typename V2<R>::T;
     constexpr int N = 1 << K, PER = N / kPT;
     __shared__ T tile[N];
-    const int ti = find_task(tasks, ntasks, blockIdx.x);
-    const BigTask &tk = tasks[ti];
+    const BigTask &tk = tasks[find_task(tasks, index, blockIdx.x)];
     const uint64_t base = insert_zeros64(uint64_t(blockIdx.x - tk.block0), tk.qmask);
     T *psi = arena + tk.off;
     const uint64_t off_t = deposit_pos<kPTLog>(threadIdx.x, tk.pos, kPTLog);
@@ -466,14 +456,13 @@ __global__ __launch_bounds__(kPT) void k_batch_pass(typename V2<R>::T *__restric
 
 template <typename R, int K>
 __global__ __launch_bounds__(kBT) void k_batch_expect(const typename V2<R>::T *__restrict__ arena,
-                                                      const BigTask *__restrict__ tasks, int ntasks,
+                                                      const BigTask *__restrict__ tasks, const uint32_t *__restrict__ index,
                                                       const ETerm *__restrict__ terms, double *__restrict__ part) {
     using T = typename V2<R>::T;
     constexpr int N = 1 << K, PER = N / kBT;
     __shared__ T tile[N];
     __shared__ double sh[4 * 4];
-    const int ti = find_task(tasks, ntasks, blockIdx.x);
-    const BigTask &tk = tasks[ti];
+    const BigTask &tk = tasks[find_task(tasks, index, blockIdx.x)];
     const uint32_t local = blockIdx.x - tk.block0;
     const uint64_t base = insert_zeros64(uint64_t(local), tk.qmask);
     const T *psi = arena + tk.off;
@@ -549,14 +538,15 @@ struct Batch {
     // device
     DevBuf d_ops, d_terms, d_small, d_big, d_fold, d_angles, d_coef, d_part, d_energy, d_arena;
     DevBuf d_wops, d_wpasses, d_wtasks, d_ptab;     // one-wave passes: ops, passes, tasks, slot coefficients
+    DevBuf d_index;                                 // every launch's task index
     int exec = QI_BATCH_WAVE;
-    std::vector<std::pair<size_t, size_t>> levels;  // [task begin, task end) of each pass level
-    std::vector<uint32_t> level_blocks;
-    std::vector<std::pair<size_t, size_t>> wlevels;  // the same for one-wave passes
-    std::vector<uint32_t> wlevel_blocks;
+    // a launch: its first task, its blocks, its first entry of the task index
+    struct Level {
+        size_t task0, index0;
+        uint32_t blocks;
+    };
+    std::vector<Level> levels, wlevels, elevels;     // LDS passes, one-wave passes, expectation passes
     std::vector<char> wsparse;                       // the level has tasks whose state is still partly known to be zero
-    std::vector<std::pair<size_t, size_t>> elevels;
-    std::vector<uint32_t> elevel_blocks;
     size_t nsmall = 0, nfold = 0;
     int K = 0, KS = 0;        // tile width of tiled circuits, largest LDS-resident circuit (0: defaults)
     std::unordered_multimap<uint64_t, uint32_t> prog_index;  // shape hash -> program
@@ -567,7 +557,7 @@ struct Batch {
     double last_ms = 0.0;
     ~Batch() {
         for (DevBuf *b : {&d_ops, &d_terms, &d_small, &d_big, &d_fold, &d_angles, &d_coef, &d_part, &d_energy, &d_arena,
-                          &d_wops, &d_wpasses, &d_wtasks, &d_ptab})
+                          &d_wops, &d_wpasses, &d_wtasks, &d_ptab, &d_index})
             if (b->p) (void)hipFree(b->p);
         if (graph) (void)hipGraphExecDestroy(graph);
         if (side) (void)hipStreamDestroy(side);
@@ -955,28 +945,28 @@ Status batch_plan(Batch &B) {
     }
     // flatten levels: block0 becomes the running block offset inside the level
     std::vector<BigTask> big;
-    B.levels.clear(); B.level_blocks.clear(); B.elevels.clear(); B.elevel_blocks.clear();
-    auto flatten = [&](std::vector<std::vector<BigTask>> &lv, std::vector<std::pair<size_t, size_t>> &rng,
-                       std::vector<uint32_t> &blocks) {
+    std::vector<WaveTask> wtasks;
+    std::vector<uint32_t> index;
+    const auto flatten = [&](auto &lv, auto &tasks, std::vector<Batch::Level> &out) {
+        out.clear();
         for (auto &v : lv) {
-            size_t b0 = big.size();
-            uint32_t acc = 0;
-            for (auto &t : v) { uint32_t tiles = t.block0; t.block0 = acc; acc += tiles; big.push_back(t); }
-            rng.push_back({b0, big.size()});
-            blocks.push_back(acc);
+            Batch::Level L{tasks.size(), index.size(), 0};
+            for (size_t k = 0; k < v.size(); k++) {
+                auto t = v[k];
+                const uint32_t tiles = t.block0, end = L.blocks + tiles;
+                t.block0 = L.blocks;
+                // index entries whose first block is one of this task's
+                for (uint64_t g = index.size() - L.index0; (g << kTaskIndexLog2) < end; g++) index.push_back((uint32_t)k);
+                L.blocks = end;
+                tasks.push_back(t);
+            }
+            index.push_back(v.empty() ? 0u : (uint32_t)v.size() - 1);
+            out.push_back(L);
         }
     };
-    flatten(per_level, B.levels, B.level_blocks);
-    flatten(per_elevel, B.elevels, B.elevel_blocks);
-    std::vector<WaveTask> wtasks;
-    B.wlevels.clear(); B.wlevel_blocks.clear();
-    for (auto &v : per_wlevel) {
-        const size_t b0 = wtasks.size();
-        uint32_t acc = 0;
-        for (auto &t : v) { const uint32_t tiles = t.block0; t.block0 = acc; acc += tiles; wtasks.push_back(t); }
-        B.wlevels.push_back({b0, wtasks.size()});
-        B.wlevel_blocks.push_back(acc);
-    }
+    flatten(per_level, big, B.levels);
+    flatten(per_elevel, big, B.elevels);
+    flatten(per_wlevel, wtasks, B.wlevels);
     B.nsmall = small.size();
     B.nfold = folds.size();
     Status e;
@@ -990,6 +980,7 @@ Status batch_plan(Batch &B) {
     if (!(e = upload_vec(B.d_wops, wops)).ok()) return e;
     if (!(e = upload_vec(B.d_wpasses, wpasses)).ok()) return e;
     if (!(e = upload_vec(B.d_wtasks, wtasks)).ok()) return e;
+    if (!(e = upload_vec(B.d_index, index)).ok()) return e;
     if (!(e = ensure(B.d_ptab, std::max<size_t>(B.angles.size(), 1) * kParamRow * (c128 ? 8 : 4))).ok()) return e;
     if (!(e = ensure(B.d_part, std::max<size_t>(nparts, 1) * 4 * sizeof(double))).ok()) return e;
     if (!(e = ensure(B.d_energy, std::max<size_t>(B.circs.size(), 1) * 2 * sizeof(double))).ok()) return e;
@@ -1011,26 +1002,23 @@ template <typename R, int K> static Status launch_levels(Batch &B, hipStream_t s
     using T = typename V2<R>::T;
     const BigTask *big = (const BigTask *)B.d_big.p;
     const WaveTask *wt = (const WaveTask *)B.d_wtasks.p;
+    const uint32_t *index = (const uint32_t *)B.d_index.p;
     for (size_t l = 0; l < std::max(B.levels.size(), B.wlevels.size()); l++) {
         if (l < B.levels.size()) {
-            auto r = B.levels[l];
-            hipLaunchKernelGGL((k_batch_pass<R, K>), dim3(B.level_blocks[l]), dim3(kPT), 0, st, (T *)B.d_arena.p,
-                               big + r.first, (int)(r.second - r.first), (const TileOp *)B.d_ops.p,
-                               (const double *)B.d_coef.p);
+            const Batch::Level &L = B.levels[l];
+            hipLaunchKernelGGL((k_batch_pass<R, K>), dim3(L.blocks), dim3(kPT), 0, st, (T *)B.d_arena.p, big + L.task0,
+                               index + L.index0, (const TileOp *)B.d_ops.p, (const double *)B.d_coef.p);
         }
         if (l < B.wlevels.size()) {
-            auto r = B.wlevels[l];
-            Status e = launch_batch_wave(B.prec, B.wsparse[l] != 0, B.wlevel_blocks[l], st, B.d_arena.p, wt + r.first,
-                                         (int)(r.second - r.first), (const RegPass *)B.d_wpasses.p,
-                                         (const RegOp *)B.d_wops.p, B.d_ptab.p);
+            const Batch::Level &L = B.wlevels[l];
+            Status e = launch_batch_wave(B.prec, B.wsparse[l] != 0, L.blocks, st, B.d_arena.p, wt + L.task0, index + L.index0,
+                                         (const RegPass *)B.d_wpasses.p, (const RegOp *)B.d_wops.p, B.d_ptab.p);
             if (!e.ok()) return e;
         }
     }
-    for (size_t l = 0; l < B.elevels.size(); l++) {
-        auto r = B.elevels[l];
-        hipLaunchKernelGGL((k_batch_expect<R, K>), dim3(B.elevel_blocks[l]), dim3(kBT), 0, st, (const T *)B.d_arena.p,
-                           big + r.first, (int)(r.second - r.first), (const ETerm *)B.d_terms.p, (double *)B.d_part.p);
-    }
+    for (const Batch::Level &L : B.elevels)
+        hipLaunchKernelGGL((k_batch_expect<R, K>), dim3(L.blocks), dim3(kBT), 0, st, (const T *)B.d_arena.p, big + L.task0,
+                           index + L.index0, (const ETerm *)B.d_terms.p, (double *)B.d_part.p);
     if (B.nfold)
         hipLaunchKernelGGL(k_batch_fold, dim3((unsigned)B.nfold), dim3(256), 0, st, (const FoldTask *)B.d_fold.p,
                            (const double *)B.d_part.p, (double *)B.d_energy.p);

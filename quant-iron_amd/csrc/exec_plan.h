@@ -188,9 +188,25 @@ struct WaveTask {
     uint32_t last;      // the circuit's last pass: tiles outside `known` are written as zeros
     uint64_t known;     // qubits the earlier passes' tiles spanned: amplitudes with another bit set are zero (0: |0..0>)
 };
+// Blocks per entry of a launch's task index: entry g is the task of block
+// g << kTaskIndexLog2, the last one the launch's last task.
+constexpr int kTaskIndexLog2 = 6;
+// The task that covers block b, tasks ascending in block0: between two entries
+// of the index (for a large circuit one and the same task), by bisection. (A
+// bisection over all tasks is a chain of eight loads per wave at 256 tasks:
+// batches of 200-256 circuits 1.0-1.7% slower.)
+template <typename Task>
+__host__ __device__ inline uint32_t find_task(const Task *tasks, const uint32_t *index, uint32_t b) {
+    uint32_t lo = index[b >> kTaskIndexLog2], hi = index[(b >> kTaskIndexLog2) + 1];
+    while (lo < hi) {
+        const uint32_t mid = (lo + hi + 1) >> 1;
+        if (tasks[mid].block0 <= b) lo = mid; else hi = mid - 1;
+    }
+    return lo;
+}
 // sparse: some task's `known` is not all of its circuit's qubits.
 Status launch_batch_wave(int prec, bool sparse, uint32_t blocks, hipStream_t st, void *arena, const WaveTask *tasks,
-                         int ntasks, const RegPass *passes, const RegOp *ops, const void *ptab);
+                         const uint32_t *index, const RegPass *passes, const RegOp *ops, const void *ptab);
 
 Status plan_fused(const State &s, const std::vector<Lowered> &gates, int kb, ExecPlan &plan);
 Status launch_fused_block(State &s, const FusedBlock &b, const void *dmat, hipStream_t st);

@@ -1242,15 +1242,6 @@ template <typename R> __device__ __forceinline__ void param_coeffs(RegOp &op, co
     }
 }
 
-__device__ __forceinline__ int find_wave_task(const WaveTask *__restrict__ tasks, int ntasks, uint32_t b) {
-    int lo = 0, hi = ntasks - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (tasks[mid].block0 <= b) lo = mid; else hi = mid - 1;
-    }
-    return lo;
-}
-
 // Pass p of many circuits in one launch (the batched energies): workgroup b
 // is one wave holding one tile of the circuit whose task covers b (tasks in
 // block order); the task names the circuit's state in the arena, its pass
@@ -1265,12 +1256,12 @@ __device__ __forceinline__ int find_wave_task(const WaveTask *__restrict__ tasks
 // circuits of 10-22 qubits, complex64: first level 0.94 ms -> 0.09.
 template <typename R, int K, bool SPARSE>
 __global__ __launch_bounds__(64) void k_batch_wave(typename V2<R>::T *__restrict__ arena, const WaveTask *__restrict__ tasks,
-                                                   int ntasks, const RegPass *__restrict__ passes,
+                                                   const uint32_t *__restrict__ index, const RegPass *__restrict__ passes,
                                                    const RegOp *__restrict__ ops, const R *__restrict__ ptab) {
     using T = typename V2<R>::T;
     constexpr int TB = kLaneBits, RB = K - TB, E = 1 << RB;
     const uint32_t lane = threadIdx.x;
-    const WaveTask &tk = tasks[find_wave_task(tasks, ntasks, blockIdx.x)];
+    const WaveTask &tk = tasks[find_task(tasks, index, blockIdx.x)];
     const RegPass &pass = passes[tk.pass];
     const uint64_t base = insert_zeros64(blockIdx.x - tk.block0, pass.qmask);
     T *psi = arena + tk.off;
@@ -1398,22 +1389,22 @@ Status launch_reg_pass(State &s, const RegPass &p, const RegOp *dops, hipStream_
 }
 
 Status launch_batch_wave(int prec, bool sparse, uint32_t blocks, hipStream_t st, void *arena, const WaveTask *tasks,
-                         int ntasks, const RegPass *passes, const RegOp *ops, const void *ptab) {
-    if (!blocks || ntasks <= 0) return Status{};
+                         const uint32_t *index, const RegPass *passes, const RegOp *ops, const void *ptab) {
+    if (!blocks) return Status{};
     const dim3 g(blocks), b(64);
     if (prec == QI_C128) {
         if (sparse)
-            hipLaunchKernelGGL((k_batch_wave<double, kBatchWaveK128, true>), g, b, 0, st, (double2 *)arena, tasks, ntasks,
+            hipLaunchKernelGGL((k_batch_wave<double, kBatchWaveK128, true>), g, b, 0, st, (double2 *)arena, tasks, index,
                                passes, ops, (const double *)ptab);
         else
-            hipLaunchKernelGGL((k_batch_wave<double, kBatchWaveK128, false>), g, b, 0, st, (double2 *)arena, tasks, ntasks,
+            hipLaunchKernelGGL((k_batch_wave<double, kBatchWaveK128, false>), g, b, 0, st, (double2 *)arena, tasks, index,
                                passes, ops, (const double *)ptab);
     } else {
         if (sparse)
-            hipLaunchKernelGGL((k_batch_wave<float, kBatchWaveK64, true>), g, b, 0, st, (float2 *)arena, tasks, ntasks,
+            hipLaunchKernelGGL((k_batch_wave<float, kBatchWaveK64, true>), g, b, 0, st, (float2 *)arena, tasks, index,
                                passes, ops, (const float *)ptab);
         else
-            hipLaunchKernelGGL((k_batch_wave<float, kBatchWaveK64, false>), g, b, 0, st, (float2 *)arena, tasks, ntasks,
+            hipLaunchKernelGGL((k_batch_wave<float, kBatchWaveK64, false>), g, b, 0, st, (float2 *)arena, tasks, index,
                                passes, ops, (const float *)ptab);
     }
     QI_HIP_TRY(hipGetLastError());
