@@ -41,3 +41,20 @@ def test_states_grow_from_zero_pass_by_pass(ctx, prec):
             for e, ref, (n, g, t) in zip(b.run(), refs[::order], circuits[::order]):
                 # each gate: four products and sums per component, in bra and ket
                 assert abs(e - ref) <= np.sum(np.abs(t["c_re"])) * (8 * g.size * eps + 1e-13), n
+
+
+@pytest.mark.parametrize("prec", ["c64", "c128"])
+def test_a_term_that_only_the_widest_tile_holds(ctx, prec):
+    """One term of one circuit spans the widest expectation tile (13 / 12 qubits
+    with the low ones): the whole batch takes that width, else one less."""
+    rng = np.random.default_rng(8)
+    n, low, wide = 15, 4 if prec == "c64" else 3, 13 if prec == "c64" else 12
+    span = ((1 << (wide - low)) - 1) << low
+    gates = gates_array(gates_on(list(range(n)), 60, rng))
+    psi = O.apply_gates(O.init(n, 0), gates)
+    eps = 2.0 ** -24 if prec == "c64" else 2.0 ** -53
+    for masks in ([span, 3, 0], [span >> 1 & ~((1 << low) - 1), 3, 0]):
+        terms = term_array([(x, int(rng.integers(1 << n)), float(rng.normal()), 0.0) for x in masks])
+        b = qiron.CircuitBatch(prec)
+        b.add(n, gates, terms)
+        assert abs(b.run()[0] - O.expectation(psi, terms)) <= np.sum(np.abs(terms["c_re"])) * (8 * 60 * eps + 1e-13)
