@@ -16,6 +16,8 @@
 // Unitary2 :2253-2254, Matchgate :1000-1006) and this file is compiled
 // without FMA contraction, so a complex128 state gets the reference's results
 // bit for bit (up to the sign of zero). All constants are computed on the host.
+#include <cstddef>
+
 #include "qi_internal.h"
 
 #pragma clang fp contract(off)
@@ -511,12 +513,23 @@ Status launch_c128(State &s, const Lowered &L, hipStream_t st) {
 // gate updates the LDS copy with the streaming kernels' formulas (the same
 // results bit for bit), the state is written once. A gate is an LDS round trip
 // and a barrier (0.5 us) instead of a launch; the ops are staged in LDS in
-// blocks. Bound by the latency of that chain. 10 qubits, complex128, 68 gates:
-// 31 us in one launch, 180 us in 68.
+// blocks. Bound by the latency of that chain; reading an op's 96 bytes in every
+// lane took as much LDS time as the amplitudes, so a wave reads its index sets
+// as one word per lane and only the coefficients that its kind uses. 10 qubits,
+// complex128, 68 gates: 31 us in one launch (35 with whole ops), 180 us in 68;
+// calls on 8 and 11 qubits 50.4 -> 46.4 and 84.2 -> 78.2 us.
 constexpr int kSmallStage = 64;  // ops staged at a time
+// The coefficients a kind uses, read from the staged op where they are used.
+template <typename R> __device__ __forceinline__ GateK<R> small_coeffs(const SmallOp &op) {
+    GateK<R> g;
+#pragma unroll
+    for (int q = 0; q < 8; q++) g.c[q] = R(op.c[q]);
+    return g;
+}
 template <typename R, int KIND, typename T>
 __device__ __forceinline__ void small_pairs(T *tile, uint32_t items, uint32_t fixed, uint32_t set, uint32_t pmask,
-                                            const GateK<R> &g) {
+                                            const SmallOp &op) {
+    const GateK<R> g = small_coeffs<R>(op);
     for (uint32_t k = threadIdx.x; k < items; k += blockDim.x) {
         uint32_t i = k;
         for (uint32_t f = fixed; f; f &= f - 1) {
@@ -532,7 +545,8 @@ __device__ __forceinline__ void small_pairs(T *tile, uint32_t items, uint32_t fi
     }
 }
 template <typename R, int KIND, typename T>
-__device__ __forceinline__ void small_diag(T *tile, uint32_t items, uint32_t fixed, uint32_t set, const GateK<R> &g) {
+__device__ __forceinline__ void small_diag(T *tile, uint32_t items, uint32_t fixed, uint32_t set, const SmallOp &op) {
+    const GateK<R> g = small_coeffs<R>(op);
     for (uint32_t k = threadIdx.x; k < items; k += blockDim.x) {
         uint32_t i = k;
         for (uint32_t f = fixed; f; f &= f - 1) {
@@ -557,23 +571,25 @@ __global__ __launch_bounds__(512) void k_small_gates(typename V2<R>::T *__restri
         for (int w = threadIdx.x; w < cnt * W; w += blockDim.x)
             reinterpret_cast<f32x4 *>(sops)[w] = reinterpret_cast<const f32x4 *>(ops + o0)[w];
         __syncthreads();
-        SmallOp nxt = sops[0];
+        // an op's index sets, a word per lane, read while the op before runs
+        static_assert(offsetof(SmallOp, c) == 32, "eight words before the coefficients");
+        const auto sets = [&](int o) { return reinterpret_cast<const uint32_t *>(sops + o)[threadIdx.x & 7]; };
+        uint32_t nxt = sets(0);
         for (int o = 0; o < cnt; o++) {
-            const SmallOp op = nxt;
-            nxt = sops[o + 1 < cnt ? o + 1 : o];  // read while this op runs
-            auto u = [](uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); };
-            const uint32_t items = u(op.items), fixed = u(op.fixed), set = u(op.set), pmask = u(op.pmask);
-            GateK<R> g;
-#pragma unroll
-            for (int q = 0; q < 8; q++) g.c[q] = R(op.c[q]);
-            switch ((int)u((uint32_t)op.kind)) {
-#define QI_SMALL(K) case K: small_pairs<R, K>(tile, items, fixed, set, pmask, g); break;
+            const uint32_t cur = nxt;
+            const SmallOp &op = sops[o];
+            nxt = sets(o + 1 < cnt ? o + 1 : o);
+            const auto u = [&](int k) { return (uint32_t)__builtin_amdgcn_readlane((int)cur, k); };
+            const uint32_t items = u(1), fixed = u(2), set = u(3), pmask = u(4);
+            switch ((int)u(0)) {
+#define QI_SMALL(K) case K: small_pairs<R, K>(tile, items, fixed, set, pmask, op); break;
                 QI_SMALL(LK_H) QI_SMALL(LK_X) QI_SMALL(LK_Y) QI_SMALL(LK_RX) QI_SMALL(LK_RY) QI_SMALL(LK_U2) QI_SMALL(LK_RZ)
 #undef QI_SMALL
-            case LK_Z: small_diag<R, LK_Z>(tile, items, fixed, set, g); break;
-            case LK_PHASE: small_diag<R, LK_PHASE>(tile, items, fixed, set, g); break;
+            case LK_Z: small_diag<R, LK_Z>(tile, items, fixed, set, op); break;
+            case LK_PHASE: small_diag<R, LK_PHASE>(tile, items, fixed, set, op); break;
             default: {  // LK_MATCH, as k_match
-                const uint32_t tb = u(op.tb), tb2 = u(op.tb2), cmask = u(op.cmask);
+                const uint32_t tb = u(5), tb2 = u(6), cmask = u(7);
+                const GateK<R> g = small_coeffs<R>(op);
                 for (uint32_t k = threadIdx.x; k < items; k += blockDim.x) {
                     uint32_t l = k;
                     for (uint32_t f = fixed; f; f &= f - 1) {
