@@ -5,14 +5,15 @@
 // registers. A layout assigns the K local index bits to TB thread bits (6
 // lane bits, TB-6 wave bits) and K-TB register bits. A 2x2 gate acts on a
 // target held in registers (the pair lives in one thread) or on lanes (each
-// lane fetches its partner with ds_bpermute, the LDS crossbar without LDS
-// memory, and computes its half of the pair). Controls and diagonal targets
+// lane fetches its partner, by a DPP move across lane bits 0-3 or with
+// ds_bpermute, the LDS crossbar without LDS memory, and computes its half of
+// the pair). Controls and diagonal targets
 // on register bits are compile-time facts of each register; on thread bits
 // they are a per-lane mask. With wave bits (TB = 8, 9), a target on a wave bit
 // takes a transpose of the tile through LDS, and controlled SWAPs and
 // Matchgates run on the LDS copy. A one-wave tile (TB = 6: complex64, up to
 // 4096 amplitudes, 64 per lane) has no wave bits: no LDS and no barriers;
-// its only layout changes are lane/register exchanges at the end of a pass.
+// its only layout changes are exchanges between lane and register bits.
 //
 // Arithmetic: both precisions use fused multiply-adds in the register ops
 // (complex128 tiles agree with the reference's unfused products to about
@@ -90,8 +91,6 @@ template <int F> __device__ __forceinline__ uint32_t swz(uint32_t e) {
     if constexpr (F == 4) return e ^ (((e >> 4) ^ (e >> 8) ^ (e >> 12)) & 15u);
     else return e ^ (((e >> 3) ^ (e >> 6) ^ (e >> 9) ^ (e >> 12)) & 7u);
 }
-
-template <typename T> __device__ __forceinline__ T sel(bool on, T x, T y) { return mk<T>(on ? x.x : y.x, on ? x.y : y.y); }
 
 // The amplitude of lane `addr / 4` (ds_bpermute: the LDS crossbar, no LDS memory).
 __device__ __forceinline__ float xlane(int addr, float x) {
@@ -244,7 +243,6 @@ __device__ __forceinline__ void ip_xor3(float &d, float x, float m) {  // d = x 
     asm("v_xor_b32 %0, %1, %2" : "+v"(d) : "v"(__float_as_uint(m)), "v"(x));
 }
 __device__ __forceinline__ float xor_bits(float x, float m) { return __uint_as_float(__float_as_uint(x) ^ __float_as_uint(m)); }
-__device__ __forceinline__ float xor_sign(float x, uint32_t m) { return __uint_as_float(__float_as_uint(x) ^ m); }
 __device__ __forceinline__ float fma_r(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 
 // The same in-place updates for complex128 tiles. FP64 arithmetic works on
@@ -296,9 +294,6 @@ __device__ __forceinline__ void ip_xor3(double &d, double x, double m) {  // d =
 }
 __device__ __forceinline__ double xor_bits(double x, double m) {
     return __longlong_as_double(__double_as_longlong(x) ^ __double_as_longlong(m));
-}
-__device__ __forceinline__ double xor_sign(double x, uint32_t m) {
-    return __longlong_as_double(__double_as_longlong(x) ^ (long long)((uint64_t)m << 32));
 }
 __device__ __forceinline__ double fma_r(double a, double b, double c) { return __builtin_fma(a, b, c); }
 // the sign-flip pattern of a component as a value of its own type
