@@ -365,24 +365,25 @@ __global__ __launch_bounds__(256) void k_head(const bf16 *__restrict__ H, const 
     }
 }
 
-// Column sums of X (rows x cols, FP32) over 256-row chunks: workgroup (64
-// columns, chunk).
-__device__ __forceinline__ void colsum_chunk(const float *__restrict__ X, int rows, int cols, float *__restrict__ part, float (*sh)[64]) {
-    const int c = blockIdx.x * 64 + (threadIdx.x & 63), g = threadIdx.x >> 6;
-    const int r0 = blockIdx.y * 256;
+// Column sums of X (rows x cols, FP32) over 256-row chunks: columns 64 bx ..,
+// chunk by; by the workgroup's first 256 threads.
+__device__ __forceinline__ void colsum_chunk(const float *__restrict__ X, int rows, int cols, float *__restrict__ part, float (*sh)[64],
+                                             int bx, int by) {
+    const int c = bx * 64 + (threadIdx.x & 63), g = threadIdx.x >> 6;
+    const int r0 = by * 256;
     float s = 0.f;
     // (unrolled: the loads of eight rows are in flight together; the sum
     // keeps its row order)
-    if (c < cols)
+    if (c < cols && g < 4)
 #pragma unroll 8
         for (int r = r0 + g; r < r0 + 256 && r < rows; r += 4) s += X[size_t(r) * cols + c];
-    sh[g][threadIdx.x & 63] = s;
+    if (g < 4) sh[g][threadIdx.x & 63] = s;
     __syncthreads();
-    if (g == 0 && c < cols) part[size_t(blockIdx.y) * cols + c] = sh[0][threadIdx.x] + sh[1][threadIdx.x] + sh[2][threadIdx.x] + sh[3][threadIdx.x];
+    if (g == 0 && c < cols) part[size_t(by) * cols + c] = sh[0][threadIdx.x] + sh[1][threadIdx.x] + sh[2][threadIdx.x] + sh[3][threadIdx.x];
 }
 __global__ __launch_bounds__(256) void k_colsum_part(const float *__restrict__ X, int rows, int cols, float *__restrict__ part) {
     __shared__ float sh[4][64];
-    colsum_chunk(X, rows, cols, part, sh);
+    colsum_chunk(X, rows, cols, part, sh, blockIdx.x, blockIdx.y);
 }
 __global__ __launch_bounds__(256) void k_colsum_fold(const float *__restrict__ part, int chunks, int cols, float *__restrict__ out) {
     const int c = blockIdx.x * 256 + threadIdx.x;
@@ -405,22 +406,22 @@ __global__ __launch_bounds__(256) void k_head_fold(const float *__restrict__ par
 // Partial sums of dw[k] = sum_r H[r,k] dy[r] (head weights) over chunks of 256
 // rows, as k_colsum_part (folded by k_colsum_fold).
 __device__ __forceinline__ void head_grad_chunk(const bf16 *__restrict__ H, const float *__restrict__ dy, int rows, int hid,
-                                                float *__restrict__ part, float (*sh)[64]) {
-    const int c = blockIdx.x * 64 + (threadIdx.x & 63), g = threadIdx.x >> 6;
-    const int r0 = blockIdx.y * 256;
+                                                float *__restrict__ part, float (*sh)[64], int bx, int by) {
+    const int c = bx * 64 + (threadIdx.x & 63), g = threadIdx.x >> 6;
+    const int r0 = by * 256;
     float s = 0.f;
-    if (c < hid)
+    if (c < hid && g < 4)
 #pragma unroll 8
         for (int r = r0 + g; r < r0 + 256 && r < rows; r += 4) s += bf2f(H[size_t(r) * hid + c]) * dy[r];
-    sh[g][threadIdx.x & 63] = s;
+    if (g < 4) sh[g][threadIdx.x & 63] = s;
     __syncthreads();
     if (g == 0 && c < hid)
-        part[size_t(blockIdx.y) * hid + c] = sh[0][threadIdx.x] + sh[1][threadIdx.x] + sh[2][threadIdx.x] + sh[3][threadIdx.x];
+        part[size_t(by) * hid + c] = sh[0][threadIdx.x] + sh[1][threadIdx.x] + sh[2][threadIdx.x] + sh[3][threadIdx.x];
 }
 __global__ __launch_bounds__(256) void k_head_grad_part(const bf16 *__restrict__ H, const float *__restrict__ dy, int rows,
                                                         int hid, float *__restrict__ part) {
     __shared__ float sh[4][64];
-    head_grad_chunk(H, dy, rows, hid, part, sh);
+    head_grad_chunk(H, dy, rows, hid, part, sh, blockIdx.x, blockIdx.y);
 }
 
 // Adam on one FP32 master parameter; returns its new value.
@@ -532,8 +533,10 @@ __global__ __launch_bounds__(256) void k_gather_rows(const bf16 *__restrict__ X,
 // acc += sum of the loss partials of one batch (one workgroup, fixed order)
 __device__ __forceinline__ void loss_accum(const float *__restrict__ part, int n, double *__restrict__ acc, double *sh) {
     double s = 0.0;
-    for (int i = threadIdx.x; i < n; i += 256) s += part[i];
-    sh[threadIdx.x] = s;
+    if (threadIdx.x < 256) {
+        for (int i = threadIdx.x; i < n; i += 256) s += part[i];
+        sh[threadIdx.x] = s;
+    }
     __syncthreads();
     for (int w = 128; w >= 1; w >>= 1) {
         if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
@@ -549,14 +552,44 @@ __global__ __launch_bounds__(256) void k_loss_accum(const float *__restrict__ pa
 // ------------------------------------------------ small-batch training --
 // A training step on a batch whose layers have too few 128 x 128 tiles to fill
 // the chip is a chain of short dependent kernels (bounded by launches and load
-// round trips, not by bytes or operations), so it runs as nine launches (three
-// layers, head, two backward layers, the three weight gradients in one, all
-// column sums and the loss in one, Adam with every copy of the weights and the
-// next batch's rows in one) where the large-batch path takes 37. Each producer also writes the
-// transposed copy that a weight gradient reads. Every sum keeps the order of
-// the large-batch path's kernels (same K slices, slice order, row groups and
-// chunks): the same bits. Per step of 1024 rows at 195 -> 512 x 3 -> 1 the
-// large-batch kernels take 188 us, these 67.
+// round trips, not by bytes or operations), so it runs as eight launches (three
+// layers, head, two backward layers, the three weight gradients with all column
+// sums and the loss, Adam with every copy of the weights and the next batch's
+// rows; nine where the column sums take a launch of their own) where the
+// large-batch path takes 37. Each producer also writes the transposed copy that
+// a weight gradient reads. Every sum keeps the order of the large-batch path's
+// kernels (same K slices, slice order, row groups and chunks): the same bits. Per step of 1024 rows at 195 -> 512 x 3 -> 1 the
+// large-batch kernels take 188 us, these 66.
+
+// Chunk sums of the bias gradients (dZ of the three layers), the head's weight
+// and bias gradients, and the batch's loss: `which` 0-4, columns 64 blockIdx.x
+// .., chunks blockIdx.y, blockIdx.y + gridDim.y, ...; at least 256 threads.
+struct StepSums {
+    const float *dZ[3], *dy, *lossp;
+    const bf16 *H;
+    float *part[5];  // b1, b2, b3, w4, b4: chunks x width
+    double *lacc;    // null: no loss
+    int rows, hid, nloss;
+};
+__device__ __forceinline__ void step_sums(const StepSums &s, int which, unsigned char *lds) {
+    float(*const sh)[64] = reinterpret_cast<float(*)[64]>(lds);
+    const int bx = blockIdx.x;
+    if (which == 4 && bx == 1 && blockIdx.y == 0 && s.lacc) {
+        loss_accum(s.lossp, s.nloss, s.lacc, reinterpret_cast<double *>(lds));
+        return;
+    }
+    if (bx * 64 >= (which == 4 ? 1 : s.hid)) return;
+    for (int by = blockIdx.y; by * 256 < s.rows; by += gridDim.y) {
+        if (which < 3) colsum_chunk(s.dZ[which], s.rows, s.hid, s.part[which], sh, bx, by);
+        else if (which == 3) head_grad_chunk(s.H, s.dy, s.rows, s.hid, s.part[3], sh, bx, by);
+        else colsum_chunk(s.dy, s.rows, 1, s.part[4], sh, bx, by);
+        __syncthreads();
+    }
+}
+__global__ __launch_bounds__(256) void k_step_sums(StepSums s) {
+    __shared__ __attribute__((aligned(16))) unsigned char lds[256 * sizeof(double)];
+    step_sums(s, blockIdx.z, lds);
+}
 
 // C[M x N] = A[M x K] B[N x K]^T, both K-contiguous: one 32 x 32 tile per
 // workgroup, one wave per K slice of kper (blockDim / 64 slices), the slices
@@ -571,12 +604,18 @@ struct SmallGemm {
 };
 struct SmallGemms {
     SmallGemm g[3];
+    int count;      // problems; EPI_STORE launches may hold five more grid planes:
+    StepSums sums;  // the step's column sums, which need only what the products need
 };
 constexpr int kSlicesMax = kMaxSplits;
 template <int EPI> __global__ __launch_bounds__(64 * kSlicesMax) void k_small_gemm(SmallGemms gs) {
     extern __shared__ __attribute__((aligned(16))) unsigned char sg_lds[];
     float(*const red)[32][36] = reinterpret_cast<float(*)[32][36]>(sg_lds);  // a slice's tile, padded rows
     __shared__ __attribute__((aligned(16))) bf16 tr[32][40];
+    if (EPI == EPI_STORE && (int)blockIdx.z >= gs.count) {  // (256 threads at least, 18 KiB of LDS)
+        step_sums(gs.sums, blockIdx.z - gs.count, sg_lds);
+        return;
+    }
     const SmallGemm &g = gs.g[blockIdx.z];
     const int m0 = blockIdx.y * 32, n0 = blockIdx.x * 32;
     if (m0 >= g.M || n0 >= g.N) return;  // whole workgroups (several problems in one grid)
@@ -721,25 +760,6 @@ __device__ __forceinline__ void gather_rows8(const GatherRows &g, int block, bf1
 __global__ __launch_bounds__(256) void k_gather_rows8(GatherRows g) {
     extern __shared__ __attribute__((aligned(16))) unsigned char gr_lds[];
     gather_rows8(g, blockIdx.x, reinterpret_cast<bf16 *>(gr_lds));
-}
-
-// Chunk sums of the bias gradients (dZ of the three layers), the head's weight
-// and bias gradients, and the batch's loss: workgroup (64 columns, chunk, which).
-struct StepSums {
-    const float *dZ[3], *dy, *lossp;
-    const bf16 *H;
-    float *part[5];  // b1, b2, b3, w4, b4: chunks x width
-    double *lacc;    // null: no loss
-    int rows, hid, nloss;
-};
-__global__ __launch_bounds__(256) void k_step_sums(StepSums s) {
-    __shared__ float sh[4][64];
-    __shared__ double shd[256];
-    const int w = blockIdx.z;
-    if (w < 3) colsum_chunk(s.dZ[w], s.rows, s.hid, s.part[w], sh);
-    else if (w == 3) head_grad_chunk(s.H, s.dy, s.rows, s.hid, s.part[3], sh);
-    else if (blockIdx.x == 0) colsum_chunk(s.dy, s.rows, 1, s.part[4], sh);
-    else if (blockIdx.x == 1 && blockIdx.y == 0 && s.lacc) loss_accum(s.lossp, s.nloss, s.lacc, shd);
 }
 
 // The gradients folded from those chunks in order.
@@ -1359,7 +1379,7 @@ static int gradient_slices(int M, int Nn, int K, int &kper) {
 // Batches whose layers have fewer than kSplitBelowTiles 128 x 128 tiles (at
 // that line the large-batch path stops splitting K), up to widths where the
 // two meet: us per step, large-batch kernels -> these, at 195 inputs: width 512
-// batch 128 137 -> 46, 3072 226 -> 130; width 1024 batch 1024 233 -> 158; width
+// batch 128 137 -> 46, 3072 226 -> 131; width 1024 batch 1024 233 -> 158; width
 // 2048 batch 256 248 -> 198; 4000 inputs, width and batch 1024 291 -> 288.
 static bool small_step(const Mlp &N, size_t rows) {
     const size_t tiles = ((rows + TM - 1) / TM) * size_t((N.hid + TN - 1) / TN);
@@ -1385,10 +1405,11 @@ static Status small_alloc(Mlp &N, size_t rows) {
     N.tcap = rows;
     return Status{};
 }
-template <int EPI> static void small_gemm(hipStream_t st, const SmallGemms &gs, int count, int slices) {
+template <int EPI> static void small_gemm(hipStream_t st, SmallGemms &gs, int count, int slices, int planes = 0) {
     int mx = 0, nx = 0;
+    gs.count = count;
     for (int k = 0; k < count; k++) { mx = std::max(mx, gs.g[k].M); nx = std::max(nx, gs.g[k].N); }
-    hipLaunchKernelGGL(k_small_gemm<EPI>, dim3((unsigned)(nx / 32), (unsigned)((mx + 31) / 32), (unsigned)count), dim3(64 * slices),
+    hipLaunchKernelGGL(k_small_gemm<EPI>, dim3((unsigned)(nx / 32), (unsigned)((mx + 31) / 32), (unsigned)(count + planes)), dim3(64 * slices),
                        size_t(slices) * 32 * 36 * sizeof(float), st, gs);
 }
 static void small_forward(Mlp &N, hipStream_t st, int rows) {
@@ -1442,7 +1463,23 @@ static void small_backward(Mlp &N, hipStream_t st, int rows, double *lacc) {
         slices[l] = gradient_slices(g.M, H, rows, g.kper);
         g.Cf = N.g + N.off[2 * l];
     }
-    if (slices[0] == slices[1] && slices[1] == slices[2]) {
+    const VecParams v = vec_params(N, rows);
+    StepSums &s = gs.sums;
+    for (int l = 0; l < 3; l++) s.dZ[l] = N.dZf[l];
+    s.dy = N.dy; s.lossp = N.lossp; s.H = N.H[2]; s.lacc = lacc;
+    for (int k = 0; k < 5; k++) s.part[k] = const_cast<float *>(v.part[k]);
+    s.rows = rows; s.hid = H; s.nloss = (rows + 3) / 4;
+    const bool one_launch = slices[0] == slices[1] && slices[1] == slices[2];
+    // The sums in the same launch, where its workgroups have the 256 threads they
+    // need (4 slices) and enough grid rows for a chunk each, up to 2048 rows; us per
+    // step at 195 inputs, in a launch of their own -> here: width 512 batch 512 55.2
+    // -> 52.1, 1024 67.1 -> 65.5, 2048 96.6 both, 3072 130 -> 132; width 64 batch 4096
+    // (two grid rows) 60.2 -> 66.7.
+    if (one_launch && slices[0] >= 4 && rows <= 2048 && v.chunks <= (std::max(N.k_in, H) + 31) / 32) {
+        small_gemm<EPI_STORE>(st, gs, 3, slices[0], 5);
+        return;
+    }
+    if (one_launch) {
         small_gemm<EPI_STORE>(st, gs, 3, slices[0]);
     } else {
         for (int l = 0; l < 3; l++) {
@@ -1451,12 +1488,6 @@ static void small_backward(Mlp &N, hipStream_t st, int rows, double *lacc) {
             small_gemm<EPI_STORE>(st, one, 1, slices[l]);
         }
     }
-    const VecParams v = vec_params(N, rows);
-    StepSums s{};
-    for (int l = 0; l < 3; l++) s.dZ[l] = N.dZf[l];
-    s.dy = N.dy; s.lossp = N.lossp; s.H = N.H[2]; s.lacc = lacc;
-    for (int k = 0; k < 5; k++) s.part[k] = const_cast<float *>(v.part[k]);
-    s.rows = rows; s.hid = H; s.nloss = (rows + 3) / 4;
     // (x: 64-column blocks; the last z takes two single workgroups)
     hipLaunchKernelGGL(k_step_sums, dim3((unsigned)std::max(2, (H + 63) / 64), (unsigned)v.chunks, 5), dim3(256), 0, st, s);
 }
