@@ -2,8 +2,8 @@
 // owns: no allocation of its own (the no-allocation entry point plans with it).
 #include "expect_plan.h"
 
+#include <algorithm>
 #include <cstring>
-#include <unordered_map>
 
 namespace qi {
 
@@ -29,40 +29,89 @@ uint32_t reg_bits(uint32_t l, const ExpSet &s) {
 // while they fit; above kGreedyMax masks simply in list order (the search is
 // quadratic).
 constexpr size_t kGreedyMax = 256;
-uint64_t grow_tile(uint64_t q, const uint64_t *xs, size_t count, int K) {
+template <typename F> uint64_t grow_tile(uint64_t q, size_t count, int K, F mask) {
     for (bool grown = true; grown;) {
         grown = false;
         size_t best = SIZE_MAX;
         int least = 64;
         for (size_t g = 0; g < count; g++) {
-            const int add = popc(xs[g] & ~q);
+            const int add = popc(mask(g) & ~q);
             if (!add || popc(q) + add > K || add >= least) continue;
             best = g; least = add;
             if (count > kGreedyMax || add == 1) break;
         }
-        if (best != SIZE_MAX) { q |= xs[best]; grown = true; }
+        if (best != SIZE_MAX) { q |= mask(best); grown = true; }
     }
     return q;
 }
 
+// Finds the entry of a list by its key: a few by looking at each, more through
+// an open-addressing table, so that a list of any length is planned in linear
+// time (one x mask with 16384 Z supports took 0.4 s, its product 3 s).
+constexpr size_t kLookAtEach = 16;
+size_t exp_table_entries(size_t nt) {
+    size_t n = 1;
+    while (n < 4 * nt) n <<= 1;
+    return n;
+}
+uint64_t mix(uint64_t a, uint64_t b) {  // (multiply-xorshift, odd constants)
+    uint64_t h = a * 0x9E3779B97F4A7C15ull ^ (b + 1) * 0xC2B2AE3D27D4EB4Full;
+    h ^= h >> 32;
+    h *= 0xD6E8FEB86659FD93ull;
+    return h ^ (h >> 32);
+}
+struct Finder {
+    uint32_t *table;
+    size_t last = 0;  // table entries - 1 (0: no table)
+    // Entries of at most 2 `terms` keys; `table` holds exp_table_entries(terms).
+    Finder(uint32_t *table, size_t terms) : table(table) {
+        if (terms <= kLookAtEach) return;
+        last = exp_table_entries(terms) - 1;
+        std::fill(table, table + last + 1, UINT32_MAX);
+    }
+    // The entry of [first, end) that is(k) accepts; `end` if none, which the caller then adds.
+    template <typename F> size_t find(uint64_t hash, size_t first, size_t end, F is) {
+        if (!last) {
+            while (first < end && !is(first)) first++;
+            return first;
+        }
+        for (size_t at = hash & last;; at = (at + 1) & last) {
+            if (table[at] == UINT32_MAX) {
+                table[at] = (uint32_t)end;
+                return end;
+            }
+            if (is(table[at])) return table[at];
+        }
+    }
+};
+
 }  // namespace
 
-size_t exp_plan_bytes(size_t nt) {
-    return up16(nt * sizeof(ExpPass)) + up16(nt * sizeof(ExpSet)) + up16((4 * nt + 1) * sizeof(ExpUnit)) +
-           up16(nt * sizeof(ExpDiag)) + 2 * up16(nt * sizeof(uint64_t)) +
-           up16(2 * nt * sizeof(uint32_t));
+size_t exp_max_units(const qi_pauli_term *terms, size_t nt) {
+    size_t n = 0;
+    for (size_t k = 0; k < nt; k++)
+        if (terms[k].x_mask) n += (popc(terms[k].x_mask) > 4 ? 2 : 1) * (terms[k].c_im != 0.0 ? 2 : 1);
+    return n;
 }
 
-void exp_plan_carve(ExpPlan &p, void *arena, size_t nt) {
+size_t exp_plan_bytes(size_t nt, size_t units) {
+    return up16(nt * sizeof(ExpPass)) + up16(nt * sizeof(ExpSet)) + up16((units + 1) * sizeof(ExpUnit)) +
+           up16(nt * sizeof(ExpDiag)) + up16(nt * sizeof(uint64_t)) + 2 * up16(nt * sizeof(uint32_t)) +
+           up16(nt * sizeof(ExpMask)) + up16(exp_table_entries(nt) * sizeof(uint32_t));
+}
+
+void exp_plan_carve(ExpPlan &p, void *arena, size_t nt, size_t units) {
     unsigned char *a = (unsigned char *)arena;
     auto take = [&](size_t bytes) { void *r = a; a += up16(bytes); return r; };
     p.passes = (ExpPass *)take(nt * sizeof(ExpPass));
     p.sets = (ExpSet *)take(nt * sizeof(ExpSet));
-    p.units = (ExpUnit *)take((4 * nt + 1) * sizeof(ExpUnit));
+    p.units = (ExpUnit *)take((units + 1) * sizeof(ExpUnit));
     p.diags = (ExpDiag *)take(nt * sizeof(ExpDiag));
     p.far = (uint64_t *)take(nt * sizeof(uint64_t));
-    p.xs = (uint64_t *)take(nt * sizeof(uint64_t));
-    p.gid = (uint32_t *)take(2 * nt * sizeof(uint32_t));
+    p.far_head = (uint32_t *)take(nt * sizeof(uint32_t));
+    p.next = (uint32_t *)take(nt * sizeof(uint32_t));
+    p.masks = (ExpMask *)take(nt * sizeof(ExpMask));
+    p.table = (uint32_t *)take(exp_table_entries(nt) * sizeof(uint32_t));
 }
 
 int exp_tile_qubits(uint32_t n, bool c128) {
@@ -74,25 +123,30 @@ void plan_expect(uint32_t n, bool c128, const qi_pauli_term *terms, size_t nt, E
     const int low = exp_low_qubits(c128);
     p.npasses = p.nsets = p.nunits = p.ndiags = p.nfar = 0;
     p.complex_out = false;
-    // distinct nonzero x masks in order of appearance; next term of the same mask in gid[nt + k]
+    // distinct x masks in order of appearance (the zero mask apart, where there are tiles)
     size_t nx = 0;
-    uint32_t *const head = p.gid, *const next = p.gid + nt;  // head: first term of mask g
+    ExpMask *const m = p.masks;
     bool diag = false;
+    Finder by_mask(p.table, nt);
     for (size_t k = 0; k < nt; k++) {
+        const uint64_t x = terms[k].x_mask;
         p.complex_out = p.complex_out || terms[k].c_im != 0.0;
-        next[k] = UINT32_MAX;
-        if (!terms[k].x_mask) { diag = true; continue; }
-        size_t g = nx;
-        // (terms of one mask are often neighbours: look from the back)
-        while (g > 0 && p.xs[g - 1] != terms[k].x_mask) g--;
-        if (g == 0) {
-            p.xs[nx] = terms[k].x_mask;
-            head[nx++] = (uint32_t)k;
+        p.next[k] = UINT32_MAX;
+        if (!x && n >= 4) { diag = true; continue; }
+        const size_t g = by_mask.find(mix(x, 0), 0, nx, [&](size_t i) { return m[i].x == x; });
+        if (g == nx) {
+            m[nx++] = ExpMask{x, (uint32_t)k, (uint32_t)k, 1, 0};
         } else {
-            uint32_t t = head[g - 1];
-            while (next[t] != UINT32_MAX) t = next[t];
-            next[t] = (uint32_t)k;
+            p.next[m[g].tail] = (uint32_t)k;
+            m[g].tail = (uint32_t)k;
+            m[g].count++;
         }
+    }
+    const auto stream = [&](const ExpMask &x) { p.far[p.nfar] = x.x; p.far_head[p.nfar++] = x.head; };
+    p.K = 0;
+    if (n < 4) {
+        for (size_t g = 0; g < nx; g++) stream(m[g]);
+        return;
     }
     // A complex64 state of more qubits than its widest tile takes tiles of one
     // qubit less, unless a mask needs that one: at half the LDS, four
@@ -106,22 +160,21 @@ void plan_expect(uint32_t n, bool c128, const qi_pauli_term *terms, size_t nt, E
     if (!c128 && !whole) {
         K--;
         for (size_t g = 0; g < nx; g++)
-            if (popc(p.xs[g] | lowmask) == K + 1) { K++; break; }
+            if (popc(m[g].x | lowmask) == K + 1) { K++; break; }
     }
     p.K = K;
     // masks that no tile holds go to the streaming kernel
     size_t nleft = 0;
     for (size_t g = 0; g < nx; g++) {
-        if (popc(p.xs[g] | lowmask) > K) { p.far[p.nfar++] = p.xs[g]; continue; }
-        p.xs[nleft] = p.xs[g];
-        head[nleft++] = head[g];
+        if (popc(m[g].x | lowmask) > K) stream(m[g]);
+        else m[nleft++] = m[g];
     }
     bool diag_todo = diag;
     size_t at = 0;  // masks [at, nleft) are unplanned; a pass moves its masks to the front
     while (at < nleft || diag_todo) {
         ExpPass &ps = p.passes[p.npasses++];
         memset(&ps, 0, sizeof ps);
-        uint64_t q = grow_tile(lowmask, p.xs + at, nleft - at, K);
+        uint64_t q = grow_tile(lowmask, nleft - at, K, [&](size_t g) { return m[at + g].x; });
         for (uint32_t b = 0; b < n && popc(q) < K; b++) q |= uint64_t(1) << b;
         ps.qmask = q;
         for (int k = 0, b = 0; k < K; b++)
@@ -129,9 +182,9 @@ void plan_expect(uint32_t n, bool c128, const qi_pauli_term *terms, size_t nt, E
         ps.s0 = (uint32_t)p.nsets;
         const size_t first = at;
         for (size_t g = at; g < nleft; g++)
-            if (!(p.xs[g] & ~q)) {
-                const uint64_t x = p.xs[g]; p.xs[g] = p.xs[at]; p.xs[at] = x;
-                const uint32_t h = head[g]; head[g] = head[at]; head[at] = h;
+            if (!(m[g].x & ~q)) {
+                std::swap(m[g], m[at]);
+                m[at].xl = local_bits(m[at].x, ps, K);
                 at++;
             }
         // register sets over this pass's masks [first, at)
@@ -147,12 +200,12 @@ void plan_expect(uint32_t n, bool c128, const qi_pauli_term *terms, size_t nt, E
                 size_t best = SIZE_MAX;
                 int least = 64;
                 for (size_t g = s_at; g < at; g++) {
-                    const int add = popc(local_bits(p.xs[g], ps, K) & ~r);
+                    const int add = popc(m[g].xl & ~r);
                     if (!add || popc(r) + add > 4 || add >= least) continue;
                     best = g; least = add;
                     if (at - s_at > kGreedyMax || add == 1) break;
                 }
-                if (best != SIZE_MAX) { r |= local_bits(p.xs[best], ps, K); grown = true; }
+                if (best != SIZE_MAX) { r |= m[best].xl; grown = true; }
             }
             for (int b = K - 1; b >= 0 && popc(r) < 4; b--) r |= 1u << b;
             for (int j = 0, b = 0; j < 4; b++)
@@ -160,7 +213,7 @@ void plan_expect(uint32_t n, bool c128, const qi_pauli_term *terms, size_t nt, E
             st.u0 = (uint32_t)p.nunits;
             // the masks inside the set, and (with no set of their own) the ones of more than four bits
             for (size_t g = s_at; g < at; g++) {
-                const uint32_t xl = local_bits(p.xs[g], ps, K);
+                const uint32_t xl = m[g].xl;
                 const bool wide = popc(xl) > 4;
                 if (!wide && (xl & ~r)) continue;
                 const uint32_t xm = wide ? 0 : reg_bits(xl, st);
@@ -169,7 +222,8 @@ void plan_expect(uint32_t n, bool c128, const qi_pauli_term *terms, size_t nt, E
                 for (int run = 0; run < (wide ? 4 : 2); run++) {
                     const int im_w = run & 1, high = run >> 1;
                     const size_t e0 = p.nunits;
-                    for (uint32_t t = head[g]; t != UINT32_MAX; t = next[t]) {
+                    Finder by_signs(p.table, m[g].count);
+                    for (uint32_t t = m[g].head; t != UINT32_MAX; t = p.next[t]) {
                         const qi_pauli_term &tm = terms[t];
                         const int ny = popc(tm.x_mask & tm.z_mask);
                         if ((ny & 1) != im_w) continue;
@@ -182,10 +236,9 @@ void plan_expect(uint32_t n, bool c128, const qi_pauli_term *terms, size_t nt, E
                             if (part && c == 0.0) continue;
                             const uint64_t zo = tm.z_mask & ~q;
                             const uint32_t fl = part ? kExpImag : 0u;
-                            size_t e = e0;
-                            while (e < p.nunits && !(p.units[e].zo == zo && p.units[e].zl == (zl & ~r) &&
-                                                     (p.units[e].flags() & kExpImag) == fl))
-                                e++;
+                            const size_t e = by_signs.find(mix(zo, uint64_t(zl & ~r) << 1 | part), e0, p.nunits, [&](size_t u) {
+                                return p.units[u].zo == zo && p.units[u].zl == (zl & ~r) && (p.units[u].flags() & kExpImag) == fl;
+                            });
                             ExpUnit &un = p.units[e];
                             if (e == p.nunits) {
                                 memset(&un, 0, sizeof un);
@@ -204,8 +257,7 @@ void plan_expect(uint32_t n, bool c128, const qi_pauli_term *terms, size_t nt, E
                         }
                     }
                 }
-                const uint64_t x = p.xs[g]; p.xs[g] = p.xs[s_at]; p.xs[s_at] = x;
-                const uint32_t h = head[g]; head[g] = head[s_at]; head[s_at] = h;
+                std::swap(m[g], m[s_at]);
                 s_at++;
             }
             st.nu = (uint32_t)p.nunits - st.u0;
@@ -242,14 +294,21 @@ template <typename R> void plan_apply(uint32_t n, const qi_pauli_term *terms, si
     p.K = K;
     const bool whole = (int)n == K;
     const uint64_t lowmask = whole ? (uint64_t(1) << n) - 1 : (uint64_t(1) << exp_low_qubits(c128)) - 1;
-    std::vector<uint64_t> xs;
-    std::unordered_map<uint64_t, std::vector<uint32_t>> of;  // terms of each mask
+    std::vector<ExpMask> m;  // the distinct masks and their terms, as in plan_expect
+    std::vector<uint32_t> next(nt, UINT32_MAX), table(exp_table_entries(nt)), unit_of(nt);
     bool diag = false;
+    Finder by_mask(table.data(), nt);
     for (size_t k = 0; k < nt; k++) {
-        if (!terms[k].x_mask) { diag = true; continue; }
-        std::vector<uint32_t> &v = of[terms[k].x_mask];
-        if (v.empty()) xs.push_back(terms[k].x_mask);
-        v.push_back((uint32_t)k);
+        const uint64_t x = terms[k].x_mask;
+        if (!x) { diag = true; continue; }
+        const size_t g = by_mask.find(mix(x, 0), 0, m.size(), [&](size_t i) { return m[i].x == x; });
+        if (g == m.size()) {
+            m.push_back(ExpMask{x, (uint32_t)k, (uint32_t)k, 1, 0});
+        } else {
+            next[m[g].tail] = (uint32_t)k;
+            m[g].tail = (uint32_t)k;
+            m[g].count++;
+        }
     }
     const uint32_t slots = apply_slots(K, c128);
     constexpr int SB = apply_slot_bits(sizeof(R) == 8), NS = 1 << SB;
@@ -260,12 +319,13 @@ template <typename R> void plan_apply(uint32_t n, const qi_pauli_term *terms, si
         for (int j = 0; j < SB; j++) r |= ((l >> exp_pos(&slots, j)) & 1u) << j;
         return r;
     };
-    std::vector<std::vector<uint64_t>> local;  // the masks of each pass; the rest (left) are remote
-    std::vector<uint64_t> tiles, left = xs;
+    std::vector<std::vector<ExpMask>> local;  // the masks of each pass; the rest (left) are remote
+    std::vector<uint64_t> tiles;
+    std::vector<ExpMask> left = m;
     for (;;) {
-        const uint64_t q0 = grow_tile(lowmask, left.data(), left.size(), K);
-        std::vector<uint64_t> in, out;
-        for (uint64_t x : left) ((x & ~q0) ? out : in).push_back(x);
+        const uint64_t q0 = grow_tile(lowmask, left.size(), K, [&](size_t g) { return left[g].x; });
+        std::vector<ExpMask> in, out;
+        for (const ExpMask &x : left) ((x.x & ~q0) ? out : in).push_back(x);
         if (!tiles.empty() && in.size() < kApplyPassMasks) break;
         uint64_t q = q0;
         for (uint32_t b = 0; b < n && popc(q) < K; b++) q |= uint64_t(1) << b;
@@ -274,6 +334,7 @@ template <typename R> void plan_apply(uint32_t n, const qi_pauli_term *terms, si
         left = out;
         if (left.empty()) break;
     }
+    std::vector<double> sums;  // a mask's coefficients: per unit, real then imaginary parts
     for (size_t ip = 0; ip < tiles.size(); ip++) {
         const uint64_t q = tiles[ip];
         ExpPass ps{};  // positions for local_bits
@@ -286,45 +347,48 @@ template <typename R> void plan_apply(uint32_t n, const qi_pauli_term *terms, si
         pass.u0 = (uint32_t)p.units.size();
         const bool last = ip + 1 == tiles.size();  // takes the remote masks
         const size_t nlocal = local[ip].size(), total = nlocal + (last ? left.size() : 0);
-        for (size_t m = 0; m < total; m++) {
-            const bool remote = m >= nlocal;
-            const uint64_t x = remote ? left[m - nlocal] : local[ip][m];
+        for (size_t g = 0; g < total; g++) {
+            const bool remote = g >= nlocal;
+            const ExpMask &mask = remote ? left[g - nlocal] : local[ip][g];
             const size_t e0 = p.units.size();
-            for (uint32_t t : of[x]) {
-                const qi_pauli_term &tm = terms[t];
-                const uint32_t zl = local_bits(tm.z_mask, ps, K);
-                const uint64_t zo = tm.z_mask & ~q;
-                size_t e = e0;
-                while (e < p.units.size() && !(p.units[e].zo == zo && p.units[e].zl == (zl & ~sm))) e++;
+            // the mask's units, and the one of each of its terms
+            Finder by_signs(table.data(), mask.count);
+            for (uint32_t t = mask.head; t != UINT32_MAX; t = next[t]) {
+                const uint32_t zl = local_bits(terms[t].z_mask, ps, K) & ~sm;
+                const uint64_t zo = terms[t].z_mask & ~q;
+                const size_t e = by_signs.find(mix(zo, zl), e0, p.units.size(),
+                                               [&](size_t u) { return p.units[u].zo == zo && p.units[u].zl == zl; });
                 if (e == p.units.size()) {
                     ApplyUnit<R> un{};
-                    un.zo = zo; un.x = x; un.zl = zl & ~sm;
-                    un.xl = remote ? 0 : local_bits(x, ps, K);
+                    un.zo = zo; un.x = mask.x; un.zl = zl;
+                    un.xl = remote ? 0 : local_bits(mask.x, ps, K);
                     un.flags = remote ? (uint32_t)kApplyRemote : 0u;
                     p.units.push_back(un);
                 }
+                unit_of[t] = (uint32_t)(e - e0);
             }
-            // the unit's coefficients, summed in FP64: c (-i)^ny (-1)^{popcount(slot & z)}
+            // the units' coefficients, summed in FP64: c (-i)^ny (-1)^{popcount(slot & z)}
+            sums.assign(2 * NS * (p.units.size() - e0), 0.0);
+            for (uint32_t t = mask.head; t != UINT32_MAX; t = next[t]) {
+                const qi_pauli_term &tm = terms[t];
+                const uint32_t zr = slot_bits(local_bits(tm.z_mask, ps, K));
+                double *const hr = sums.data() + 2 * NS * unit_of[t], *const hi = hr + NS;
+                double cr = tm.c_re, ci = tm.c_im, r;
+                switch (popc(tm.x_mask & tm.z_mask) & 3) {
+                case 1: r = cr; cr = ci; ci = -r; break;   // times -i
+                case 2: cr = -cr; ci = -ci; break;
+                case 3: r = cr; cr = -ci; ci = r; break;   // times i
+                default: break;
+                }
+                for (uint32_t s = 0; s < (uint32_t)NS; s++) {
+                    const bool odd = popc(s & zr) & 1;
+                    hr[s] += odd ? -cr : cr;
+                    hi[s] += odd ? -ci : ci;
+                }
+            }
             for (size_t e = e0; e < p.units.size(); e++) {
                 ApplyUnit<R> &un = p.units[e];
-                double hr[NS] = {0}, hi[NS] = {0};
-                for (uint32_t t : of[x]) {
-                    const qi_pauli_term &tm = terms[t];
-                    const uint32_t zl = local_bits(tm.z_mask, ps, K), zr = slot_bits(zl);
-                    if (un.zo != (tm.z_mask & ~q) || un.zl != (zl & ~sm)) continue;
-                    double cr = tm.c_re, ci = tm.c_im, r;
-                    switch (popc(tm.x_mask & tm.z_mask) & 3) {
-                    case 1: r = cr; cr = ci; ci = -r; break;   // times -i
-                    case 2: cr = -cr; ci = -ci; break;
-                    case 3: r = cr; cr = -ci; ci = r; break;   // times i
-                    default: break;
-                    }
-                    for (uint32_t s = 0; s < (uint32_t)NS; s++) {
-                        const bool odd = popc(s & zr) & 1;
-                        hr[s] += odd ? -cr : cr;
-                        hi[s] += odd ? -ci : ci;
-                    }
-                }
+                const double *const hr = sums.data() + 2 * NS * (e - e0), *const hi = hr + NS;
                 for (int s = 0; s < NS; s++) {
                     un.re[s] = (R)hr[s];
                     un.im[s] = (R)hi[s];

@@ -72,28 +72,43 @@ struct ExpPass {
 // Byte k of a packed position list.
 QI_HD inline uint32_t exp_pos(const uint32_t *p, int k) { return (p[k >> 2] >> (8 * (k & 3))) & 255u; }
 
+// The distinct x masks of a term list, each with its terms as a list in order.
+struct ExpMask {
+    uint64_t x;
+    uint32_t head, tail, count;  // terms: the first, the last (linked by ExpPlan::next), how many
+    uint32_t xl;                 // tile-local bits in the mask's pass
+};
 // The plan, in arrays the caller owns (capacities for nt terms below).
 struct ExpPlan {
     ExpPass *passes;    // <= nt
     ExpSet *sets;       // <= nt
-    ExpUnit *units;     // <= 4 nt + 1 (one spare: the kernel reads a unit ahead)
+    ExpUnit *units;     // <= exp_max_units + 1 (one spare: the kernel reads a unit ahead)
     ExpDiag *diags;     // <= nt
     uint64_t *far;      // x masks that no tile can hold: <= nt
-    uint64_t *xs;       // scratch: the distinct x masks, <= nt
-    uint32_t *gid;      // scratch: 2 per term
+    uint32_t *far_head; // and the first term of each
+    ExpMask *masks;     // scratch: <= nt
+    uint32_t *next;     // the next term of the same mask, UINT32_MAX: none
+    uint32_t *table;    // scratch: exp_table_entries(nt)
     size_t npasses, nsets, nunits, ndiags, nfar;
-    int K;              // tile qubits
+    int K;              // tile qubits (0: no tiles, every mask is streamed)
     bool complex_out;   // an imaginary part can be nonzero
 };
-// Bytes of the planning arena for nt terms.
-size_t exp_plan_bytes(size_t nt);
-// Carves the arrays out of `arena` (exp_plan_bytes(nt) bytes, 16-byte aligned).
-void exp_plan_carve(ExpPlan &p, void *arena, size_t nt);
+// Units that a term list can take at most: one per mask and Z support, two for
+// masks of more than four qubits, again as many for imaginary coefficients.
+size_t exp_max_units(const qi_pauli_term *terms, size_t nt);
+// Bytes of the planning arena for nt terms of at most `units` units (any nt
+// terms without it).
+size_t exp_plan_bytes(size_t nt, size_t units);
+inline size_t exp_plan_bytes(size_t nt) { return exp_plan_bytes(nt, 4 * nt); }
+// Carves the arrays out of `arena` (exp_plan_bytes bytes, 16-byte aligned).
+void exp_plan_carve(ExpPlan &p, void *arena, size_t nt, size_t units);
+inline void exp_plan_carve(ExpPlan &p, void *arena, size_t nt) { exp_plan_carve(p, arena, nt, 4 * nt); }
 // Widest tile for n qubits (n >= 4): the whole state, at most 13 (complex64) or
 // 12 (complex128) qubits of it.
 int exp_tile_qubits(uint32_t n, bool c128);
 // Qubits 0 .. low-1 are always in a tile: 128-byte runs in memory.
 inline int exp_low_qubits(bool c128) { return c128 ? 3 : 4; }
+// A state of fewer than 4 qubits has no tiles: every mask is streamed.
 void plan_expect(uint32_t n, bool c128, const qi_pauli_term *terms, size_t nt, ExpPlan &p);
 
 // ---- SumOp::apply on the same tiles ----
