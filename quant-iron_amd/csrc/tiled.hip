@@ -439,6 +439,7 @@ template <int I, typename R, int G> __device__ __forceinline__ void fetch_partne
 // Four words' worth of components (flat indices idx) flipped across lane bit I < 4 in place.
 template <int I, int E, typename R> __device__ __forceinline__ void flip_block(Regs<R, E> &v, const int *idx) {
     constexpr int W = kWords<R>, N = 4 / W;
+    static_assert(N <= 2 * E, "a tile holds a whole block");
     uint32_t x[4];
 #pragma unroll
     for (int q = 0; q < N; q++) to_words(v.d[idx[q]], x + W * q);
@@ -451,6 +452,7 @@ template <int KIND, bool CT, int I, int E, typename T, typename R>
 __device__ __forceinline__ void pairs_lane(Regs<R, E> &v, int addr, const R *k, uint32_t rcm, bool tok) {
     if constexpr (!CT && KIND == RO_X && I >= 0) {  // every amplitude moves: in place
         constexpr int N = 4 / kWords<R>;
+        static_assert(2 * E % N == 0, "whole blocks of components");
 #pragma unroll
         for (int q = 0; q < 2 * E; q += N) {
             int idx[N];
@@ -650,21 +652,25 @@ __device__ __forceinline__ void x_lane_c1(Regs<R, E> &v, int i, int addr) {
         for (int r = 0; r < E; r++) if ((r >> C) & 1) rs[n++] = r;
     }
     constexpr int N = 4 / kWords<R>;  // components per block of four words
-    const auto flip = [&](auto bit) {
+    // (a complex64 tile of two registers per thread has one register to move:
+    // two words, less than a block, so its partners come by ds_bpermute)
+    if constexpr (2 * H % N == 0) {
+        const auto flip = [&](auto bit) {
 #pragma unroll
-        for (int q = 0; q < 2 * H; q += N) {
-            int idx[N];
+            for (int q = 0; q < 2 * H; q += N) {
+                int idx[N];
 #pragma unroll
-            for (int j = 0; j < N; j++) idx[j] = 2 * rs[(q + j) / 2] + (q + j) % 2;
-            flip_block<decltype(bit)::value, E, R>(v, idx);
+                for (int j = 0; j < N; j++) idx[j] = 2 * rs[(q + j) / 2] + (q + j) % 2;
+                flip_block<decltype(bit)::value, E, R>(v, idx);
+            }
+        };
+        switch (i) {
+        case 0: flip(std::integral_constant<int, 0>{}); return;
+        case 1: flip(std::integral_constant<int, 1>{}); return;
+        case 2: flip(std::integral_constant<int, 2>{}); return;
+        case 3: flip(std::integral_constant<int, 3>{}); return;
+        default: break;
         }
-    };
-    switch (i) {
-    case 0: flip(std::integral_constant<int, 0>{}); return;
-    case 1: flip(std::integral_constant<int, 1>{}); return;
-    case 2: flip(std::integral_constant<int, 2>{}); return;
-    case 3: flip(std::integral_constant<int, 3>{}); return;
-    default: break;
     }
 #pragma unroll
     for (int g0 = 0; g0 < H; g0 += G) {
@@ -763,8 +769,10 @@ template <int B, bool XS, int E>
 __device__ __forceinline__ void shear_reg(Regs<float, E> &v, float a, float b) {
     const float na = -a, nb = -b;
     // two register pairs (four chains of three) interleaved: 545 cycles per
-    // 64 amplitudes against 618 one pair at a time
-    constexpr int G = 2;
+    // 64 amplitudes against 618 one pair at a time (a tile of two registers per
+    // thread holds one pair)
+    constexpr int G = E / 2 < 2 ? E / 2 : 2;
+    static_assert(E / 2 % G == 0, "whole groups of pairs");
 #pragma unroll
     for (int n0 = 0; n0 < E / 2; n0 += G)
 #pragma unroll
@@ -850,6 +858,7 @@ template <int I> __device__ __forceinline__ void swap_rows4(uint32_t (&a)[4], ui
 }
 template <int B, int I, int E, typename R> __device__ __forceinline__ void xlr_bits(Regs<R, E> &v, uint32_t lane) {
     constexpr int W = kWords<R>, N = 4 / W;
+    static_assert(E % N == 0, "whole blocks of register pairs");
     const uint32_t hi = I < 2 && ((lane >> I) & 1u) ? ~0u : 0u;
 #pragma unroll
     for (int n = 0; n < E; n += N) {  // n: component n % 2 of register pair n / 2
@@ -894,6 +903,7 @@ __device__ __forceinline__ void xll_op(Regs<R, E> &v, uint32_t lane, int i, int 
     const int addr = int((lane ^ ((1u << i) | (1u << i2))) << 2);
     const uint64_t m = __builtin_amdgcn_ballot_w64(((lane >> i) & 1u) != ((lane >> i2) & 1u));
     constexpr int G = sizeof(R) == 4 ? 8 : 4;
+    static_assert(2 * E % G == 0, "whole groups of components");
 #pragma unroll
     for (int k0 = 0; k0 < 2 * E; k0 += G) {
         R y[G];

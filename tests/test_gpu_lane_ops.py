@@ -47,3 +47,21 @@ def test_low_qubit_gates_match_the_oracle(ctx, prec, K, seed):
     s.apply_gates_inplace(gates, mode=L.EXEC_TILED, tile_qubits=K)
     tol = 150 * 4 * (2.0 ** -24 if prec == "c64" else 2.0 ** -53)
     assert np.max(np.abs(s.state_vector - O.apply_gates(psi, gates))) <= tol
+
+
+# two registers per thread (one register bit): the smallest tile that the
+# options accept, in both precisions
+@pytest.mark.parametrize("prec,threads", [("c64", 9), ("c128", 9), ("c64", 8)])
+@pytest.mark.parametrize("seed", [1, 2])
+def test_tiles_of_few_registers_match_the_oracle(ctx, prec, threads, seed):
+    rng = np.random.default_rng([seed, threads, 40])
+    gates = low_gates(rng, 150)
+    cnots = [{"kind": "X", "targets": [t], "controls": [c]} for c in range(N) for t in range(6) if c != t]
+    turns = [{"kind": k, "targets": [q], "params": [float(rng.uniform(0, 2 * np.pi))]} for q in range(N) for k in ("RX", "RY")]
+    more = cnots + turns
+    gates = np.concatenate([gates, gates_array([more[i] for i in rng.permutation(len(more))])])
+    psi = random_state(N, rng)
+    s = qiron.State.from_vector_unchecked(psi, prec)
+    s.apply_gates_inplace(gates, mode=L.EXEC_TILED, tile_qubits=10, tile_threads_log2=threads)
+    tol = gates.size * 4 * (2.0 ** -24 if prec == "c64" else 2.0 ** -53)
+    assert np.max(np.abs(s.state_vector - O.apply_gates(psi, gates))) <= tol
