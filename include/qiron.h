@@ -195,7 +195,12 @@ qi_status qi_state_clone(qi_state_t src, qi_state_t *out, qi_error *err);
 qi_status qi_state_copy(qi_state_t dst, qi_state_t src, qi_error *err);
 uint32_t qi_state_num_qubits(qi_state_t s);
 int32_t qi_state_precision(qi_state_t s);
-/* Device address of the amplitude array (interop; owned by the handle). */
+/* Device address of the amplitude array (interop; owned by the handle).
+ * Callers order their own kernels on it with the engine's calls themselves
+ * (each call has finished when it returns). qi_state_destroy waits for
+ * everything that is queued on the device when the address has been asked for,
+ * so that work queued before it is done with the array; after it the address
+ * may belong to another state. */
 void *qi_state_device_ptr(qi_state_t s);
 /* Constructors: new_zero / new_basis_n / new_plus / new_minus / new_ghz
  * (state.rs:165-300); `basis` is used by QI_INIT_BASIS only. */

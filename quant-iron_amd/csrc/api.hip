@@ -83,10 +83,19 @@ static Status alloc_state(Ctx &C, uint32_t n, int prec, State &out) {
     if (e != hipSuccess) { out.d = nullptr; return oom_err(e); }
     return Status{};
 }
-// The caller has waited for the context's stream.
+// The caller has waited for all work that can use the buffer.
 static void free_state(State &s) {
     if (s.d) s.ctx->idle.put(s.d, s.bytes());
     s.d = nullptr;
+}
+
+// Waits for every stream of a device, the caller's own among them.
+static void wait_device(int device) {
+    int dev = device;
+    (void)hipGetDevice(&dev);
+    if (dev != device) (void)hipSetDevice(device);
+    (void)hipDeviceSynchronize();
+    if (dev != device) (void)hipSetDevice(dev);
 }
 
 Status ensure(DevBuf &b, size_t bytes) {
@@ -763,7 +772,8 @@ qi_status qi_state_destroy(qi_state_t s) {
     if (!s) return QI_OK;
     {
         QI_LOCK(s->s.ctx);
-        (void)hipStreamSynchronize(s->s.ctx->stream);
+        if (s->lent.load()) wait_device(s->s.ctx->device);  // the caller's kernels may still use the address
+        else (void)hipStreamSynchronize(s->s.ctx->stream);
         free_state(s->s);
     }
     delete s;
@@ -795,7 +805,11 @@ qi_status qi_state_copy(qi_state_t dst, qi_state_t src, qi_error *err) {
 
 uint32_t qi_state_num_qubits(qi_state_t s) { return s ? s->s.n : 0; }
 int32_t qi_state_precision(qi_state_t s) { return s ? s->s.prec : -1; }
-void *qi_state_device_ptr(qi_state_t s) { return s ? s->s.d : nullptr; }
+void *qi_state_device_ptr(qi_state_t s) {
+    if (!s) return nullptr;
+    s->lent.store(true);
+    return s->s.d;
+}
 
 qi_status qi_state_init(qi_state_t s, qi_init kind, uint64_t basis, qi_error *err) {
     QI_NULLCHK(s);

@@ -5,6 +5,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <cstring>
 #include <memory>
@@ -63,13 +64,15 @@ template <typename T> hipError_t dev_malloc(T **p, size_t bytes) { return dev_ma
 // SumOp product takes 0.66 ms, with hipMalloc and hipFree around it 0.8 to
 // 5 ms). Bounded (kIdleBytes and kIdleBuffers per context, the oldest go
 // first), given back when an allocation fails and when the context ends. A
-// buffer is idle only after the context's stream has been waited for.
+// buffer is idle only after the context's stream has been waited for, and the
+// whole device where the caller has had its address (qi_state_s::lent).
 constexpr size_t kIdleBytes = size_t(2) << 30;
 constexpr size_t kIdleBuffers = 32;
 struct IdleBuffers {
     std::mutex mu;
     std::vector<DevBuf> idle;  // oldest first
     size_t bytes = 0;
+    IdleBuffers() { idle.reserve(kIdleBuffers); }  // put() runs in destructors and allocates nothing
     void *take(size_t want);       // null: none of that size
     void put(void *p, size_t bytes);
     void release();
@@ -254,4 +257,5 @@ struct qi_ctx_s {
 };
 struct qi_state_s {
     qi::State s;
+    std::atomic<bool> lent{false};  // qi_state_device_ptr has given the address out
 };
