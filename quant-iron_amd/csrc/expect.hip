@@ -4,8 +4,8 @@
 // term whose X and Y factors lie inside the tile's qubits from that one read:
 // the tile is staged in LDS, a thread takes the 16 amplitudes of a register
 // set into FP64 registers and forms w = conj(a) b once per pair and x mask.
-// Terms that no tile holds (X support too wide) stream the state, one pass per
-// x mask (k_expect_group).
+// Terms that no tile holds (X support too wide) stream the state, one read per
+// x mask (k_expect_far).
 #include <algorithm>
 
 #include "expect_plan.h"
@@ -217,12 +217,16 @@ __global__ __launch_bounds__(512, CPLX ? 2 : 4) void k_expect_tiles(const T *__r
     }
 }
 
-// A term for the streaming kernel.
+// A term for the streaming kernel, and the terms of one x mask.
 struct TermK {
     uint64_t x, z;
     unsigned q0;  // 3 * nY mod 4
     unsigned pad;
     double c[2];
+};
+struct FarMask {
+    uint64_t x;
+    uint32_t t0, nt;
 };
 
 // Quarter turns of (-i)^{nY} (-1)^{popcount(i & z)}.
@@ -233,17 +237,24 @@ __device__ __forceinline__ uint64_t insert_zero(uint64_t k, unsigned p) {
     return ((k >> p) << (p + 1)) | (k & ((uint64_t(1) << p) - 1));
 }
 
-// Expectation of a group of terms sharing the same x mask, one pass over the
-// state (masks wider than a tile, states of fewer than 4 qubits):
+// Expectation of the terms that no tile holds (x masks wider than a tile, states
+// of fewer than 4 qubits), one read of the state per x mask:
 //   sum_i conj(psi_i) psi_{i^x} h(i),  h(i) = sum_t c_t i^{q_t(i)}.
-// FP64 accumulation with two-sum compensation; one partial per block.
+// FP64 accumulation with two-sum compensation; per_mask blocks of each mask,
+// one partial per block. All masks run in one launch: a mask of many has few
+// blocks, and a launch of its own would leave the chip to them alone (26
+// qubits, 100 random strings: 324 ms in complex64, 418 in complex128).
 template <typename T>
-__global__ __launch_bounds__(256) void k_expect_group(const T *__restrict__ psi, uint64_t items, uint64_t x,
-                                                      unsigned pivot, const TermK *__restrict__ terms, int nt,
-                                                      double *__restrict__ part) {
+__global__ __launch_bounds__(256) void k_expect_far(const T *__restrict__ psi, uint64_t dim, const FarMask *__restrict__ masks,
+                                                    uint32_t per_mask, const TermK *__restrict__ all_terms, double *__restrict__ part) {
     __shared__ double sh[4 * 4];
+    const FarMask &fm = masks[blockIdx.x / per_mask];
+    const uint64_t x = fm.x, items = x ? dim / 2 : dim;
+    const unsigned pivot = x ? __builtin_ctzll(x) : 0;
+    const TermK *__restrict__ terms = all_terms + fm.t0;
+    const int nt = (int)fm.nt;
     DD v[2] = {dd_zero(), dd_zero()};
-    for (uint64_t k = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; k < items; k += uint64_t(gridDim.x) * blockDim.x) {
+    for (uint64_t k = uint64_t(blockIdx.x % per_mask) * blockDim.x + threadIdx.x; k < items; k += uint64_t(per_mask) * blockDim.x) {
         uint64_t i = x == 0 ? k : insert_zero(k, pivot);
         uint64_t j = i ^ x;
         double ar = psi[i].x, ai = psi[i].y, br = psi[j].x, bi = psi[j].y;
@@ -465,7 +476,7 @@ constexpr uint64_t kExpBlocks = 4096, kExpBlocksMin = 16;
 size_t up16(size_t b) { return (b + 15) & ~size_t(15); }
 
 struct ExpLaunch {
-    size_t sets, units, diags, far, bytes;  // offsets in the device tables (passes first), their size
+    size_t sets, units, diags, far, masks, bytes;  // offsets in the device tables (passes first), their size
     uint32_t per_pass, per_far;
     uint64_t tiles;
     size_t blocks;  // partials of the whole call
@@ -479,32 +490,20 @@ TermK far_term(const qi_pauli_term &p) {
     return t;
 }
 
-// Plans into `arena` (exp_plan_bytes(nt)); a state of fewer than 4 qubits has
-// no tiles: every mask is streamed.
-ExpLaunch plan_launch(const State &s, const qi_pauli_term *terms, size_t nt, void *arena, ExpPlan &p, size_t *far_terms) {
+// Plans into `arena` (exp_plan_bytes(nt)).
+ExpLaunch plan_launch(const State &s, const qi_pauli_term *terms, size_t nt, void *arena, ExpPlan &p) {
     exp_plan_carve(p, arena, nt);
-    const bool c128 = s.prec == QI_C128;
-    if (s.n >= 4) {
-        plan_expect(s.n, c128, terms, nt, p);
-    } else {
-        p.npasses = p.nsets = p.nunits = p.ndiags = p.nfar = 0;
-        p.K = 0;
-        for (size_t k = 0; k < nt; k++) {
-            size_t g = 0;
-            while (g < p.nfar && p.far[g] != terms[k].x_mask) g++;
-            if (g == p.nfar) p.far[p.nfar++] = terms[k].x_mask;
-        }
-    }
+    plan_expect(s.n, s.prec == QI_C128, terms, nt, p);
     size_t nf = 0;
     for (size_t g = 0; g < p.nfar; g++)
-        for (size_t k = 0; k < nt; k++) nf += terms[k].x_mask == p.far[g];
-    *far_terms = nf;
+        for (uint32_t t = p.far_head[g]; t != UINT32_MAX; t = p.next[t]) nf++;
     ExpLaunch L{};
     L.sets = up16(p.npasses * sizeof(ExpPass));
     L.units = L.sets + up16(p.nsets * sizeof(ExpSet));
     L.diags = L.units + up16((p.nunits + 1) * sizeof(ExpUnit));
     L.far = L.diags + up16(p.ndiags * sizeof(ExpDiag));
-    L.bytes = L.far + up16(nf * sizeof(TermK));
+    L.masks = L.far + up16(nf * sizeof(TermK));
+    L.bytes = L.masks + up16(p.nfar * sizeof(FarMask));
     const uint64_t dim = uint64_t(1) << s.n;
     if (p.npasses) {
         L.tiles = dim >> p.K;
@@ -516,20 +515,24 @@ ExpLaunch plan_launch(const State &s, const qi_pauli_term *terms, size_t nt, voi
 }
 
 // Device tables in the order of ExpLaunch's offsets.
-void pack_tables(const ExpPlan &p, const ExpLaunch &L, const qi_pauli_term *terms, size_t nt, unsigned char *dst) {
+void pack_tables(const ExpPlan &p, const ExpLaunch &L, const qi_pauli_term *terms, unsigned char *dst) {
     memcpy(dst, p.passes, p.npasses * sizeof(ExpPass));
     memcpy(dst + L.sets, p.sets, p.nsets * sizeof(ExpSet));
     if (p.npasses) memcpy(dst + L.units, p.units, (p.nunits + 1) * sizeof(ExpUnit));
     memcpy(dst + L.diags, p.diags, p.ndiags * sizeof(ExpDiag));
-    TermK *f = reinterpret_cast<TermK *>(dst + L.far);
-    for (size_t g = 0; g < p.nfar; g++)
-        for (size_t k = 0; k < nt; k++)
-            if (terms[k].x_mask == p.far[g]) *f++ = far_term(terms[k]);
+    TermK *const f = reinterpret_cast<TermK *>(dst + L.far);
+    FarMask *const m = reinterpret_cast<FarMask *>(dst + L.masks);
+    uint32_t k = 0;
+    for (size_t g = 0; g < p.nfar; g++) {
+        m[g] = FarMask{p.far[g], k, 0};
+        for (uint32_t t = p.far_head[g]; t != UINT32_MAX; t = p.next[t]) f[k++] = far_term(terms[t]);
+        m[g].nt = k - m[g].t0;
+    }
 }
 
 template <typename T>
-Status launch_all(const State &s, const ExpPlan &p, const ExpLaunch &L, const qi_pauli_term *terms, size_t nt,
-                  const unsigned char *tab, double *part, double *out, hipStream_t st) {
+Status launch_all(const State &s, const ExpPlan &p, const ExpLaunch &L, const unsigned char *tab, double *part, double *out,
+                  hipStream_t st) {
     if (p.npasses) {
         const unsigned threads = std::max(64u, 1u << (p.K - 4));
         auto *const kernel = p.complex_out ? k_expect_tiles<T, true> : k_expect_tiles<T, false>;
@@ -538,17 +541,10 @@ Status launch_all(const State &s, const ExpPlan &p, const ExpLaunch &L, const qi
                            (const ExpSet *)(tab + L.sets), (const ExpUnit *)(tab + L.units),
                            (const ExpDiag *)(tab + L.diags), p.K, L.per_pass, L.tiles, part);
     }
-    const TermK *f = reinterpret_cast<const TermK *>(tab + L.far);
-    double *pg = part + size_t(L.per_pass) * p.npasses * 4;
-    for (size_t g = 0; g < p.nfar; g++) {
-        const uint64_t x = p.far[g], dim = uint64_t(1) << s.n;
-        int cnt = 0;
-        for (size_t k = 0; k < nt; k++) cnt += terms[k].x_mask == x;
-        hipLaunchKernelGGL(k_expect_group<T>, dim3(L.per_far), dim3(256), 0, st, (const T *)s.d, x ? dim / 2 : dim, x,
-                           x ? (unsigned)__builtin_ctzll(x) : 0u, f, cnt, pg);
-        f += cnt;
-        pg += size_t(L.per_far) * 4;
-    }
+    if (p.nfar)
+        hipLaunchKernelGGL(k_expect_far<T>, dim3(L.per_far * (unsigned)p.nfar), dim3(256), 0, st, (const T *)s.d, uint64_t(1) << s.n,
+                           (const FarMask *)(tab + L.masks), L.per_far, (const TermK *)(tab + L.far),
+                           part + size_t(L.per_pass) * p.npasses * 4);
     hipLaunchKernelGGL(k_reduce_partials<2>, dim3(1), dim3(256), 0, st, (const double *)part, (int)L.blocks, out);
     QI_HIP_TRY(hipGetLastError());
     return Status{};
@@ -556,14 +552,14 @@ Status launch_all(const State &s, const ExpPlan &p, const ExpLaunch &L, const qi
 
 // Uploads the packed tables through the context's pinned staging buffer and
 // runs the launches; the result lands in the context's pinned words.
-Status expect_run(State &s, const qi_pauli_term *terms, size_t nt, const ExpPlan &p, const ExpLaunch &L, void *dtab,
-                  double *part, double *re, double *im, hipStream_t st) {
+Status expect_run(State &s, const qi_pauli_term *terms, const ExpPlan &p, const ExpLaunch &L, void *dtab, double *part,
+                  double *re, double *im, hipStream_t st) {
     Ctx &C = *s.ctx;
-    pack_tables(p, L, terms, nt, (unsigned char *)C.stage);
+    pack_tables(p, L, terms, (unsigned char *)C.stage);
     QI_HIP_TRY(hipMemcpyAsync(dtab, C.stage, L.bytes, hipMemcpyHostToDevice, st));
     Status e = s.prec == QI_C128
-                   ? launch_all<double2>(s, p, L, terms, nt, (const unsigned char *)dtab, part, C.host_pinned, st)
-                   : launch_all<float2>(s, p, L, terms, nt, (const unsigned char *)dtab, part, C.host_pinned, st);
+                   ? launch_all<double2>(s, p, L, (const unsigned char *)dtab, part, C.host_pinned, st)
+                   : launch_all<float2>(s, p, L, (const unsigned char *)dtab, part, C.host_pinned, st);
     if (!e.ok()) return e;
     QI_HIP_TRY(hipStreamSynchronize(st));
     *re = C.host_pinned[0];
@@ -606,18 +602,17 @@ Status sumop_apply_tiles(const State &in, State &out, const qi_pauli_term *terms
                               : apply_tiles<float2, float>(in, out, terms, nt, st);
 }
 
-size_t expect_stage_bytes(size_t nt) { return exp_plan_bytes(nt) + nt * sizeof(TermK) + 256; }
+size_t expect_stage_bytes(size_t nt) { return exp_plan_bytes(nt) + nt * (sizeof(TermK) + sizeof(FarMask)) + 256; }
 
 Status sumop_expectation(State &s, const qi_pauli_term *terms, size_t nt, double *re, double *im, hipStream_t st) {
     Ctx &C = *s.ctx;
     Status e = ensure_stage(C, expect_stage_bytes(nt));
     if (!e.ok()) return e;
     ExpPlan p;
-    size_t nf;
-    const ExpLaunch L = plan_launch(s, terms, nt, C.plan_arena.data(), p, &nf);
+    const ExpLaunch L = plan_launch(s, terms, nt, C.plan_arena.data(), p);
     if (!(e = ensure(C.ops, L.bytes)).ok()) return e;
     if (!(e = ensure(C.red, L.blocks * 4 * sizeof(double))).ok()) return e;
-    return expect_run(s, terms, nt, p, L, C.ops.p, (double *)C.red.p, re, im, st);
+    return expect_run(s, terms, p, L, C.ops.p, (double *)C.red.p, re, im, st);
 }
 
 // ---------------------------------------------------- no-allocation variant --
@@ -632,7 +627,7 @@ Status sumop_expectation(State &s, const qi_pauli_term *terms, size_t nt, double
 namespace {
 struct NoAllocScratch {
     unsigned char tab[kNoAllocMaxTerms * (sizeof(ExpPass) + sizeof(ExpSet) + 4 * sizeof(ExpUnit) + sizeof(ExpDiag) +
-                                          sizeof(TermK)) + 512];
+                                          sizeof(TermK) + sizeof(FarMask)) + 512];
     double part[(kExpBlocks + 2 * kExpBlocksMin * kNoAllocMaxTerms) * 4];
 };
 }  // namespace
@@ -664,11 +659,10 @@ Status sumop_expectation_noalloc(State &s, const qi_pauli_term *terms, size_t nt
     if (nt == 0) return Status{};
     NoAllocScratch *sc = reinterpret_cast<NoAllocScratch *>(base);
     ExpPlan p;
-    size_t nf;
-    const ExpLaunch L = plan_launch(s, terms, nt, s.ctx->plan_arena.data(), p, &nf);
+    const ExpLaunch L = plan_launch(s, terms, nt, s.ctx->plan_arena.data(), p);
     if (L.bytes > sizeof sc->tab || L.blocks * 4 * sizeof(double) > sizeof sc->part)
         return make_err(QI_ERR_DEVICE, 0, 0, 0, 0, "expectation scratch");
-    return expect_run(s, terms, nt, p, L, sc->tab, sc->part, re, im, st);
+    return expect_run(s, terms, p, L, sc->tab, sc->part, re, im, st);
 }
 
 }  // namespace qi
