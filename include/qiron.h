@@ -240,7 +240,8 @@ qi_status qi_pauli_exp_neg_i_dt(qi_state_t s, const qi_pauli_term *t, double dt,
 /* out <- SumOp::apply(in) (pauli_string.rs:453-466). in != out. */
 qi_status qi_sumop_apply(qi_state_t in, qi_state_t out, const qi_pauli_term *terms, size_t nterms,
                          qi_error *err);
-/* SumOp::expectation_value (pauli_string.rs:485-507): FP64 compensated sums. */
+/* SumOp::expectation_value (pauli_string.rs:485-507): FP64, every product added by
+ * two-sum. */
 qi_status qi_sumop_expectation(qi_state_t s, const qi_pauli_term *terms, size_t nterms,
                                double *re, double *im, qi_error *err);
 /* qi_sumop_expectation with no allocation of any kind: no counterpart in the

@@ -4,6 +4,7 @@
 // term whose X and Y factors lie inside the tile's qubits from that one read:
 // the tile is staged in LDS, a thread takes the 16 amplitudes of a register
 // set into FP64 registers and forms w = conj(a) b once per pair and x mask.
+// Every pair's product is added by two-sum.
 // Terms that no tile holds (X support too wide) stream the state, one read per
 // x mask (k_expect_far).
 #include <algorithm>
@@ -68,14 +69,16 @@ __device__ __forceinline__ void pair_products(const double (&ar)[kExpSlots], con
     }
 }
 
-// What bounds it: FP64 issue (VALU busy 44% of the time) and one read of the
-// state per pass (2.6 TB/s), neither hidden well behind the other: a CU holds
-// 16 waves (128 VGPRs), in two workgroups at 64 KiB tiles, four at 32 KiB. The
+// What bounds it: FP64 issue (VALU busy 66% of the time) and one read of the
+// state per pass (3.0 TB/s), neither hidden well behind the other: a CU holds
+// 16 waves (125 VGPRs), in two workgroups at 64 KiB tiles, four at 32 KiB. The
 // four-bit register sets share the LDS reads (16 per thread and set) and the
 // FP64 conversions among the masks of the set; a Heisenberg bond costs a
-// multiply-add pair and one multiply-add per amplitude pair, whatever its
+// multiply-add pair and a compensated product per amplitude pair, whatever its
 // number of terms. 29 qubits, complex64, a chain with fields (113 terms, 29 x
-// masks): 67.1 ms with one read of the state per mask, 5.0 ms in four passes.
+// masks): 66 ms with one read of the state per mask, 5.7 ms in four passes (5.0
+// with plain FP64 sums inside a register set, which lose what two large
+// products that cancel leave between them).
 // The imaginary sums (complex coefficients) take registers that cost half the
 // waves, so they have an instance of their own.
 template <typename T, bool CPLX>
@@ -134,7 +137,6 @@ __global__ __launch_bounds__(512, CPLX ? 2 : 4) void k_expect_tiles(const T *__r
                 ar[s] = a.x;
                 ai[s] = a.y;
             }
-            double sr = 0.0, sm = 0.0;  // this set's sums
             double u[8] = {0, 0, 0, 0, 0, 0, 0, 0};
             ExpUnit nxt = units[st.u0];
             for (uint32_t ui = st.u0; ui < st.u0 + st.nu; ui++) {
@@ -165,31 +167,26 @@ __global__ __launch_bounds__(512, CPLX ? 2 : 4) void k_expect_tiles(const T *__r
                     } break;
                     }
                 }
-                double v0 = u[0] * un.h[0], v1 = u[1] * un.h[1];
+                // every product by two-sum: first the unit's own sum, whose sign
+                // is the same for all eight
+                DD v{u[0] * un.h[0], 0.0};
 #pragma unroll
-                for (int k = 2; k < 8; k += 2) {
-                    v0 = __builtin_fma(u[k], un.h[k], v0);
-                    v1 = __builtin_fma(u[k + 1], un.h[k + 1], v1);
+                for (int k = 1; k < 8; k++) dd_acc(v, u[k] * un.h[k]);
+                const uint32_t odd = __popcll(base & un.zo) + __popc(tl & un.zl);
+                if (CPLX && (un.flags() & kExpImag)) {
+                    dd_acc(acc[1], flip_sign(v.s, odd));
+                    acc[1].c += flip_sign(v.c, odd);
+                } else {
+                    dd_acc(acc[0], flip_sign(v.s, odd));
+                    acc[0].c += flip_sign(v.c, odd);
                 }
-                const double v = flip_sign(v0 + v1, __popcll(base & un.zo) + __popc(tl & un.zl));
-                if (CPLX && (un.flags() & kExpImag)) sm += v;
-                else sr += v;
             }
             if (st.diag) {
-                // Walsh sums W[p] = sum_s (-1)^{popcount(s & p)} |a_s|^2: a term adds
-                // its signed coefficient times the sum of its register-bit pattern
-                double w[kExpSlots];
+                // the signed sums of the coefficients by register-bit pattern, then
+                // their Walsh transform: the factor of each |a|^2
+                double w[kExpSlots], h[kExpSlots], hi[kExpSlots];
 #pragma unroll
                 for (int s = 0; s < kExpSlots; s++) w[s] = __builtin_fma(ar[s], ar[s], ai[s] * ai[s]);
-#pragma unroll
-                for (int b = 1; b < kExpSlots; b <<= 1)
-#pragma unroll
-                    for (int s = 0; s < kExpSlots; s++)
-                        if (!(s & b)) {
-                            const double x = w[s], y = w[s | b];
-                            w[s] = x + y;
-                            w[s | b] = x - y;
-                        }
 #pragma unroll
                 for (int p = 0; p < kExpSlots; p++) {
                     double cr = 0.0, ci = 0.0;
@@ -200,12 +197,25 @@ __global__ __launch_bounds__(512, CPLX ? 2 : 4) void k_expect_tiles(const T *__r
                         cr += flip_sign(t1.re, odd);
                         if (CPLX) ci += flip_sign(t1.im, odd);
                     }
-                    sr = __builtin_fma(w[p], cr, sr);
-                    if (CPLX) sm = __builtin_fma(w[p], ci, sm);
+                    h[p] = cr;
+                    hi[p] = ci;
+                }
+#pragma unroll
+                for (int b = 1; b < kExpSlots; b <<= 1)
+#pragma unroll
+                    for (int s = 0; s < kExpSlots; s++)
+                        if (!(s & b)) {
+                            const double x = h[s], y = h[s | b], z = hi[s], t1 = hi[s | b];
+                            h[s] = x + y;
+                            h[s | b] = x - y;
+                            if (CPLX) { hi[s] = z + t1; hi[s | b] = z - t1; }
+                        }
+#pragma unroll
+                for (int s = 0; s < kExpSlots; s++) {
+                    dd_acc(acc[0], w[s] * h[s]);
+                    if (CPLX) dd_acc(acc[1], w[s] * hi[s]);
                 }
             }
-            dd_acc(acc[0], sr);
-            if (CPLX) dd_acc(acc[1], sm);
         }
         __syncthreads();  // the next tile overwrites the LDS copy
     }

@@ -150,10 +150,10 @@ void plan_expect(uint32_t n, bool c128, const qi_pauli_term *terms, size_t nt, E
     }
     // A complex64 state of more qubits than its widest tile takes tiles of one
     // qubit less, unless a mask needs that one: at half the LDS, four
-    // workgroups per CU load and compute out of step instead of two. 28 qubits,
-    // 4 x 7 lattice: 3.76 -> 3.48 ms; 24-qubit chain 232 -> 207 us; 29-qubit chain
-    // 5.09 -> 5.01 ms (11 qubits: 3.86 ms, 211 us, 5.07 ms; complex128 with 11
-    // instead of 12: 1.92 -> 2.16 ms at 27 qubits).
+    // workgroups per CU load and compute out of step instead of two. Tiles of 13
+    // -> 12 qubits: 28 qubits, 4 x 7 lattice 4.45 -> 4.01 ms; 24-qubit chain 216 ->
+    // 189 us; 29-qubit chain 6.07 -> 5.63 ms (11 qubits: 4.49 ms, 200 us, 5.95 ms;
+    // complex128 with 11 instead of 12: 3.03 -> 3.25 ms at 27 qubits).
     int K = exp_tile_qubits(n, c128);
     const bool whole = (int)n == K;
     const uint64_t lowmask = whole ? (uint64_t(1) << n) - 1 : (uint64_t(1) << low) - 1;
