@@ -173,7 +173,8 @@ __global__ __launch_bounds__(256) void k_expand(const double *__restrict__ hd, d
 // as three launches: the chain of the total, the quotients (in parallel), the
 // chain of the cumulative sum. A chain is one lane's dependent FP64 additions:
 // the rest of the workgroup stages the values in LDS a block ahead, the lane
-// reads them sixteen ahead of their additions. 2^16 values: see k_chain.
+// reads them sixteen ahead of their additions. Up to a block of values, one
+// launch does the three.
 constexpr int kChainBlock = 2048;  // values staged at a time
 struct Group16 {
     double2 x[8];
@@ -183,6 +184,37 @@ __device__ __forceinline__ Group16 group_at(const double *lds) {
 #pragma unroll
     for (int j = 0; j < 8; j++) r.x[j] = reinterpret_cast<const double2 *>(lds)[j];
     return r;
+}
+// cum + lds[0] + ... + lds[cnt - 1] by one lane; with CDF every partial sum goes
+// to cdf[i]. lds holds kChainBlock values.
+template <bool CDF>
+__device__ __forceinline__ double chain_block(const double *lds, int cnt, double cum, double *__restrict__ cdf) {
+    Group16 nxt = group_at(lds);
+    int i = 0;
+    for (; i + 16 <= cnt; i += 16) {
+        const Group16 cur = nxt;
+        nxt = group_at(lds + (i + 32 <= kChainBlock ? i + 16 : i));
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (CDF) {
+            double2 v[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                v[j].x = (j ? v[j - 1].y : cum) + cur.x[j].x;
+                v[j].y = v[j].x + cur.x[j].y;
+            }
+            cum = v[7].y;
+#pragma unroll
+            for (int j = 0; j < 8; j++) *reinterpret_cast<double2 *>(cdf + i + 2 * j) = v[j];
+        } else {
+#pragma unroll
+            for (int j = 0; j < 8; j++) { cum += cur.x[j].x; cum += cur.x[j].y; }
+        }
+    }
+    for (; i < cnt; i++) {
+        cum += lds[i];
+        if constexpr (CDF) cdf[i] = cum;
+    }
+    return cum;
 }
 // cum + p[lo] + ... + p[hi - 1]; with CDF every partial sum goes to cdf[i].
 // 256 threads; buf: 2 blocks. The result is valid in thread 0.
@@ -206,35 +238,27 @@ __device__ __forceinline__ double chain(const double *__restrict__ p, uint64_t l
         if (tid >= 64 && at + kChainBlock < hi) stage(b ^ 1, at + kChainBlock, 64, 192);
         if (tid == 0) {
             const int cnt = hi - at < kChainBlock ? int(hi - at) : kChainBlock;
-            Group16 nxt = group_at(buf[b]);
-            int i = 0;
-            for (; i + 16 <= cnt; i += 16) {
-                const Group16 cur = nxt;
-                nxt = group_at(buf[b] + (i + 32 <= kChainBlock ? i + 16 : i));
-                __builtin_amdgcn_sched_barrier(0);
-                if constexpr (CDF) {
-                    double2 v[8];
-#pragma unroll
-                    for (int j = 0; j < 8; j++) {
-                        v[j].x = (j ? v[j - 1].y : cum) + cur.x[j].x;
-                        v[j].y = v[j].x + cur.x[j].y;
-                    }
-                    cum = v[7].y;
-#pragma unroll
-                    for (int j = 0; j < 8; j++) *reinterpret_cast<double2 *>(cdf + at + i + 2 * j) = v[j];
-                } else {
-#pragma unroll
-                    for (int j = 0; j < 8; j++) { cum += cur.x[j].x; cum += cur.x[j].y; }
-                }
-            }
-            for (; i < cnt; i++) {
-                cum += buf[b][i];
-                if constexpr (CDF) cdf[at + i] = cum;
-            }
+            cum = chain_block<CDF>(buf[b], cnt, cum, CDF ? cdf + at : nullptr);
         }
         __syncthreads();
     }
     return cum;
+}
+// At most one block of values: total, quotients and cumulative sums in one
+// launch, each value by the same operations as in three. A measurement of a few
+// qubits is a handful of launches and one read-back: 3 of 4 qubits 52 us with
+// one launch here, 63 with three.
+__global__ __launch_bounds__(256) void k_chain_small(const double *__restrict__ p, uint32_t bins, double *__restrict__ cdf,
+                                                     double *__restrict__ total_out) {
+    __shared__ __attribute__((aligned(16))) double buf[kChainBlock];
+    __shared__ double total;
+    for (uint32_t i = threadIdx.x; i < kChainBlock; i += 256) buf[i] = i < bins ? p[i] : 0.0;
+    __syncthreads();
+    if (threadIdx.x == 0) *total_out = total = chain_block<false>(buf, (int)bins, 0.0, nullptr);
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < bins; i += 256) buf[i] = buf[i] / total;
+    __syncthreads();
+    if (threadIdx.x == 0) (void)chain_block<true>(buf, (int)bins, 0.0, cdf);
 }
 __global__ __launch_bounds__(256) void k_chain_total(const double *__restrict__ p, uint64_t bins, double *__restrict__ total_out) {
     __shared__ __attribute__((aligned(16))) double buf[2][kChainBlock];
@@ -438,9 +462,11 @@ Status measure_sample_collapse(State &s, State &dst, const uint64_t *qubits, uin
     double *cdf = hm + bins;
     double *tot = cdf + bins;  // 64 doubles reserved; chunk totals go to ctx.red
     // total and cdf
-    const double *q = hm;  // the quotients p_i / total replace the histogram
+    const double *q = hm;  // the quotients p_i / total replace the histogram (of more than one block)
     const unsigned qblocks = (unsigned)((bins + 255) / 256);
-    if (bins <= (uint64_t(1) << 16)) {
+    if (bins <= kChainBlock) {
+        hipLaunchKernelGGL(k_chain_small, dim3(1), dim3(256), 0, st, (const double *)hm, (uint32_t)bins, cdf, tot);
+    } else if (bins <= (uint64_t(1) << 16)) {
         hipLaunchKernelGGL(k_chain_total, dim3(1), dim3(256), 0, st, (const double *)hm, bins, tot);
         hipLaunchKernelGGL(k_quotients, dim3(qblocks), dim3(256), 0, st, hm, bins, (const double *)tot);
         hipLaunchKernelGGL(k_chain_cdf, dim3(1), dim3(256), 0, st, q, bins, cdf);
