@@ -108,7 +108,7 @@ inline void exp_plan_carve(ExpPlan &p, void *arena, size_t nt) { exp_plan_carve(
 int exp_tile_qubits(uint32_t n, bool c128);
 // Qubits 0 .. low-1 are always in a tile: 128-byte runs in memory.
 inline int exp_low_qubits(bool c128) { return c128 ? 3 : 4; }
-// A state of fewer than 4 qubits has no tiles: every mask is streamed.
+// Without tiles (fewer than 4 qubits, a term or two) every mask is streamed.
 void plan_expect(uint32_t n, bool c128, const qi_pauli_term *terms, size_t nt, ExpPlan &p);
 
 // ---- SumOp::apply on the same tiles ----
