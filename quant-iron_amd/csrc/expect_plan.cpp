@@ -295,6 +295,14 @@ void plan_expect(uint32_t n, bool c128, const qi_pauli_term *terms, size_t nt, E
 // the input once more: passes of fewer masks than this are not worth it.
 constexpr size_t kApplyPassMasks = 3;
 
+bool apply_as_gathers(uint32_t n, bool c128, const qi_pauli_term *terms, size_t nt) {
+    if (nt > (c128 ? 4u : 2u)) return false;
+    const uint64_t lowmask = (uint64_t(1) << exp_low_qubits(c128)) - 1;
+    for (size_t k = 0; k < nt; k++)
+        if (!terms[k].x_mask || popc(terms[k].x_mask | lowmask) <= exp_tile_qubits(n, c128)) return false;
+    return true;
+}
+
 template <typename R> void plan_apply(uint32_t n, const qi_pauli_term *terms, size_t nt, ApplyPlan<R> &p) {
     const bool c128 = sizeof(R) == 8;
     const int K = exp_tile_qubits(n, c128);

@@ -7,6 +7,7 @@
 // swapping and negating parts, so the result equals the reference's
 // op-by-op application. The coefficient multiply, cosh/sinh mix and term sums
 // then follow the reference's complex operations one for one.
+#include "expect_plan.h"
 #include "qi_internal.h"
 
 #pragma clang fp contract(off)
@@ -93,7 +94,7 @@ __global__ __launch_bounds__(256) void k_pauli_exp(typename V2<R>::T *psi, uint6
 }
 
 // out_i = sum_t (P_t in)_i * c_t, folded in term order (SumOp::apply of states
-// up to 20 qubits).
+// up to 20 qubits, and of a few wide terms).
 template <typename R>
 __global__ __launch_bounds__(256) void k_sumop_apply(const typename V2<R>::T *__restrict__ in,
                                                      typename V2<R>::T *__restrict__ out, uint64_t dim,
@@ -196,7 +197,8 @@ Status launch_sumop_apply(const State &in, State &out, const qi_pauli_term *term
     // workgroups; the crossover lies between 20 and 21 qubits in both precisions
     // (us, one chain or lattice of each size): 4 x 5 qubits 112 / 145 (complex64),
     // 125 / 136 (complex128), 3 x 7: 198 / 156 and 224 / 162.
-    if (in.n > 20) return sumop_apply_tiles(in, out, terms, nt, st);
+    // Above, a few terms that no tile holds are gathers too.
+    if (in.n > 20 && !apply_as_gathers(in.n, in.prec == QI_C128, terms, nt)) return sumop_apply_tiles(in, out, terms, nt, st);
     Ctx &C = *in.ctx;
     std::vector<TermK> h(nt);
     for (size_t k = 0; k < nt; k++) h[k] = make_term(terms[k]);

@@ -36,5 +36,18 @@ int main() {
             streamed("three terms", n, c128, {z, zz, z}, false);
         }
     for (uint32_t n : {1u, 2u, 3u}) streamed("no tiles", n, true, {{0, 1, 0.5, 0.0}, {1, 1, 0.5, 0.0}, {0, 1, 0.5, 0.0}}, true);
+    // products: few terms, all wider than a tile (13 qubits in complex64, 12 in complex128, the low ones among them)
+    for (int c128 = 0; c128 < 2; c128++) {
+        const uint64_t full = (1 << 22) - 1, wide = full & ~uint64_t(0x1ff0), fits = c128 ? 0xff8 : 0x1ff0;
+        const size_t most = c128 ? 4 : 2;
+        for (size_t count = 1; count <= 5; count++) {
+            std::vector<qi_pauli_term> t(count, {wide, 3, 0.5, 0.0});
+            if (apply_as_gathers(22, c128, t.data(), count) != (count <= most)) wrong = 2;
+            t.back().x_mask = fits;  // one mask a tile holds, or a diagonal term
+            if (apply_as_gathers(22, c128, t.data(), count)) wrong = 3;
+            t.back().x_mask = 0;
+            if (apply_as_gathers(22, c128, t.data(), count)) wrong = 4;
+        }
+    }
     return wrong;
 }
