@@ -38,7 +38,7 @@ int main() {
     for (uint32_t n : {1u, 2u, 3u}) streamed("no tiles", n, true, {{0, 1, 0.5, 0.0}, {1, 1, 0.5, 0.0}, {0, 1, 0.5, 0.0}}, true);
     // products: few terms, all wider than a tile (13 qubits in complex64, 12 in complex128, the low ones among them)
     for (int c128 = 0; c128 < 2; c128++) {
-        const uint64_t full = (1 << 22) - 1, wide = full & ~uint64_t(0x1ff0), fits = c128 ? 0xff8 : 0x1ff0;
+        const uint64_t full = (1 << 22) - 1, wide = full & ~uint64_t(0xff0), fits = c128 ? 0xff8 : 0x1ff0;
         const size_t most = c128 ? 4 : 2;
         for (size_t count = 1; count <= 5; count++) {
             std::vector<qi_pauli_term> t(count, {wide, 3, 0.5, 0.0});
