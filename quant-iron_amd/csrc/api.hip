@@ -112,21 +112,6 @@ Status ensure(DevBuf &b, size_t bytes) {
     return Status{};
 }
 
-Status ensure_stage(Ctx &C, size_t bytes) {
-    try {
-        if (C.plan_arena.size() < bytes) C.plan_arena.resize(bytes);
-    } catch (const std::bad_alloc &) {
-        return make_err(QI_ERR_OUT_OF_MEMORY, 0, 0, 0, 0, "host memory");
-    }
-    if (C.stage_bytes >= bytes) return Status{};
-    if (C.stage) (void)hipHostFree(C.stage);
-    C.stage = nullptr;
-    C.stage_bytes = 0;
-    QI_HIP_TRY(hipHostMalloc((void **)&C.stage, bytes));
-    C.stage_bytes = bytes;
-    return Status{};
-}
-
 // ------------------------------------------------------------- validation --
 // validate_qubits, operator.rs:214-273.
 static Status validate_qubits(uint32_t n, const uint64_t *t, uint32_t nt, const uint64_t *c, uint32_t nc, uint32_t expected) {
@@ -576,14 +561,14 @@ static Status apply_gates(State &s, uint32_t n_circuit, const qi_gate *gates, si
             if (!(e = ensure(C.plan, plan->blob_bytes())).ok()) return e;
             // a cached graph reads the op table about to be overwritten
             if (C.graph_exec) { (void)hipGraphExecDestroy(C.graph_exec); C.graph_exec = nullptr; C.graph_key.clear(); }
-            // through the pinned staging buffer (idle between calls); the stream
-            // orders the copy after the previous plan's launches
-            if (!(e = ensure_stage(C, plan->blob_bytes())).ok()) return e;
-            if (!plan->reg_ops.empty()) memcpy(C.stage, plan->reg_ops.data(), plan->reg_ops.size() * sizeof(RegOp));
-            if (!plan->mats.empty()) memcpy(C.stage + plan->mats_offset(), plan->mats.data(), plan->mats.size());
+            // the stream orders the copy after the previous plan's launches
+            Staging tab;
+            if (!(e = stage_tables(C, plan->blob_bytes(), tab)).ok()) return e;
+            if (!plan->reg_ops.empty()) memcpy(tab.p, plan->reg_ops.data(), plan->reg_ops.size() * sizeof(RegOp));
+            if (!plan->mats.empty()) memcpy(tab.p + plan->mats_offset(), plan->mats.data(), plan->mats.size());
             if (!plan->small_ops.empty())
-                memcpy(C.stage + plan->small_offset(), plan->small_ops.data(), plan->small_ops.size() * sizeof(SmallOp));
-            QI_HIP_TRY(hipMemcpyAsync(C.plan.p, C.stage, plan->blob_bytes(), hipMemcpyHostToDevice, C.stream));
+                memcpy(tab.p + plan->small_offset(), plan->small_ops.data(), plan->small_ops.size() * sizeof(SmallOp));
+            if (!(e = send_tables(tab, C.plan.p, plan->blob_bytes(), C.stream)).ok()) return e;
         }
         C.cached_plan = plan;
         C.plan_key.resize(sizeof head + gate_bytes);
@@ -596,7 +581,9 @@ static Status apply_gates(State &s, uint32_t n_circuit, const qi_gate *gates, si
     const uint64_t key[3] = {C.plan_serial, (uint64_t)(uintptr_t)C.plan.p, (uint64_t)(uintptr_t)(allow_oop ? C.alt.p : nullptr)};
     void *alt = allow_oop ? C.alt.p : nullptr;
     auto launch = [&]() -> Status { return launch_plan(s, *plan, gates, C.plan.p, alt); };
-    return run_maybe_graph(C, s, use_graph, key, sizeof key, launch);
+    Status e = run_maybe_graph(C, s, use_graph, key, sizeof key, launch);
+    if (!e.ok()) (void)hipStreamSynchronize(C.stream);  // the plan's copy is done with the staging buffer
+    return e;
 }
 
 static Status check_pair(const State &a, const State &b) {
@@ -695,7 +682,10 @@ qi_status qi_ctx_create(int device, qi_ctx_t *out, qi_error *err) {
     // the no-allocation scratch array's address on this device (the device is current)
     {
         Status ns = noalloc_scratch(device, &C.noalloc);
-        if (ns.ok()) ns = ensure_stage(C, expect_stage_bytes(kNoAllocMaxTerms));
+        std::vector<unsigned char> none;
+        unsigned char *p = nullptr;
+        if (ns.ok()) ns = ensure_stage(C, expect_table_bytes(kNoAllocMaxTerms));
+        if (ns.ok()) ns = plan_memory(C, expect_arena_bytes(kNoAllocMaxTerms), none, &p);
         if (!ns.ok()) QI_RET(ns);
     }
     // an unseeded context draws from an OS-seeded stream, as rand::rng() does

@@ -500,9 +500,9 @@ TermK far_term(const qi_pauli_term &p) {
     return t;
 }
 
-// Plans into `arena` (exp_plan_bytes(nt)).
-ExpLaunch plan_launch(const State &s, const qi_pauli_term *terms, size_t nt, void *arena, ExpPlan &p) {
-    exp_plan_carve(p, arena, nt);
+// Plans into `arena` (exp_plan_bytes(nt, units)).
+ExpLaunch plan_launch(const State &s, const qi_pauli_term *terms, size_t nt, void *arena, size_t units, ExpPlan &p) {
+    exp_plan_carve(p, arena, nt, units);
     plan_expect(s.n, s.prec == QI_C128, terms, nt, p);
     size_t nf = 0;
     for (size_t g = 0; g < p.nfar; g++)
@@ -560,18 +560,19 @@ Status launch_all(const State &s, const ExpPlan &p, const ExpLaunch &L, const un
     return Status{};
 }
 
-// Uploads the packed tables through the context's pinned staging buffer and
-// runs the launches; the result lands in the context's pinned words.
-Status expect_run(State &s, const qi_pauli_term *terms, const ExpPlan &p, const ExpLaunch &L, void *dtab, double *part,
+// Uploads the packed tables and runs the launches; the result lands in the
+// context's pinned words.
+Status expect_run(State &s, const qi_pauli_term *terms, const ExpPlan &p, const ExpLaunch &L, Staging &stage, void *dtab, double *part,
                   double *re, double *im, hipStream_t st) {
     Ctx &C = *s.ctx;
-    pack_tables(p, L, terms, (unsigned char *)C.stage);
-    QI_HIP_TRY(hipMemcpyAsync(dtab, C.stage, L.bytes, hipMemcpyHostToDevice, st));
-    Status e = s.prec == QI_C128
-                   ? launch_all<double2>(s, p, L, (const unsigned char *)dtab, part, C.host_pinned, st)
-                   : launch_all<float2>(s, p, L, (const unsigned char *)dtab, part, C.host_pinned, st);
+    pack_tables(p, L, terms, stage.p);
+    Status e = send_tables(stage, dtab, L.bytes, st);
+    if (e.ok())
+        e = s.prec == QI_C128 ? launch_all<double2>(s, p, L, (const unsigned char *)dtab, part, C.host_pinned, st)
+                              : launch_all<float2>(s, p, L, (const unsigned char *)dtab, part, C.host_pinned, st);
+    const hipError_t done = hipStreamSynchronize(st);
     if (!e.ok()) return e;
-    QI_HIP_TRY(hipStreamSynchronize(st));
+    QI_HIP_TRY(done);
     *re = C.host_pinned[0];
     *im = C.host_pinned[1];
     return Status{};
@@ -586,12 +587,13 @@ Status apply_tiles(const State &in, State &out, const qi_pauli_term *terms, size
     ApplyPlan<R> p;
     plan_apply<R>(in.n, terms, nt, p);
     const size_t diags = up16(p.units.size() * sizeof(ApplyUnit<R>)), bytes = diags + p.diags.size() * sizeof(ExpDiag);
+    Staging tab;
     Status s = ensure(C.ops, bytes);
-    if (s.ok()) s = ensure_stage(C, bytes);
+    if (s.ok()) s = stage_tables(C, bytes, tab);
     if (!s.ok()) return s;
-    memcpy(C.stage, p.units.data(), p.units.size() * sizeof(ApplyUnit<R>));
-    memcpy(C.stage + diags, p.diags.data(), p.diags.size() * sizeof(ExpDiag));
-    if (bytes) QI_HIP_TRY(hipMemcpyAsync(C.ops.p, C.stage, bytes, hipMemcpyHostToDevice, st));
+    if (!p.units.empty()) memcpy(tab.p, p.units.data(), p.units.size() * sizeof(ApplyUnit<R>));
+    if (!p.diags.empty()) memcpy(tab.p + diags, p.diags.data(), p.diags.size() * sizeof(ExpDiag));
+    if (!(s = send_tables(tab, C.ops.p, bytes, st)).ok()) return s;
     const uint64_t tiles = (uint64_t(1) << in.n) >> p.K;
     const unsigned threads = 1u << (p.K - apply_slot_bits(sizeof(R) == 8));  // one slot set each: 512
     for (size_t k = 0; k < p.passes.size(); k++) {
@@ -601,8 +603,9 @@ Status apply_tiles(const State &in, State &out, const qi_pauli_term *terms, size
         hipLaunchKernelGGL(kernel, dim3((unsigned)tiles), dim3(threads), sizeof(T) << p.K, st, (const T *)in.d, (T *)out.d,
                            p.passes[k], (const ApplyUnit<R> *)C.ops.p, (const ExpDiag *)((const unsigned char *)C.ops.p + diags), p.K);
     }
-    QI_HIP_TRY(hipGetLastError());
-    QI_HIP_TRY(hipStreamSynchronize(st));  // the tables and the staging buffer are reused by the next call
+    const hipError_t launched = hipGetLastError(), done = hipStreamSynchronize(st);  // the next call reuses the tables and the staging buffer
+    QI_HIP_TRY(launched);
+    QI_HIP_TRY(done);
     return Status{};
 }
 }  // namespace
@@ -612,17 +615,25 @@ Status sumop_apply_tiles(const State &in, State &out, const qi_pauli_term *terms
                               : apply_tiles<float2, float>(in, out, terms, nt, st);
 }
 
-size_t expect_stage_bytes(size_t nt) { return exp_plan_bytes(nt) + nt * (sizeof(TermK) + sizeof(FarMask)) + 256; }
+size_t expect_arena_bytes(size_t nt) { return exp_plan_bytes(nt); }
+size_t expect_table_bytes(size_t nt) {
+    return nt * (sizeof(ExpPass) + sizeof(ExpSet) + 4 * sizeof(ExpUnit) + sizeof(ExpDiag) + sizeof(TermK) + sizeof(FarMask)) + 512;
+}
 
 Status sumop_expectation(State &s, const qi_pauli_term *terms, size_t nt, double *re, double *im, hipStream_t st) {
     Ctx &C = *s.ctx;
-    Status e = ensure_stage(C, expect_stage_bytes(nt));
+    const size_t units = exp_max_units(terms, nt);
+    std::vector<unsigned char> own;
+    unsigned char *arena = nullptr;
+    Status e = plan_memory(C, exp_plan_bytes(nt, units), own, &arena);
     if (!e.ok()) return e;
     ExpPlan p;
-    const ExpLaunch L = plan_launch(s, terms, nt, C.plan_arena.data(), p);
+    Staging stage;
+    const ExpLaunch L = plan_launch(s, terms, nt, arena, units, p);
+    if (!(e = stage_tables(C, L.bytes, stage)).ok()) return e;
     if (!(e = ensure(C.ops, L.bytes)).ok()) return e;
     if (!(e = ensure(C.red, L.blocks * 4 * sizeof(double))).ok()) return e;
-    return expect_run(s, terms, p, L, C.ops.p, (double *)C.red.p, re, im, st);
+    return expect_run(s, terms, p, L, stage, C.ops.p, (double *)C.red.p, re, im, st);
 }
 
 // ---------------------------------------------------- no-allocation variant --
@@ -637,7 +648,7 @@ Status sumop_expectation(State &s, const qi_pauli_term *terms, size_t nt, double
 namespace {
 struct NoAllocScratch {
     unsigned char tab[kNoAllocMaxTerms * (sizeof(ExpPass) + sizeof(ExpSet) + 4 * sizeof(ExpUnit) + sizeof(ExpDiag) +
-                                          sizeof(TermK) + sizeof(FarMask)) + 512];
+                                          sizeof(TermK) + sizeof(FarMask)) + 512];  // expect_table_bytes(kNoAllocMaxTerms)
     double part[(kExpBlocks + 2 * kExpBlocksMin * kNoAllocMaxTerms) * 4];
 };
 }  // namespace
@@ -668,11 +679,16 @@ Status sumop_expectation_noalloc(State &s, const qi_pauli_term *terms, size_t nt
     *re = 0.0; *im = 0.0;
     if (nt == 0) return Status{};
     NoAllocScratch *sc = reinterpret_cast<NoAllocScratch *>(base);
+    Ctx &C = *s.ctx;
+    const size_t units = exp_max_units(terms, nt);
+    if (exp_plan_bytes(nt, units) > C.plan_arena.size()) return make_err(QI_ERR_DEVICE, 0, 0, 0, 0, "expectation planning memory");
     ExpPlan p;
-    const ExpLaunch L = plan_launch(s, terms, nt, s.ctx->plan_arena.data(), p);
-    if (L.bytes > sizeof sc->tab || L.blocks * 4 * sizeof(double) > sizeof sc->part)
+    const ExpLaunch L = plan_launch(s, terms, nt, C.plan_arena.data(), units, p);
+    if (L.bytes > sizeof sc->tab || L.bytes > C.stage_bytes || L.blocks * 4 * sizeof(double) > sizeof sc->part)
         return make_err(QI_ERR_DEVICE, 0, 0, 0, 0, "expectation scratch");
-    return expect_run(s, terms, p, L, sc->tab, sc->part, re, im, st);
+    Staging stage;
+    stage.p = C.stage;
+    return expect_run(s, terms, p, L, stage, sc->tab, sc->part, re, im, st);
 }
 
 }  // namespace qi

@@ -102,9 +102,9 @@ struct Ctx {
     // (the reference draws from rand::rng(), state.rs:601-602)
     uint64_t rng = 0;
     void *noalloc = nullptr;  // this device's copy of the no-allocation scratch array (expect.hip)
-    // SumOp expectations: host planning arena and the pinned staging buffer of
-    // the device tables, both large enough for kNoAllocMaxTerms terms from the
-    // context's creation and grown by longer term lists
+    // the planning memory of SumOp expectations and the pinned staging buffer
+    // of device tables (stage.cpp), both large enough for kNoAllocMaxTerms terms
+    // from the context's creation
     std::vector<unsigned char> plan_arena;
     unsigned char *stage = nullptr;
     size_t stage_bytes = 0;
@@ -202,9 +202,25 @@ struct DiagPass {
 Status launch_diag_tables(State &s, const DiagPass &p, const double2 *dtables, hipStream_t st);
 // Expectation of a list of terms (expect.hip); result (re, im) summed in FP64 compensated.
 Status sumop_expectation(State &s, const qi_pauli_term *terms, size_t nt, double *re, double *im, hipStream_t st);
-size_t expect_stage_bytes(size_t nt);
-// Ctx::plan_arena and Ctx::stage of at least `bytes` bytes (no call of the context in flight).
+// Planning memory and packed tables of any list of nt terms.
+size_t expect_arena_bytes(size_t nt);
+size_t expect_table_bytes(size_t nt);
+
+// ------------------------------------------------ planning and staging memory --
+constexpr size_t kArenaKept = ~size_t(0), kStageKept = ~size_t(0);
+// Planning memory: the context's, or `own` above kArenaKept.
+Status plan_memory(Ctx &C, size_t bytes, std::vector<unsigned char> &own, unsigned char **p);
+// Where a call packs its tables: the context's pinned buffer, or memory of its
+// own above kStageKept. No copy from the pinned buffer is in flight: a call that
+// has queued one waits for the stream before it returns, errors included.
+struct Staging {
+    unsigned char *p = nullptr;
+    std::vector<unsigned char> own;
+};
 Status ensure_stage(Ctx &C, size_t bytes);
+Status stage_tables(Ctx &C, size_t bytes, Staging &s);
+// Queues the copy of the packed tables.
+Status send_tables(const Staging &s, void *dst, size_t bytes, hipStream_t st);
 // The no-allocation expectation: at most kNoAllocMaxTerms terms, all scratch in
 // a static device array whose per-device address noalloc_scratch returns.
 constexpr int kNoAllocMaxTerms = 512;
