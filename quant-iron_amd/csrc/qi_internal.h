@@ -207,7 +207,10 @@ size_t expect_arena_bytes(size_t nt);
 size_t expect_table_bytes(size_t nt);
 
 // ------------------------------------------------ planning and staging memory --
-constexpr size_t kArenaKept = ~size_t(0), kStageKept = ~size_t(0);
+// A context keeps this much planning and pinned staging memory at most; a call
+// that needs more (more than about 20000 terms, or 190000 gates in tile passes) has
+// memory of its own for its duration.
+constexpr size_t kArenaKept = size_t(8) << 20, kStageKept = size_t(32) << 20;
 // Planning memory: the context's, or `own` above kArenaKept.
 Status plan_memory(Ctx &C, size_t bytes, std::vector<unsigned char> &own, unsigned char **p);
 // Where a call packs its tables: the context's pinned buffer, or memory of its

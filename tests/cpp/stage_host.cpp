@@ -1,6 +1,7 @@
 // The staging and planning memory of stage.cpp on the CPU: the HIP calls are
 // replaced by host ones that can be told to fail. Exit code 0 when a failed
-// growth leaves what was there and nothing is freed twice or lost.
+// growth leaves what was there, large requests leave the context's buffers alone
+// and nothing is freed twice or lost.
 #include <cstdio>
 #include <cstdlib>
 #include <map>
@@ -60,11 +61,27 @@ int main() {
     CHECK(!stage_tables(C, 100000, s).ok() && C.stage == first);
     fail_host = false;
     CHECK(ensure_stage(C, 100000).ok() && C.stage_bytes >= 100000 && live.size() == 1);
-    std::vector<unsigned char> dst(64);
+    // tables above the limit: memory of the call's own, sent before it can go
+    const size_t kept = C.stage_bytes, big = kStageKept + 1;
+    std::vector<unsigned char> dst(big);
+    {
+        Staging large;
+        CHECK(stage_tables(C, big, large).ok() && large.p != C.stage && C.stage_bytes == kept && live.size() == 1);
+        large.p[big - 1] = 9;
+        CHECK(send_tables(large, dst.data(), big, nullptr).ok() && copies == 1 && waits == 1 && dst[big - 1] == 9);
+    }
     Staging small;
     CHECK(stage_tables(C, 64, small).ok() && small.p == C.stage);
-    CHECK(send_tables(small, dst.data(), 64, nullptr).ok() && copies == 1 && waits == 0);
-    CHECK(send_tables(small, nullptr, 0, nullptr).ok() && copies == 1);
+    CHECK(send_tables(small, dst.data(), 64, nullptr).ok() && copies == 2 && waits == 1);
+    CHECK(send_tables(small, nullptr, 0, nullptr).ok() && copies == 2);
+    // planning memory: kept up to its limit, the call's own above
+    std::vector<unsigned char> own;
+    unsigned char *p = nullptr;
+    CHECK(plan_memory(C, 5000, own, &p).ok() && p == C.plan_arena.data() && own.empty() && C.plan_arena.size() >= 5000);
+    CHECK(plan_memory(C, kArenaKept + 1, own, &p).ok() && p == own.data() && C.plan_arena.size() <= kArenaKept);
+    // no more than the limit is ever pinned
+    for (size_t n = 1 << 20; n <= kStageKept; n += 3 << 20) CHECK(ensure_stage(C, n).ok() && C.stage_bytes <= kStageKept);
+    CHECK(ensure_stage(C, kStageKept).ok() && C.stage_bytes == kStageKept && live.size() == 1);
     (void)hipHostFree(C.stage);
     return 0;
 }

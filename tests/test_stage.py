@@ -1,6 +1,6 @@
 """Staging and planning memory (stage.cpp) on the CPU with the HIP calls
 replaced (tests/cpp/stage_host.cpp), under the address and undefined-behaviour
-sanitizers: a failed growth loses nothing."""
+sanitizers: a failed growth loses nothing, large tables are not kept."""
 import subprocess
 from pathlib import Path
 
