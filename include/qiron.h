@@ -389,7 +389,8 @@ qi_status qi_batch_info(qi_batch_t b, uint64_t *ncircuits, uint64_t *nsmall, uin
                         double *last_ms, qi_error *err);
 /* Schedule of the batch: circuits with n <= ks qubits run LDS-resident (one
  * workgroup each); larger ones run tiled passes of 2^k amplitudes.
- * 10 <= k <= ks <= 13 (complex64) / 12 (complex128). Default k = ks = 13 / 12. */
+ * 10 <= k <= ks <= 13 (complex64) / 12 (complex128). Default k = ks = 13 / 12;
+ * asking for the default is the default. */
 qi_status qi_batch_set_schedule(qi_batch_t b, uint32_t k, uint32_t ks, qi_error *err);
 qi_status qi_batch_get_schedule(qi_batch_t b, uint32_t *k, uint32_t *ks, qi_error *err);
 /* Executor of the circuits larger than ks qubits. QI_BATCH_WAVE (default):

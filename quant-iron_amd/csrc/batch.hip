@@ -549,7 +549,6 @@ struct Batch {
     std::vector<char> wsparse;                       // the level has tasks whose state is still partly known to be zero
     size_t nsmall = 0, nfold = 0;
     int K = 0, KS = 0;        // tile width of tiled circuits, largest LDS-resident circuit (0: defaults)
-    bool chosen = false;      // K was asked for (set or autotuned)
     int EK = 0;               // tile width of the expectation passes
     std::unordered_multimap<uint64_t, uint32_t> prog_index;  // shape hash -> program
     bool planned = false;
@@ -774,13 +773,13 @@ Status batch_plan(Batch &B) {
     if (!B.KS) B.KS = B.K;
     if (B.KS < B.K) return make_err(QI_ERR_INVALID_ARGUMENT, 0, 0, 0, 0, "LDS-resident limit below the tile width");
     const int L = c128 ? 3 : 4;
-    // Expectation passes take tiles of one qubit less than the default width
+    // With the widest tiles, expectation passes take tiles of one qubit less
     // unless a term needs it: at half the LDS twice the workgroups per CU hide
     // each other's latency. 256 circuits of 10-22 qubits, complex64: 10.26 ->
     // 9.99 ms (11 qubits 9.86, 10 qubits 10.27); complex128 9.05 -> 8.67 ms
     // (10 qubits 8.72); 14-20 qubits 3.57 -> 3.47 and 3.46 -> 3.36 ms.
     B.EK = B.K;
-    if (!B.chosen) {
+    if (B.K == (c128 ? 12 : 13)) {
         B.EK--;
         for (const auto &C : B.circs)
             if ((int)B.progs[C.prog].n > B.KS)
@@ -1296,7 +1295,6 @@ qi_status qi_batch_set_schedule(qi_batch_t b, uint32_t k, uint32_t ks, qi_error 
     std::lock_guard<std::mutex> lk(B.ctx->mu);
     B.K = (int)k;
     B.KS = (int)ks;
-    B.chosen = true;
     B.planned = false;
     QB_RET(Status{});
 }
@@ -1351,7 +1349,6 @@ qi_status qi_batch_autotune(qi_batch_t b, uint32_t trials, uint32_t *k_out, uint
         for (int k = 10; k <= kmax; k++)
             for (int ks = k; ks <= kmax; ks++) {
                 B.exec = ex;
-                B.chosen = true;
                 B.K = k;
                 B.KS = ks;
                 B.planned = false;
