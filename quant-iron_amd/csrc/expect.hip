@@ -33,6 +33,14 @@ __device__ __forceinline__ double flip_sign(double x, uint32_t odd) {
     return __longlong_as_double((long long)b);
 }
 
+// a += x y by two-sum: the rounding error of the sum goes to a.c (one multiply-add
+// less than a product and dd_acc, and the product is not rounded by itself).
+__device__ __forceinline__ void dd_fma(DD &a, double x, double y) {
+    const double s = __builtin_fma(x, y, a.s), bb = s - a.s;
+    a.c += (a.s - (s - bb)) + __builtin_fma(x, y, -bb);
+    a.s = s;
+}
+
 // The index of tile t's first amplitude: t with a zero inserted at each of the
 // K tile qubits. (The positions sit in scalar registers: loaded from memory a
 // position per trip is a wait per trip.)
@@ -76,7 +84,7 @@ __device__ __forceinline__ void pair_products(const double (&ar)[kExpSlots], con
 // FP64 conversions among the masks of the set; a Heisenberg bond costs a
 // multiply-add pair and a compensated product per amplitude pair, whatever its
 // number of terms. 29 qubits, complex64, a chain with fields (113 terms, 29 x
-// masks): 66 ms with one read of the state per mask, 5.7 ms in four passes (5.0
+// masks): 66 ms with one read of the state per mask, 5.6 ms in four passes (5.0
 // with plain FP64 sums inside a register set, which lose what two large
 // products that cancel leave between them).
 // The imaginary sums (complex coefficients) take registers that cost half the
@@ -171,7 +179,7 @@ __global__ __launch_bounds__(512, CPLX ? 2 : 4) void k_expect_tiles(const T *__r
                 // is the same for all eight
                 DD v{u[0] * un.h[0], 0.0};
 #pragma unroll
-                for (int k = 1; k < 8; k++) dd_acc(v, u[k] * un.h[k]);
+                for (int k = 1; k < 8; k++) dd_fma(v, u[k], un.h[k]);
                 const uint32_t odd = __popcll(base & un.zo) + __popc(tl & un.zl);
                 if (CPLX && (un.flags() & kExpImag)) {
                     dd_acc(acc[1], flip_sign(v.s, odd));
@@ -212,8 +220,8 @@ __global__ __launch_bounds__(512, CPLX ? 2 : 4) void k_expect_tiles(const T *__r
                         }
 #pragma unroll
                 for (int s = 0; s < kExpSlots; s++) {
-                    dd_acc(acc[0], w[s] * h[s]);
-                    if (CPLX) dd_acc(acc[1], w[s] * hi[s]);
+                    dd_fma(acc[0], w[s], h[s]);
+                    if (CPLX) dd_fma(acc[1], w[s], hi[s]);
                 }
             }
         }
