@@ -153,10 +153,8 @@ __global__ __launch_bounds__(256) void k_fold_bins_block(const double *__restric
 struct ExpandSlots {
     uint8_t s[64];  // of each listed qubit among the distinct ones, ascending
 };
-__global__ __launch_bounds__(256) void k_expand(const double *__restrict__ hd, double *__restrict__ hm, uint64_t bins_m,
-                                                ExpandSlots slot, int m) {
-    uint64_t o = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (o >= bins_m) return;
+// The value of outcome o of the m listed qubits.
+__device__ __forceinline__ double expanded(const double *__restrict__ hd, uint64_t o, const ExpandSlots &slot, int m) {
     uint64_t d = 0, seen = 0;
     bool ok = true;
     for (int b = 0; b < m; b++) {
@@ -165,7 +163,12 @@ __global__ __launch_bounds__(256) void k_expand(const double *__restrict__ hd, d
         if ((seen >> s) & 1) { if (((d >> s) & 1) != bit) ok = false; }
         else { seen |= uint64_t(1) << s; d |= bit << s; }
     }
-    hm[o] = ok ? hd[d] : 0.0;
+    return ok ? hd[d] : 0.0;
+}
+__global__ __launch_bounds__(256) void k_expand(const double *__restrict__ hd, double *__restrict__ hm, uint64_t bins_m,
+                                                ExpandSlots slot, int m) {
+    uint64_t o = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (o < bins_m) hm[o] = expanded(hd, o, slot, m);
 }
 
 // Sequential scan (state.rs:590-606): total = sum p_i in index order, then
@@ -245,14 +248,16 @@ __device__ __forceinline__ double chain(const double *__restrict__ p, uint64_t l
     return cum;
 }
 // At most one block of values: total, quotients and cumulative sums in one
-// launch, each value by the same operations as in three. A measurement of a few
-// qubits is a handful of launches and one read-back: 3 of 4 qubits 52 us with
-// one launch here, 63 with three.
-__global__ __launch_bounds__(256) void k_chain_small(const double *__restrict__ p, uint32_t bins, double *__restrict__ cdf,
-                                                     double *__restrict__ total_out) {
+// launch, each value by the same operations as in three; m > 0: of the listed
+// qubits' outcomes, p a histogram over the distinct ones. A measurement of a few
+// qubits is a handful of launches and one read-back: one of 4 qubits 37 us
+// with one launch here, 63 with three.
+__global__ __launch_bounds__(256) void k_chain_small(const double *__restrict__ p, uint32_t bins, ExpandSlots slot, int m,
+                                                     double *__restrict__ cdf, double *__restrict__ total_out) {
     __shared__ __attribute__((aligned(16))) double buf[kChainBlock];
     __shared__ double total;
-    for (uint32_t i = threadIdx.x; i < kChainBlock; i += 256) buf[i] = i < bins ? p[i] : 0.0;
+    for (uint32_t i = threadIdx.x; i < kChainBlock; i += 256)
+        buf[i] = i >= bins ? 0.0 : m ? expanded(p, i, slot, m) : p[i];
     __syncthreads();
     if (threadIdx.x == 0) *total_out = total = chain_block<false>(buf, (int)bins, 0.0, nullptr);
     __syncthreads();
@@ -352,11 +357,15 @@ __global__ __launch_bounds__(256) void k_collapse(const T *src, T *dst, uint64_t
     if (threadIdx.x == 0) { part[blockIdx.x * 2] = v[0].s; part[blockIdx.x * 2 + 1] = v[0].c; }
 }
 
-}  // namespace
-
-// Histogram over `qubits` (bit b = qubits[b]); returns a device pointer to
-// 2^m FP64 probabilities inside ctx.probs.
-Status measure_probs_device(State &s, const uint64_t *qubits, uint32_t m, double **dprobs, hipStream_t st) {
+// Histogram over `qubits` (bit b = qubits[b]): 2^m FP64 probabilities inside
+// ctx.probs. With `later`, a histogram of at most one block is left over the
+// distinct qubits (later->m > 0; else it is the result).
+struct Unexpanded {
+    const double *hd = nullptr;
+    ExpandSlots slot{};
+    int m = 0;
+};
+Status histogram(State &s, const uint64_t *qubits, uint32_t m, double **dprobs, Unexpanded *later, hipStream_t st) {
     Ctx &C = *s.ctx;
     // distinct qubits, in ascending order for the bin index
     uint64_t dmask = 0;
@@ -411,11 +420,19 @@ Status measure_probs_device(State &s, const uint64_t *qubits, uint32_t m, double
         else if (chunks > 1)
             hipLaunchKernelGGL(k_fold_bins_block, dim3((unsigned)bins_d), dim3(256), 0, st, (const double *)part, bins_d, chunks, hd);
     }
-    if (!plain)
+    if (later) *later = Unexpanded{hd, slot, 0};
+    if (!plain && later && bins_m <= kChainBlock) later->m = (int)m;
+    else if (!plain)
         hipLaunchKernelGGL(k_expand, dim3((unsigned)((bins_m + 255) / 256)), dim3(256), 0, st, hd, hm, bins_m, slot, (int)m);
     QI_HIP_TRY(hipGetLastError());
     *dprobs = hm;
     return Status{};
+}
+
+}  // namespace
+
+Status measure_probs_device(State &s, const uint64_t *qubits, uint32_t m, double **dprobs, hipStream_t st) {
+    return histogram(s, qubits, m, dprobs, nullptr, st);
 }
 
 // Keep the amplitudes whose measured bits spell `outcome` (bit b of the
@@ -456,7 +473,8 @@ Status measure_sample_collapse(State &s, State &dst, const uint64_t *qubits, uin
                                size_t shots, uint64_t *outcomes_host, bool collapse, hipStream_t st) {
     Ctx &C = *s.ctx;
     double *hm = nullptr;
-    Status e = measure_probs_device(s, qubits, m, &hm, st);
+    Unexpanded hist;
+    Status e = histogram(s, qubits, m, &hm, &hist, st);
     if (!e.ok()) return e;
     const uint64_t bins = uint64_t(1) << m;
     double *cdf = hm + bins;
@@ -465,7 +483,8 @@ Status measure_sample_collapse(State &s, State &dst, const uint64_t *qubits, uin
     const double *q = hm;  // the quotients p_i / total replace the histogram (of more than one block)
     const unsigned qblocks = (unsigned)((bins + 255) / 256);
     if (bins <= kChainBlock) {
-        hipLaunchKernelGGL(k_chain_small, dim3(1), dim3(256), 0, st, (const double *)hm, (uint32_t)bins, cdf, tot);
+        hipLaunchKernelGGL(k_chain_small, dim3(1), dim3(256), 0, st, hist.m ? hist.hd : (const double *)hm, (uint32_t)bins, hist.slot,
+                           hist.m, cdf, tot);
     } else if (bins <= (uint64_t(1) << 16)) {
         hipLaunchKernelGGL(k_chain_total, dim3(1), dim3(256), 0, st, (const double *)hm, bins, tot);
         hipLaunchKernelGGL(k_quotients, dim3(qblocks), dim3(256), 0, st, hm, bins, (const double *)tot);

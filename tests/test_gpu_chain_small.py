@@ -39,3 +39,22 @@ def test_a_zero_state_is_an_error(ctx, n, m):
     s = qiron.State.from_vector_unchecked(np.zeros(1 << n, dtype=np.complex128), "c128")
     with pytest.raises(qiron.QuantIronError):
         s.measure_outcomes(list(range(m)), [0.5])
+
+
+# qubits out of order and listed again: an outcome whose bits contradict each other has no weight
+@pytest.mark.parametrize("prec", ["c64", "c128"])
+@pytest.mark.parametrize("n,qs", [(3, [2, 0]), (3, [1, 1, 1]), (9, [8, 0, 8, 3]), (13, [12, 12]), (14, [5, 3, 5, 9, 13, 0, 0, 1, 2, 7, 11]),
+                                  (14, [5, 3, 5, 9, 13, 0, 0, 1, 2, 7, 11, 12])])
+def test_lists_out_of_order_and_with_repeats(ctx, n, qs, prec):
+    s = qiron.State.from_vector_unchecked(random_state(n, np.random.default_rng([n, len(qs)])), prec)
+    p = s.measure_probs(qs)
+    for a in range(len(qs)):
+        for b in range(a):
+            if qs[a] == qs[b]:
+                o = np.arange(p.size)
+                assert not np.any(p[((o >> a) ^ (o >> b)) & 1 == 1])
+    u = np.random.default_rng(n).random(2000)
+    got = s.measure_outcomes(qs, u).astype(np.int64)
+    np.testing.assert_array_equal(got, outcomes(p, u)[0])
+    r = s.measure(qiron.MeasurementBasis.Computational, qs, float(u[0]))
+    assert sum(bit << k for k, bit in enumerate(r.outcomes)) == got[0]
