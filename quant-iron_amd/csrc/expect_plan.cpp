@@ -296,7 +296,7 @@ void plan_expect(uint32_t n, bool c128, const qi_pauli_term *terms, size_t nt, E
 constexpr size_t kApplyPassMasks = 3;
 
 bool apply_as_gathers(uint32_t n, bool c128, const qi_pauli_term *terms, size_t nt) {
-    if (nt > (c128 ? 4u : 2u)) return false;
+    if (nt > (c128 ? 4u : 3u)) return false;
     const uint64_t lowmask = (uint64_t(1) << exp_low_qubits(c128)) - 1;
     for (size_t k = 0; k < nt; k++)
         if (!terms[k].x_mask || popc(terms[k].x_mask | lowmask) <= exp_tile_qubits(n, c128)) return false;

@@ -152,7 +152,8 @@ inline uint32_t apply_slots(int K, bool c128) {
 // LDS would be read for nothing, so that each term is cheaper as a gather. 27
 // qubits, us, tile passes -> gathers: 1 term 577 -> 380 (complex64), 1185 -> 869
 // (complex128); 2 terms 577 -> 476 and 1161 -> 851; 4 terms 602 -> 760 and 1109 ->
-// 1024 (complex128 with 8 terms: between 1.22 and 0.86 times).
+// 1024; 3 random terms on 28 qubits in complex64 1912 -> 1602 (complex128 with 8
+// terms: between 1.22 and 0.86 times).
 bool apply_as_gathers(uint32_t n, bool c128, const qi_pauli_term *terms, size_t nt);
 template <typename R> void plan_apply(uint32_t n, const qi_pauli_term *terms, size_t nt, ApplyPlan<R> &p);
 

@@ -39,7 +39,7 @@ int main() {
     // products: few terms, all wider than a tile (13 qubits in complex64, 12 in complex128, the low ones among them)
     for (int c128 = 0; c128 < 2; c128++) {
         const uint64_t full = (1 << 22) - 1, wide = full & ~uint64_t(0xff0), fits = c128 ? 0xff8 : 0x1ff0;
-        const size_t most = c128 ? 4 : 2;
+        const size_t most = c128 ? 4 : 3;
         for (size_t count = 1; count <= 5; count++) {
             std::vector<qi_pauli_term> t(count, {wide, 3, 0.5, 0.0});
             if (apply_as_gathers(22, c128, t.data(), count) != (count <= most)) wrong = 2;
