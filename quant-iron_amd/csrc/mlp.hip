@@ -1258,7 +1258,8 @@ static void refresh_bf16(Mlp &N, hipStream_t st) {
 }
 
 // Hidden widths the fused prediction kernel is built for (16 NJ columns per
-// wave), and inputs that fit its LDS rows beside a second workgroup.
+// wave), and inputs that fit its LDS rows beside a second workgroup. Measured
+// for these two widths only; the other multiples of 64 up to 512 would fit.
 static bool fused_predict(const Mlp &N) { return (N.hid == 512 || N.hid == 256) && N.k_in <= 576; }
 // Dynamic LDS above 64 KiB has to be allowed per kernel (and device).
 template <typename F> static Status allow_lds() {
@@ -1285,7 +1286,8 @@ static void pack_weights(Mlp &N, hipStream_t st) {
     hipLaunchKernelGGL(k_pack_weights, dim3((unsigned)((steps * (N.hid / 16) * 64 + 255) / 256), 3), dim3(256), 0, st,
                        (const bf16 *)N.wt, L, N.wp);
 }
-// Predictions of `rows` rows of the source f (candidates from c0).
+// Predictions of `rows` rows of the source f (candidates from c0; staged rows are
+// fewer than one launch takes).
 template <typename F> static void predict_fused(Mlp &N, hipStream_t st, const F &f, uint64_t c0, uint64_t rows, float *y) {
     const int lda = std::max((N.k_in + 31) / 32 * 32, N.hid) + 8;
     const size_t lds = size_t(64) * lda * sizeof(bf16) + 4 * 64 * sizeof(float);
