@@ -8,6 +8,7 @@
 // Terms that no tile holds (X support too wide) stream the state, one read per
 // x mask (k_expect_far).
 #include <algorithm>
+#include <cmath>
 
 #include "expect_plan.h"
 #include "qi_internal.h"
@@ -583,6 +584,8 @@ Status expect_run(State &s, const qi_pauli_term *terms, const ExpPlan &p, const 
     QI_HIP_TRY(done);
     *re = C.host_pinned[0];
     *im = C.host_pinned[1];
+    // (tiles of real coefficients form no imaginary part: it is zero, or unknown with the real one)
+    if (std::isnan(*re) && !p.complex_out) *im = *re;
     return Status{};
 }
 

@@ -39,3 +39,18 @@ def test_cancelling_products_keep_what_lies_between(ctx, n, prec):
             if a == q[0]:
                 y = qiron.expectation_terms(s, term_array([(x, x, 0.5, 0.0), (x, 0, 1.0, 0.25)]))  # a Y beside it: Im w is 0
                 assert y == 2.0 + 0.5j, (p, a, b)
+
+
+# a sum with a value that is not finite is NaN in both parts, whatever the route
+@pytest.mark.parametrize("prec", ["c64", "c128"])
+@pytest.mark.parametrize("n", [2, 5, 13, 15])
+@pytest.mark.parametrize("value", [complex(np.nan, 0), complex(np.inf, 0), complex(0, -np.inf)])
+def test_values_that_are_not_finite(ctx, n, prec, value):
+    v = np.full(1 << n, 2.0 ** (-n / 2), dtype=np.complex128)
+    v[3] = value
+    s = qiron.State.from_vector_unchecked(v, prec)
+    full = (1 << n) - 1
+    for terms in ([(0, 1, 0.5, 0.0)], [(1, 0, 0.5, 0.0)], [(2, 2, 0.5, 0.0)], [(1, 0, 0.5, 0.25)], [(1, 0, 0.0, 0.0)], [(full, 0, 1.0, 0.0)],
+                  [(0, 3, 0.2, 0.0), (3, 1, 0.1, 0.0), (full, 2, -0.3, 0.0)]):
+        got = qiron.expectation_terms(s, term_array(terms))
+        assert np.isnan(got.real) and np.isnan(got.imag), terms
