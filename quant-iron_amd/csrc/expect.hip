@@ -473,6 +473,14 @@ __global__ __launch_bounds__(512, 4) void k_apply_tiles(const T *__restrict__ ps
             }
         }
     }
+    // A complex product with a coefficient of one part adds zero times the other
+    // part: no matter, unless that is infinite or NaN.
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+        const bool fx = __builtin_isfinite(acc[s].x), fy = __builtin_isfinite(acc[s].y);
+        if (fy && !fx) acc[s].y = __builtin_nan("");
+        if (fx && !fy) acc[s].x = __builtin_nan("");
+    }
 #pragma unroll
     for (int j = 0; j < NU; j++) {
         uint64_t g = at;
